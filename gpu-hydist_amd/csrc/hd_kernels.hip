@@ -269,29 +269,25 @@ __device__ __forceinline__ void roll_repairs(const HdDevG& d, int dir)
     d.flags[4 + dir] = 0;
 }
 
-/* The first wet run of each edge line (column M, column 2, row 2, row N):
- * its first cell a and its cells [lo, hi] clipped to [2, max(M, N)] as
+/* The first wet run of edge e's line (column M, column 2, row 2, row N): its
+ * first cell a and its cells [lo, hi] clipped to [2, max(M, N)] as
  * k_boundary's loop (hi < lo when the line is dry). */
-struct EdgeRuns {
-    int lo[4], hi[4], a[4];
+struct EdgeRun {
+    int loc, lo, hi, a;
 };
 
-__device__ __forceinline__ EdgeRuns edge_runs(const HdDevG& d)
+__device__ __forceinline__ EdgeRun edge_run(const HdDevG& d, int e)
 {
     const int N = d.N, M = d.M, SL = d.SL;
     const int imax = M > N ? M : N;
-    EdgeRuns r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const bool col = e < 2;
-        const int loc = e == 0 ? M : (e == 3 ? N : 2);
-        const int mc = col ? d.mocj[loc] : d.moci[loc];
-        const int a = col ? d.dauj[loc * SL] : d.daui[loc * SL];
-        const int b = col ? d.cuoij[loc * SL] : d.cuoii[loc * SL];
-        r.a[e] = a;
-        r.lo[e] = a > 2 ? a : 2;
-        r.hi[e] = mc > 0 ? (b < imax ? b : imax) : r.lo[e] - 1;
-    }
+    const bool col = e < 2;
+    EdgeRun r;
+    r.loc = e == 0 ? M : (e == 3 ? N : 2);
+    const int mc = (col ? d.mocj : d.moci)[r.loc];
+    r.a = (col ? d.dauj : d.daui)[r.loc * SL];
+    const int b = (col ? d.cuoij : d.cuoii)[r.loc * SL];
+    r.lo = r.a > 2 ? r.a : 2;
+    r.hi = mc > 0 ? (b < imax ? b : imax) : r.lo - 1;
     return r;
 }
 
@@ -361,40 +357,24 @@ __device__ __forceinline__ void run_boundary(const HdDevG& d, int line, int firs
     if (!(isU ? (line == M || line == 2 || first == 2 || last == N)
               : (line == 2 || line == N || first == 2 || last == M)))
         return;
-    const EdgeRuns er = edge_runs(d);
-    /* which cells k of this run each edge writes: [klo, khi] */
-    int klo[4], khi[4];
-    bool any = false, along = false;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const bool col = e < 2;
-        const int loc = e == 0 ? M : (e == 3 ? N : 2);
-        if (isU == col) {
-            const bool mine = line == loc && first == er.a[e] && er.hi[e] >= er.lo[e];
-            klo[e] = er.lo[e];
-            khi[e] = mine ? er.hi[e] : er.lo[e] - 1;
-            along = along || mine;
-        } else {
-            const bool mine = line >= er.lo[e] && line <= er.hi[e] && (loc == 2 ? first == 2 : last == loc);
-            klo[e] = loc;
-            khi[e] = mine ? loc : loc - 1;
-        }
-        any = any || khi[e] >= klo[e];
-    }
-    if (!any) return;
     int t1;
     double t2;
     if (!boundary_time(d, t1, t2)) return;
-    auto cell = [&](int k) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (k >= klo[e] && k <= khi[e]) edge_cell(d, e, (isU == (e < 2)) ? k : line, t1, t2);
-    };
-    if (along) {
-        for (int k = first + lane; k <= last; k += kWave) cell(k);
-    } else if (lane == 0) {
-        cell(first);
-        if (last != first) cell(last);
+    /* one copy of the edge's code, looped over: unrolled it is most of the
+     * sweep's instructions and scalar registers */
+#pragma unroll 1
+    for (int e = 0; e < 4; ++e) {
+        const int loc = e == 0 ? M : (e == 3 ? N : 2);
+        const bool along = isU == (e < 2);
+        if (along ? line != loc : (loc == 2 ? first != 2 : last != loc)) continue;
+        const EdgeRun er = edge_run(d, e);
+        if (along) {
+            if (first != er.a) continue;
+            for (int k = first + lane; k <= last; k += kWave)
+                if (k >= er.lo && k <= er.hi) edge_cell(d, e, k, t1, t2);
+        } else if (lane == ((loc - first) & (kWave - 1)) && line >= er.lo && line <= er.hi) {
+            edge_cell(d, e, line, t1, t2);
+        }
     }
 }
 
@@ -410,9 +390,9 @@ __device__ __forceinline__ void run_boundary(const HdDevG& d, int line, int firs
  * row edge also covers lies in that row's first run, which then ends at M
  * or starts at 2 and holds it. */
 template <bool isU>
-__device__ __forceinline__ void across_boundary(const HdDevG& d, const EdgeRuns& er, int lane)
+__device__ __forceinline__ void across_boundary(const HdDevG& d, int lane)
 {
-    const int N = d.N, M = d.M, SL = d.SL;
+    const int SL = d.SL;
     int t1;
     double t2;
     if (!boundary_time(d, t1, t2)) return;
@@ -420,10 +400,11 @@ __device__ __forceinline__ void across_boundary(const HdDevG& d, const EdgeRuns&
     const int* moc = isU ? d.mocj : d.moci;
     const int* dau = isU ? d.dauj : d.daui;
     const int* cuoi = isU ? d.cuoij : d.cuoii;
-#pragma unroll
+#pragma unroll 1
     for (int e = isU ? 2 : 0; e < (isU ? 4 : 2); ++e) {
-        const int loc = e == 0 ? M : (e == 3 ? N : 2);
-        for (int i = er.lo[e] + lane; i <= er.hi[e]; i += kWave) {
+        const EdgeRun er = edge_run(d, e);
+        const int loc = er.loc;
+        for (int i = er.lo + lane; i <= er.hi; i += kWave) {
             const int mc = moc[i] < SL ? moc[i] : SL;
             const bool held = mc > 0 && (loc == 2 ? dau[i * SL] == 2 : cuoi[i * SL + mc - 1] == loc);
             if (!held) edge_cell(d, e, i, t1, t2);
@@ -1263,19 +1244,165 @@ __device__ __forceinline__ Pre shfl_pre(const Pre& a, int src)
     return b;
 }
 
+/* p[base + lane's byte offset]: a wave-uniform element base and a 32-bit
+ * per-lane offset, so that the load takes its base from scalar registers */
+__device__ __forceinline__ double ld_off(HD_GLOBAL_AS const double* p, long base, unsigned off)
+{
+    return *(HD_GLOBAL_AS const double*)((HD_GLOBAL_AS const char*)(p + base) + off);
+}
+__device__ __forceinline__ void st_off(HD_GLOBAL_AS double* p, long base, unsigned off, double v)
+{
+    *(HD_GLOBAL_AS double*)((HD_GLOBAL_AS char*)(p + base) + off) = v;
+}
+
+/* pre_uz_ld / pre_vz_ld at element base + off / 8 */
+template <bool isU>
+__device__ __forceinline__ PreRaw pre_ld_off(const HdDevG& d, long b, unsigned o)
+{
+    const long W = d.W;
+    const long s = isU ? 1 : W, t = isU ? W : 1; /* across and along the line */
+    HD_GLOBAL_AS const double* a = isU ? d.u : d.v;
+    HD_GLOBAL_AS const double* x = isU ? d.v : d.u;
+    HD_GLOBAL_AS const double* ha = isU ? d.Htdu : d.Htdv;
+    HD_GLOBAL_AS const double* hx = isU ? d.Htdv : d.Htdu;
+    PreRaw r;
+    r.c = ld_off(a, b, o);
+    r.n1 = ld_off(a, b + s, o); r.n2 = ld_off(a, b + 2 * s, o);
+    r.m1 = ld_off(a, b - s, o); r.m2 = ld_off(a, b - 2 * s, o);
+    r.x0 = ld_off(x, b - s, o); r.x1 = ld_off(x, b, o);
+    r.x2 = ld_off(x, b + t - s, o); r.x3 = ld_off(x, b + t, o);
+    r.vis = ld_off(d.VISCOIDX, b, o);
+    r.ht = ld_off(ha, b, o); r.ht_m = ld_off(ha, b - t, o);
+    r.k1 = ld_off(isU ? d.Kx1 : d.Ky1, b, o);
+    r.hm_m1 = ld_off(d.H_moi, b - s, o); r.hm_p1 = ld_off(d.H_moi, b + s, o); r.hm_m2 = ld_off(d.H_moi, b - 2 * s, o);
+    r.ts = ld_off(isU ? d.Tsxw : d.Tsyw, b, o);
+    r.zz = ld_off(d.z, b, o);
+    r.hc0 = ld_off(hx, b, o); r.hc1 = ld_off(hx, b - s, o);
+    return r;
+}
+
+/* Case parameters of one sweep direction as the row assembly uses them:
+ * pre_uz_ev and pre_vz_ev are the same expressions with these. */
+struct SweepConst {
+    double k, kx;      /* dTchia2dX, dTchia2dY (UZ; exchanged for VZ) */
+    double dT, H, cor, wind;
+    double e1, e2, e3; /* dXbp, dY2, dYbp (UZ); dYbp, dX2, dXbp (VZ) */
+    double y1, y2, y3; /* their refined reciprocals */
+};
+template <bool isU>
+__device__ __forceinline__ SweepConst sweep_const(const hd_params& P)
+{
+    SweepConst K;
+    K.k = isU ? P.dTchia2dX : P.dTchia2dY;
+    K.kx = isU ? P.dTchia2dY : P.dTchia2dX;
+    K.dT = P.dT;
+    K.H = P.H_TINH;
+    K.cor = isU ? -(P.dT * P.CORIOLIS_FORCE) : P.dT * P.CORIOLIS_FORCE;
+    K.wind = isU ? P.Windx : P.Windy;
+    K.e1 = isU ? P.dXbp : P.dYbp;
+    K.e2 = isU ? P.dY2 : P.dX2;
+    K.e3 = isU ? P.dYbp : P.dXbp;
+    K.y1 = hd_div::rcp_refined(K.e1);
+    K.y2 = hd_div::rcp_refined(K.e2);
+    K.y3 = hd_div::rcp_refined(K.e3);
+    return K;
+}
+
+/* The momentum row of a cell (abcd) and its continuity coefficients, from
+ * the loaded values of the cell and the continuity coefficients of the next
+ * cell along the line (the next lane's): the operations of pre_uz_ev /
+ * pre_vz_ev and abcd with each divisor's reciprocal taken once (4 instead
+ * of 13 divisions, and no branches), the same bits while `bad` stays false.
+ * The one-sided differences next to land are chosen by sign and operand
+ * selects; 2 dT vis / dXbp is twice dT vis / dXbp, exactly. */
+struct CellRow {
+    double a1, b1, c1, d1; /* momentum row */
+    double a2, c2, d2;     /* continuity coefficients */
+    double na2, nc2, nd2;  /* those of the next cell */
+    bool bad;
+};
+__device__ __forceinline__ double lane_after(double v) { return dpp_any<0x130>(v); }
+
+__device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreRaw& r, double f4, bool mom, bool useA,
+                                                 bool useC)
+{
+    CellRow o;
+    hd_div::Range rg;
+    const double uc = r.c;
+    const double vtb = (r.x0 + r.x1 + r.x2 + r.x3) * 0.25;
+    const double htu = r.ht;
+    o.c2 = K.k * htu;
+    o.a2 = -K.k * r.ht_m;
+    o.d2 = r.zz - K.kx * (r.hc0 * r.x1 - r.hc1 * r.x0);
+    const double yc = hd_div::rcp_refined(o.c2); /* 1 / c2: the previous lane divides by it */
+    o.na2 = lane_after(o.a2);
+    o.nc2 = lane_after(o.c2);
+    o.nd2 = lane_after(o.d2);
+    const double ync = lane_after(yc);
+    const double yh = hd_div::rcp_refined(htu);
+    const double ya = hd_div::rcp_refined(o.a2);
+    /* preindex */
+    const double nv = r.vis * K.dT;
+    const double g1 = hd_div::quot_pos(nv, K.e1, K.y1);
+    const double f1 = K.k * uc + g1;
+    const double f3 = g1 - K.k * uc;
+    const double nk = r.k1 * K.dT * sqrt(uc * uc + vtb * vtb);
+    const double f2 = -(2 + hd_div::quot_pos(nk, htu, yh) + 2 * g1);
+    const bool dm = r.hm_m1 <= K.H, dp = r.hm_p1 <= K.H; /* the neighbours across are dry */
+    const bool one = dm || dp;
+    const double w1 = dm ? r.n1 : r.m1, w2 = dm ? r.n2 : r.m2;
+    const double s3 = dm ? -3.0 : 3.0, s4 = dm ? 4.0 : -4.0, s1 = dm ? -1.0 : 1.0;
+    const double pn = one ? s3 * uc + s4 * w1 + s1 * w2 : r.n1 - r.m1;
+    const double qn = one ? uc - 2 * w1 + w2 : r.n1 - 2 * uc + r.m1;
+    const bool use = !one || (dm ? vtb < 0 : (r.hm_m2 > K.H && vtb > 0));
+    const double np = use ? vtb * pn : 0.0, nq = use ? qn : 0.0;
+    const double p = hd_div::quot_pos(np, K.e2, K.y2);
+    const double q = hd_div::quot_pos(nq, K.e3, K.y3);
+    const double nw = K.dT * (K.wind - r.ts);
+    const double f5 = -2 * uc + K.dT * p + K.cor * vtb - K.dT * r.vis * q - hd_div::quot_pos(nw, htu, yh);
+    /* abcd: the terms of the face behind (divided by a2 < 0) and of the
+     * face ahead (divided by the next cell's c2 > 0) */
+    const double n2 = f1 * o.c2, n3 = f1 * o.d2, n5 = f3 * o.na2, n6 = f3 * o.nd2;
+    const double t1 = hd_div::quot(f1, o.a2, ya), t2 = hd_div::quot(n2, o.a2, ya), t3 = hd_div::quot(n3, o.a2, ya);
+    const double t4 = hd_div::quot_pos(f3, o.nc2, ync), t5 = hd_div::quot_pos(n5, o.nc2, ync),
+                 t6 = hd_div::quot_pos(n6, o.nc2, ync);
+    o.a1 = useA ? f4 - t1 : f4;
+    o.b1 = useA ? f2 - t2 : f2;
+    o.d1 = useA ? f5 - t3 : f5;
+    o.c1 = useC ? -f4 - t4 : -f4;
+    o.b1 = useC ? o.b1 - t5 : o.b1;
+    o.d1 = useC ? o.d1 - t6 : o.d1;
+    /* zero or at least 2^-400 here and divisors in 2^[-100, 100] keep the
+     * products divided above in the range of hd_fastdiv.h */
+    rg.num(nv); rg.num(nk); rg.num(np); rg.num(nq); rg.num(nw);
+    rg.num(f1); rg.num(f3); rg.num(o.d2);
+    rg.den(htu);
+    rg.den(useA ? r.ht_m : 1.0); rg.den(useC ? o.nc2 : 1.0);
+    o.bad = mom && !(rg.lo >= -400 && rg.den_ok() && htu > 0 && (!useA || r.ht_m > 0) && (!useC || o.nc2 > 0) &&
+                     hd_div::finite((o.a1 + o.b1) + (o.c1 + o.d1)));
+    return o;
+}
+
 /* Fused UZ / VZ solve of one wet run per wave with the speculative parallel
  * Thomas of hd_thomas.h: the same rows as k_adi_run (_calculate_preindex,
  * _calculate_abcd, _calculate_matrix_coeff, tridiag, _extract_solution,
  * UVZSolver_multithread.cu:203-723) and the same bits.  Chunks of 255 cells
- * (510 rows) are assembled by the 64 lanes, four cells each (cell t = lane +
- * 64 h; the preindex of cell t + 1 comes from the neighbouring lane by a
- * shuffle), into LDS; the forward sweep (factors replacing C / D) and the back
+ * (510 rows) are assembled by the lanes, 63 cells a round, into LDS; the
+ * forward sweep (factors replacing C / D) and the back
  * substitution (x replacing A) run over the chunk on all lanes; factors of
  * all but the last chunk go to the run's slice of the Ap/Bp line buffers and
  * come back for back substitution.  The run's wall-flag depths, boundary
  * depths, edge values and the first cells' preindex inputs are loaded
  * together, so a short run costs one memory round trip after its table
- * entry. */
+ * entry.
+ *
+ * A wave is alone with its run, so a run costs its instructions at 5 to 7
+ * cycles each, plus the trips to memory: rows with one reciprocal per
+ * divisor and selects instead of branches (cell_rows_rcp), loads from scalar
+ * bases with 16-byte pairs, one copy of the boundary code, the next round's
+ * loads behind this round's arithmetic.  Longest run of a launch, on the
+ * device, river 980 x 1048: 24.0 -> 19.0 us once the flow is steady, 35 -> 27
+ * while it starts up; 300-cell channel lines 38 -> 26.6 us. */
 /* repaired chunks of a sweep above which the next sweep of the same
  * direction takes 8 rows per lane */
 constexpr int kAdaptRuns = 32;
@@ -1287,9 +1414,12 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
     const int sidx = 2 + shift, eidx = isU ? d.M - shift : d.N;
     constexpr int CH = 255; /* cells per LDS chunk (the rows of cell t need cells t and t + 1) */
     constexpr int RW = 2 * CH;
-    __shared__ double sA[RW], sB[RW], sC[RW], sD[RW];
+    /* rows at SpecMap positions; the run's first row (0) and last (sn),
+     * which the sweeps leave out, at the last two words */
+    constexpr int kW = spec_words(RW), kRow0 = kW - 2, kRowN = kW - 1;
+    __shared__ double sA[kW], sB[kW], sC[kW], sD[kW];
     __shared__ double sE[6];
-    __shared__ double sX[3]; /* X(0), X(sn), X(last interior u row) */
+    __shared__ double sX[1]; /* X(last interior u row) */
     const int lane = threadIdx.x;
     const int N = d.N, M = d.M, W = d.W;
     const int tw = 2 * (N > M ? N : M) + 4;
@@ -1301,25 +1431,27 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
     const int dkfr = isU ? N : M;
     const double f4 = isU ? 2 * d.P.g * d.P.dTchia2dX : 2 * d.P.g * d.P.dTchia2dY;
     const double ND = d.P.NANGDAY;
-    double* tz = d.t_z;
-    double* tq = isU ? d.t_u : d.t_v;
+    const SweepConst K = sweep_const<isU>(d.P);
+    HD_GLOBAL_AS double* tz = d.t_z;
+    HD_GLOBAL_AS double* tq = isU ? d.t_u : d.t_v;
     const double* hh = d.h;
     const int nbr = (lane + 1) & (kWave - 1);
     /* rows per lane of the speculative forward sweep: 8 while the previous
      * sweep of this direction repaired many runs (a flow starting up), else
      * as few as the run needs; this sweep's repaired chunks are counted for
      * the next one (moved into place by the explicit pass that follows) */
-    const int minL = d.run_cnt[isU ? 2 : 3] > kAdaptRuns ? kSpecMaxL : 1;
+    const int minlg = d.run_cnt[isU ? 2 : 3] > kAdaptRuns ? kSpecMaxLg : 0;
     int* fails = d.flags + (isU ? 4 : 5);
     /* the extra last workgroup: the across edges' cells that no run holds */
     if (bnd && (int)blockIdx.x == (int)gridDim.x - 1) {
-        across_boundary<isU>(d, edge_runs(d), lane);
+        across_boundary<isU>(d, lane);
         return;
     }
     const RunSlice sl = run_slice(cnt, (int)gridDim.x - bnd);
     for (int ri = sl.start; ri < sl.end; ri += sl.step) {
         const int4 rn = runs[ri];
-        const int line = rn.x, first = rn.y, last = rn.z;
+        const int line = __builtin_amdgcn_readfirstlane(rn.x), first = __builtin_amdgcn_readfirstlane(rn.y),
+                  last = __builtin_amdgcn_readfirstlane(rn.z);
         if (line < sidx || line > eidx) continue;
         auto at = [&](int k) -> size_t { return isU ? (size_t)k * W + line : (size_t)line * W + k; };
         /* one round of loads: wall-flag depths (locate_segment_u / _v,
@@ -1339,11 +1471,12 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
         const double TZ_r = tz[at(last)];
         const double ub1 = isU ? d.ubt[line] : d.vbd[line];
         const double ub2 = isU ? d.ubp[line] : d.vbt[line];
-        PreRaw raw0;
-        {
-            const int k = first + lane <= last ? first + lane : last;
-            raw0 = isU ? pre_uz_ld(d, k, line) : pre_vz_ld(d, line, k);
-        }
+        /* element of position k, and the byte offset of position k + lane
+         * (at most the run's last) from it */
+        auto base = [&](int k) -> long { return isU ? (long)k * W + line : (long)line * W + k; };
+        const unsigned step = isU ? 8u * (unsigned)W : 8u;
+        auto cell_off = [&](int k) -> unsigned { return (unsigned)(k + lane <= last ? lane : last - k) * step; };
+        PreRaw raw = pre_ld_off<isU>(d, base(first), cell_off(first));
         const bool br1 = (first > 2) || ((first == 2) && ((hb0 + hb1) * 0.5 == ND));
         const bool br2 = isU ? (last < N) || ((last == N) && ((he0 + he1) * 0.5 == ND))
                              : (last < M) || ((last == M) && ((he0 + he1) * 0.5 == ND));
@@ -1352,117 +1485,128 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
         const int ru = (skind != S_OPEN) ? 2 * (last - 1 - first) + 1 : 2 * (last - 1 - first);
         double* gAp = d.Ap + (size_t)line * tw + 2 * first;
         double* gBp = d.Bp + (size_t)line * tw + 2 * first;
+        double x0 = 0, xn = 0; /* X(0), X(sn) */
         if (sn >= 0) {
             const int nch = sn / RW + 1;
             double ap = 0, bp = 0, xs = 0;
+            double ap0 = 0, bp0 = 0; /* row 0's factors */
+            /* rows of chunk c that the sweeps take: rb .. rb + n - 1 */
+            auto chunk_rows = [&](int c, int& rb, int& n) {
+                const int re = RW * (c + 1) - 1 < sn - 1 ? RW * (c + 1) - 1 : sn - 1;
+                rb = c == 0 ? 1 : RW * c;
+                n = re - rb + 1;
+            };
             for (int c = 0; c < nch; ++c) {
                 const int c0 = first + CH * c;
-                const int rb = RW * c;
-                const int re = (rb + RW - 1 < sn) ? rb + RW - 1 : sn;
-                /* cells t = lane + 64 h; the loads of h + 1 are issued before
-                 * the rows of h are computed */
-                auto eval_cell = [&](int h, bool have_raw) -> Pre {
-                    const int k = c0 + lane + kWave * h;
-                    PreRaw r;
-                    if (have_raw) r = raw0;
-                    else {
-                        const int kc = k <= last ? k : last;
-                        r = isU ? pre_uz_ld(d, kc, line) : pre_vz_ld(d, line, kc);
+                int rb, n;
+                chunk_rows(c, rb, n);
+                const SpecMap sm = spec_map(n, minlg);
+                /* 63 cells a round (lane 63 holds the next round's first,
+                 * for its coefficients); the next round's loads travel while
+                 * this one's rows are computed */
+                const int c1 = c0 + CH - 1 < last ? c0 + CH - 1 : last; /* the chunk's last cell */
+                if (c > 0) raw = pre_ld_off<isU>(d, base(c0), cell_off(c0));
+#pragma unroll 1
+                for (int k0 = c0; k0 <= c1; k0 += 63) {
+                    const PreRaw cur = raw;
+                    if (k0 + 63 <= c1) raw = pre_ld_off<isU>(d, base(k0 + 63), cell_off(k0 + 63));
+                    const int k = k0 + lane;
+                    const bool mom = k < last, inner = last - 1 > first;
+                    const bool useA = inner && !(br1 && k == first), useC = inner && !(br2 && k == last - 1);
+                    CellRow o = cell_rows_rcp(K, cur, f4, mom, useA, useC);
+                    if (__any(o.bad)) {
+                        const Pre pa = isU ? pre_uz_ev(d.P, cur) : pre_vz_ev(d.P, cur);
+                        const Pre pb = shfl_pre(pa, nbr);
+                        const Mom mm = abcd(pa, pb, f4, k, first, last, br1, br2);
+                        o.a1 = mm.a1; o.b1 = mm.b1; o.c1 = mm.c1; o.d1 = mm.d1;
                     }
-                    const Pre a = isU ? pre_uz_ev(d.P, r) : pre_vz_ev(d.P, r);
-                    if (k == first) { sE[0] = a.a2; sE[1] = a.c2; sE[2] = a.d2; }
-                    if (k == last) { sE[3] = a.a2; sE[4] = a.c2; sE[5] = a.d2; }
-                    return a;
-                };
-                Pre cur = eval_cell(0, c == 0);
-#pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    if (c0 + kWave * h > last) break; /* uniform */
-                    const bool more = h < 3 && c0 + kWave * (h + 1) <= last;
-                    Pre nxt = cur;
-                    if (more) nxt = eval_cell(h + 1, false);
-                    const Pre nA = shfl_pre(cur, nbr); /* cell t + 1 of lanes 0 .. 62 */
-                    const Pre nB = shfl_pre(nxt, 0);   /* cell t + 1 of lane 63 */
-                    const int t = lane + kWave * h;
-                    const int k = c0 + t;
-                    if (t < CH && k <= last) {
-                        Pre b = cur;
-                        if (k + 1 <= last) b = (lane < kWave - 1) ? nA : nB;
-                        for (int e = 0; e < 2; ++e) {
-                            int rr = 2 * (k - first) + e;
-                            if (rr > sn) break;
-                            Row4 w = cell_row(cur, b, f4, k, e, first, last, br1, br2, skind, ekind, sn, ub1, ub2, TZ_l,
-                                              TZ_r);
-                            int ix = rr - rb;
-                            sA[ix] = w.A; sB[ix] = w.B; sC[ix] = w.C; sD[ix] = w.D;
+                    if (k == first) { sE[0] = o.a2; sE[1] = o.c2; sE[2] = o.d2; }
+                    if (k == last) { sE[3] = o.a2; sE[4] = o.c2; sE[5] = o.d2; }
+                    /* rows 2 (k - first) and the one after: continuity of k
+                     * and momentum of k, or from an open start momentum of k
+                     * and continuity of k + 1; the end row's condition wins */
+                    int rc = 2 * (k - first), rm = rc + 1;
+                    double md = o.d1, cd = o.d2;
+                    if (skind == S_OPEN) {
+                        rm = rc++;
+                        o.a2 = o.na2; o.c2 = o.nc2; o.d2 = cd = o.nd2;
+                        if (rm == 0) md = o.d1 - o.a1 * TZ_l;
+                    } else if (skind == S_Q) {
+                        if (rc == 0) cd = o.d2 - o.a2 * ub1;
+                    }
+                    if (ekind == E_OPEN) {
+                        if (rm == sn) md = o.d1 - o.c1 * TZ_r;
+                    } else if (rc == sn) {
+                        cd = ekind == E_Q ? o.d2 - o.c2 * ub2 : o.d2;
+                    }
+                    if (lane < 63 && k <= c1) {
+                        if (rc <= sn) {
+                            const int ix = rc == 0 ? kRow0 : (rc == sn ? kRowN : sm.pos(rc - rb));
+                            sA[ix] = o.a2; sB[ix] = 1.0; sC[ix] = o.c2; sD[ix] = cd;
+                        }
+                        if (rm <= sn) {
+                            const int ix = rm == 0 ? kRow0 : (rm == sn ? kRowN : sm.pos(rm - rb));
+                            sA[ix] = o.a1; sB[ix] = o.b1; sC[ix] = o.c1; sD[ix] = md;
                         }
                     }
-                    cur = nxt;
                 }
                 __syncthreads();
-                int g0 = 0;
                 if (c == 0) {
                     if (sn == 0) {
-                        xs = sD[0] / sB[0];
+                        xs = sD[kRow0] / sB[kRow0];
                     } else {
-                        ap = -sC[0] / sB[0];
-                        bp = sD[0] / sB[0];
+                        ap0 = ap = -sC[kRow0] / sB[kRow0];
+                        bp0 = bp = sD[kRow0] / sB[kRow0];
                     }
-                    g0 = 1;
                 }
-                const int g1 = (re < sn - 1 ? re : sn - 1) - rb;
-                spec_forward<true>(sA, sB, sC, sD, g0, g1, ap, bp, minL, fails);
-                if (c == 0 && sn > 0) {
-                    __syncthreads();
-                    if (lane == 0) { sC[0] = -sC[0] / sB[0]; sD[0] = sD[0] / sB[0]; }
-                }
-                if (re == sn && sn > 0) {
-                    double A = sA[sn - rb], B = sB[sn - rb], D = sD[sn - rb];
+                spec_forward<kSpecMaxLg>(sA, sB, sC, sD, sm, n, ap, bp, fails);
+                if (c == nch - 1 && sn > 0) {
+                    const double A = sA[kRowN], B = sB[kRowN], D = sD[kRowN];
                     xs = (D - (A * bp)) / (B + (A * ap));
                 }
-                __syncthreads();
-                if (c + 1 < nch) { /* factors of this chunk (rows rb .. re, all < sn) to the line buffers */
-                    for (int i = lane; i <= re - rb; i += kWave) { gAp[rb + i] = sC[i]; gBp[rb + i] = sD[i]; }
+                if (c + 1 < nch) { /* this chunk's factors to the line buffers */
+                    for (int r = lane; r < n; r += kWave) {
+                        gAp[rb + r] = sC[sm.pos(r)];
+                        gBp[rb + r] = sD[sm.pos(r)];
+                    }
                     __syncthreads();
                 }
             }
             /* back substitution, last chunk first; x[r] replaces A[r] */
             double xc = xs;
             for (int c = nch - 1; c >= 0; --c) {
-                const int rb = RW * c;
-                const int re = (rb + RW - 1 < sn) ? rb + RW - 1 : sn;
+                int rb, n;
+                chunk_rows(c, rb, n);
+                const SpecMap sm = spec_map(n, minlg);
                 if (c + 1 < nch) {
                     __syncthreads();
-                    for (int i = lane; i <= re - rb; i += kWave) { sC[i] = gAp[rb + i]; sD[i] = gBp[rb + i]; }
-                    __syncthreads();
-                } else if (lane == 0) {
-                    sA[sn - rb] = xs;
-                }
-                const int hi = (re < sn - 1 ? re : sn - 1) - rb;
-                xc = spec_backward(sC, sD, sA, hi, xc);
-                __syncthreads();
-                /* scatter the unknowns of positions first .. last-1 */
-                for (int i = lane; i <= re - rb; i += kWave) {
-                    int r = rb + i;
-                    double x = sA[i];
-                    int k;
-                    bool isz;
-                    if (skind != S_OPEN) { k = first + (r >> 1); isz = (r & 1) == 0; }
-                    else { isz = (r & 1) == 1; k = first + ((r + 1) >> 1); }
-                    if (k < last) {
-                        if (isz) tz[at(k)] = x; else tq[at(k)] = x;
+                    for (int r = lane; r < n; r += kWave) {
+                        sC[sm.pos(r)] = gAp[rb + r];
+                        sD[sm.pos(r)] = gBp[rb + r];
                     }
-                    if (r == 0) sX[0] = x;
-                    if (r == sn) sX[1] = x;
-                    if (r == ru) sX[2] = x;
+                    __syncthreads();
+                }
+                xc = spec_backward<kSpecMaxLg>(sC, sD, sA, sm, n, xc);
+                if (c == 0 && sn > 0) xc = bp0 + (ap0 * xc);
+                /* scatter the unknowns of positions first .. last-1 */
+                const int r0 = c == 0 ? 0 : rb, r1 = c == nch - 1 ? sn : rb + n - 1;
+                for (int r = r0 + lane; r <= r1; r += kWave) {
+                    const double x = r == sn ? xs : (r == 0 ? xc : sA[sm.pos(r - rb)]);
+                    const int rq = skind != S_OPEN ? r : r + 1; /* even: z of position first + rq / 2, odd: its velocity */
+                    const int kk = (rq >> 1) - (r0 >> 1);
+                    const bool isz = (r & 1) == (skind != S_OPEN ? 0 : 1);
+                    if (first + (rq >> 1) < last) st_off(isz ? tz : tq, base(first + (r0 >> 1)), (unsigned)kk * step, x);
+                    if (r == ru) sX[0] = x;
                 }
             }
+            x0 = xc;
+            xn = xs;
         } else {
             /* no system (one-cell run at an open start edge): the cell's
              * preindex is still needed at the end (first == last: lane 0
              * loaded it) */
             if (lane == 0) {
-                Pre a = isU ? pre_uz_ev(d.P, raw0) : pre_vz_ev(d.P, raw0);
+                Pre a = isU ? pre_uz_ev(d.P, raw) : pre_vz_ev(d.P, raw);
                 sE[3] = a.a2; sE[4] = a.c2; sE[5] = a.d2;
             }
         }
@@ -1471,16 +1615,16 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
             if (first < last) {
                 if (br1) tq[at(first - 1)] = 0;
                 else if (dkQ1 && first == 2) tq[at(first - 1)] = ub1;
-                else if (sn >= 0) tq[at(first - 1)] = (sE[2] - TZ_l - sE[1] * sX[0]) / sE[0];
+                else if (sn >= 0) tq[at(first - 1)] = (sE[2] - TZ_l - sE[1] * x0) / sE[0];
             }
             if (br2) {
                 tq[at(last)] = 0;
-                if (sn >= 0) tz[at(last)] = sX[1];
+                if (sn >= 0) tz[at(last)] = xn;
             } else if (dkQ2 && last == dkfr) {
                 tq[at(last)] = ub2;
-                if (sn >= 0) tz[at(last)] = sX[1];
+                if (sn >= 0) tz[at(last)] = xn;
             } else {
-                double prev = (first < last && sn >= 0) ? sX[2] : tq[at(last - 1)];
+                double prev = (first < last && sn >= 0) ? sX[0] : tq[at(last - 1)];
                 tq[at(last)] = (sE[5] - sE[3] * prev - TZ_r) / sE[4];
             }
         }
@@ -3108,14 +3252,16 @@ __global__ void k_thomas_batch(int nsys, const int* off, const int* sn, const do
 /* One wave per system: the speculative parallel Thomas of the run solvers
  * (hd_thomas.h) on a caller's system, rows in LDS chunks of 510, the
  * factors of earlier chunks through Ap / Bp (as k_adi_spec spills them).
- * The same bits as k_thomas_batch; systems outside rows [0, nrows) are
- * skipped the same way. */
+ * The same bits as the serial solve of tridiag
+ * (UVZSolver_multithread.cu:203-228); a system outside rows [0, nrows) is
+ * skipped (its x is left as it is): the host checks the tables where it
+ * holds them, and this check covers tables that only the device holds. */
 __global__ void __launch_bounds__(64) k_thomas_spec(int nsys, const int* off, const int* sn, const double* A,
                                                     const double* B, const double* C, const double* D, double* x,
                                                     double* Ap, double* Bp, int nrows)
 {
     constexpr int RW = 510;
-    __shared__ double sA[RW], sB[RW], sC[RW], sD[RW];
+    __shared__ double sA[spec_words(RW)], sB[spec_words(RW)], sC[spec_words(RW)], sD[spec_words(RW)];
     const int s = blockIdx.x, lane = threadIdx.x;
     if (s >= nsys) return;
     const int o = off[s], n = sn[s];
@@ -3124,50 +3270,46 @@ __global__ void __launch_bounds__(64) k_thomas_spec(int nsys, const int* off, co
         if (lane == 0) x[o] = D[o] / B[o];
         return;
     }
-    const int nch = n / RW + 1;
-    double ap = 0, bp = 0, xs = 0;
+    /* rows 1 .. n - 1 in chunks of RW; row 0 gives the entry state */
+    const double ap0 = -C[o] / B[o], bp0 = D[o] / B[o];
+    const double An = A[o + n], Bn = B[o + n], Dn = D[o + n];
+    const int nch = n > 1 ? (n - 2) / RW + 1 : 0;
+    double ap = ap0, bp = bp0;
     for (int c = 0; c < nch; ++c) {
-        const int rb = RW * c;
-        const int re = rb + RW - 1 < n ? rb + RW - 1 : n;
-        for (int i = lane; i <= re - rb; i += kWave) {
-            sA[i] = A[o + rb + i]; sB[i] = B[o + rb + i]; sC[i] = C[o + rb + i]; sD[i] = D[o + rb + i];
+        const int rb = 1 + RW * c, nr = n - rb < RW ? n - rb : RW;
+        const SpecMap sm = spec_map(nr);
+        for (int i = lane; i < nr; i += kWave) {
+            const int p = sm.pos(i);
+            sA[p] = A[o + rb + i]; sB[p] = B[o + rb + i]; sC[p] = C[o + rb + i]; sD[p] = D[o + rb + i];
         }
         __syncthreads();
-        int g0 = 0;
-        if (c == 0) {
-            ap = -sC[0] / sB[0];
-            bp = sD[0] / sB[0];
-            g0 = 1;
-        }
-        const int g1 = (re < n - 1 ? re : n - 1) - rb;
-        hd_spec::spec_forward<true>(sA, sB, sC, sD, g0, g1, ap, bp);
-        if (c == 0) {
-            __syncthreads();
-            if (lane == 0) { sC[0] = -sC[0] / sB[0]; sD[0] = sD[0] / sB[0]; }
-        }
-        if (re == n) xs = (sD[n - rb] - (sA[n - rb] * bp)) / (sB[n - rb] + (sA[n - rb] * ap));
-        __syncthreads();
+        spec_forward<kSpecMaxLg>(sA, sB, sC, sD, sm, nr, ap, bp);
         if (c + 1 < nch) {
-            for (int i = lane; i <= re - rb; i += kWave) { Ap[o + rb + i] = sC[i]; Bp[o + rb + i] = sD[i]; }
+            for (int i = lane; i < nr; i += kWave) {
+                Ap[o + rb + i] = sC[sm.pos(i)];
+                Bp[o + rb + i] = sD[sm.pos(i)];
+            }
             __syncthreads();
         }
     }
-    if (lane == 0) x[o + n] = xs;
-    double xc = xs;
+    double xc = (Dn - (An * bp)) / (Bn + (An * ap));
+    if (lane == 0) x[o + n] = xc;
     for (int c = nch - 1; c >= 0; --c) {
-        const int rb = RW * c;
-        const int re = rb + RW - 1 < n ? rb + RW - 1 : n;
+        const int rb = 1 + RW * c, nr = n - rb < RW ? n - rb : RW;
+        const SpecMap sm = spec_map(nr);
         if (c + 1 < nch) {
             __syncthreads();
-            for (int i = lane; i <= re - rb; i += kWave) { sC[i] = Ap[o + rb + i]; sD[i] = Bp[o + rb + i]; }
+            for (int i = lane; i < nr; i += kWave) {
+                sC[sm.pos(i)] = Ap[o + rb + i];
+                sD[sm.pos(i)] = Bp[o + rb + i];
+            }
             __syncthreads();
         }
-        const int hi = (re < n - 1 ? re : n - 1) - rb;
-        xc = hd_spec::spec_backward(sC, sD, sA, hi, xc);
-        __syncthreads();
-        for (int i = lane; i <= hi; i += kWave) x[o + rb + i] = sA[i];
+        xc = spec_backward<kSpecMaxLg>(sC, sD, sA, sm, nr, xc);
+        for (int i = lane; i < nr; i += kWave) x[o + rb + i] = sA[sm.pos(i)];
         __syncthreads();
     }
+    if (lane == 0) x[o] = bp0 + (ap0 * xc);
 }
 
 } // namespace

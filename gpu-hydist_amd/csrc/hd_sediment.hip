@@ -529,7 +529,11 @@ __global__ void __launch_bounds__(64) k_fs_spec(const HdDev* __restrict__ dv, do
 {
     const HdDevG& d = dev_view(dv);
     constexpr int RW = 256;
-    __shared__ double sA[RW], sB[RW], sC[RW], sD[RW]; /* rows; factors replace C / D, x replaces A */
+    /* rows at SpecMap positions (factors replace C / D, x replaces A); the
+     * run's first row (0) and last (sn), which the sweeps leave out, at the
+     * last two words */
+    constexpr int kW = hd_spec::spec_words(RW), kRow0 = kW - 2, kRowN = kW - 1;
+    __shared__ double sA[kW], sB[kW], sC[kW], sD[kW];
     __shared__ double sV[2]; /* clamped x of the first and last row */
     const int N = d.N, M = d.M, W = d.W;
     const int lane = threadIdx.x;
@@ -553,62 +557,69 @@ __global__ void __launch_bounds__(64) k_fs_spec(const HdDev* __restrict__ dv, do
         double* gBp = d.Bp + (size_t)line * tw + k0;
         const int nch = sn / RW + 1;
         double ap = 0, bp = 0, xs = 0;
+        double ap0 = 0, bp0 = 0; /* row 0's factors */
+        /* rows of chunk c that the sweeps take: rb .. rb + n - 1 */
+        auto chunk_rows = [&](int c, int& rb, int& n) {
+            const int re = RW * (c + 1) - 1 < sn - 1 ? RW * (c + 1) - 1 : sn - 1;
+            rb = c == 0 ? 1 : RW * c;
+            n = re - rb + 1;
+        };
         for (int c = 0; c < nch; ++c) {
-            const int rb = RW * c;
-            const int re = (rb + RW - 1 < sn) ? rb + RW - 1 : sn;
-            for (int r = rb + lane; r <= re; r += 64) {
+            int rb, n;
+            chunk_rows(c, rb, n);
+            const hd_spec::SpecMap sm = hd_spec::spec_map(n);
+            const int ra = RW * c, re = ra + RW - 1 < sn ? ra + RW - 1 : sn; /* assembled rows */
+            for (int r = ra + lane; r <= re; r += 64) {
                 const int k = k0 + r;
                 const int i = isJ ? k : line, j = isJ ? line : k;
-                FsRow w = fs_row<isJ>(d, t, s_start, ketdinh, i, j, first, last, br1, br2);
-                sA[r - rb] = w.A; sB[r - rb] = w.B; sC[r - rb] = w.C; sD[r - rb] = w.D;
+                const FsRow w = fs_row<isJ>(d, t, s_start, ketdinh, i, j, first, last, br1, br2);
+                const int p = r == 0 ? kRow0 : (r == sn ? kRowN : sm.pos(r - rb));
+                sA[p] = w.A; sB[p] = w.B; sC[p] = w.C; sD[p] = w.D;
             }
             __syncthreads();
-            int g0 = 0;
             if (c == 0) {
                 if (sn == 0) {
-                    xs = sD[0] / sB[0];
+                    xs = sD[kRow0] / sB[kRow0];
                 } else {
-                    ap = -sC[0] / sB[0];
-                    bp = sD[0] / sB[0];
+                    ap0 = ap = -sC[kRow0] / sB[kRow0];
+                    bp0 = bp = sD[kRow0] / sB[kRow0];
                 }
-                g0 = 1;
             }
-            const int g1 = ((re < sn - 1) ? re : sn - 1) - rb;
-            hd_spec::spec_forward<false>(sA, sB, sC, sD, g0, g1, ap, bp);
-            if (c == 0 && sn > 0) {
-                __syncthreads();
-                if (lane == 0) { sC[0] = -sC[0] / sB[0]; sD[0] = sD[0] / sB[0]; }
-            }
-            if (re == sn && sn > 0) {
-                double A = sA[sn - rb], B = sB[sn - rb], D = sD[sn - rb];
+            hd_spec::spec_forward<2>(sA, sB, sC, sD, sm, n, ap, bp);
+            if (c == nch - 1 && sn > 0) {
+                const double A = sA[kRowN], B = sB[kRowN], D = sD[kRowN];
                 xs = (D - (A * bp)) / (B + (A * ap));
             }
-            __syncthreads();
             if (c + 1 < nch) {
-                for (int q = lane; q <= re - rb; q += 64) { gAp[rb + q] = sC[q]; gBp[rb + q] = sD[q]; }
+                for (int r = lane; r < n; r += 64) {
+                    gAp[rb + r] = sC[sm.pos(r)];
+                    gBp[rb + r] = sD[sm.pos(r)];
+                }
                 __syncthreads();
             }
         }
         double xc = xs;
         for (int c = nch - 1; c >= 0; --c) {
-            const int rb = RW * c;
-            const int re = (rb + RW - 1 < sn) ? rb + RW - 1 : sn;
+            int rb, n;
+            chunk_rows(c, rb, n);
+            const hd_spec::SpecMap sm = hd_spec::spec_map(n);
             if (c + 1 < nch) {
                 __syncthreads();
-                for (int q = lane; q <= re - rb; q += 64) { sC[q] = gAp[rb + q]; sD[q] = gBp[rb + q]; }
+                for (int r = lane; r < n; r += 64) {
+                    sC[sm.pos(r)] = gAp[rb + r];
+                    sD[sm.pos(r)] = gBp[rb + r];
+                }
                 __syncthreads();
-            } else if (lane == 0) {
-                sA[sn - rb] = xs;
             }
-            const int hi = ((re < sn - 1) ? re : sn - 1) - rb;
-            xc = hd_spec::spec_backward(sC, sD, sA, hi, xc);
-            __syncthreads();
-            for (int q = lane; q <= re - rb; q += 64) {
-                double v = sA[q];
+            xc = hd_spec::spec_backward<2>(sC, sD, sA, sm, n, xc);
+            if (c == 0 && sn > 0) xc = bp0 + (ap0 * xc);
+            const int r0 = c == 0 ? 0 : rb, r1 = c == nch - 1 ? sn : rb + n - 1;
+            for (int r = r0 + lane; r <= r1; r += 64) {
+                double v = r == sn ? xs : (r == 0 ? xc : sA[sm.pos(r - rb)]);
                 if (v < 0) v = d.P.NDnen;
-                d.tFS[at(k0 + rb + q)] = v;
-                if (rb + q == 0) sV[0] = v;
-                if (rb + q == sn) sV[1] = v;
+                d.tFS[at(k0 + r)] = v;
+                if (r == 0) sV[0] = v;
+                if (r == sn) sV[1] = v;
             }
         }
         __syncthreads();

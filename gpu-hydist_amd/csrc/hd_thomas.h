@@ -7,6 +7,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "hd_fastdiv.h"
+
 namespace hd_spec {
 
 constexpr int kSpecWave = 64;
@@ -28,7 +30,7 @@ constexpr int kSpecWave = 64;
  * few ulps apart become bit-identical after a few tens of rows.  A lane
  * therefore runs the exact recurrence -- the same IEEE operations in the same
  * order as the serial solve -- from the estimate of the state kSpecWF rows
- * (rounded up to whole lanes) before its own rows, through its own rows, and
+ * before its own rows, through its own rows, and
  * the result is verified exactly: the state a lane had on entering its rows
  * must equal, bit for bit, the state its predecessor produced at its last
  * row.  Lane 0 starts from the exact state; by induction every lane that
@@ -39,19 +41,60 @@ constexpr int kSpecWave = 64;
  * (L = rows per lane).  Back substitution, x_i = bp_i + ap_i x_{i+1}, is an
  * affine chain and is treated the same way with 2-entry affine maps.
  *
- * Repairs (spec_forward<true>, the ADI sweeps): while a flow starts from
+ * What bounds it, and the layout.  One wave works alone on a run, so the time
+ * is the length of its dependent chain: about 7 cycles per FP64 operation, 75
+ * per division, 65 per LDS read that is waited for, 140 per row with two
+ * divisions, and 50 more where a row sits behind its own branch
+ * (microbenchmarks on this part).  Hence
+ *  - the rows per lane L are a power of two, known to the compiler (one copy
+ *    of the sweep for each), and row r sits at LDS position
+ *    (r mod L) * S + r / L: the lanes of a step read consecutive words
+ *    whatever L is, every row of the warm-up is at a fixed distance, and no
+ *    row needs a branch: rows that a lane's warm-up would read outside the
+ *    sweep are identity rows written there (16 before row 0, which hand on
+ *    the entry state, and 32 identity factors after the last row for the
+ *    back substitution);
+ *  - a row takes one reciprocal for its two quotients (hd_fastdiv.h), with
+ *    the division's own bits (95 cycles); where a value leaves the range in
+ *    which that holds, the wave runs the sweep again with divisions;
+ *  - matrices are normalised once per lane before the scan, not in it (64
+ *    factors with entries at most 1 stay far inside the exponent range, and
+ *    an estimate that does overflow only costs a repair).
+ *
+ * Repairs: while a flow starts from
  * rest, bp decays ahead of the waves as fast as the estimate's relative
  * error and never merges, so long stretches of lanes fail with their ap
  * already exact.  Then every row's divisor is known, and a failing lane
- * redoes only its bp chain, from registers, with the division in
- * Markstein's reciprocal form (bp_known_e) -- the same rounding as the
- * division; spec_forward<false> (the FS sweeps, which need the registers
- * for occupancy) keeps the plain repair. */
+ * redoes only its bp chain, from registers, with known reciprocals. */
 constexpr int kSpecWF = 16;           /* forward warm-up rows after the estimate */
 constexpr int kSpecWB = 32;           /* back-substitution warm-up rows */
-constexpr int kSpecSerialF = 32;      /* up to this many rows the forward sweep stays on one lane */
-constexpr int kSpecSerialB = 96;      /* likewise for back substitution */
-constexpr int kSpecMaxL = 8;          /* rows per lane of one speculative sweep (chunks <= 512 rows) */
+constexpr int kSpecMaxLg = 3;         /* rows per lane of one sweep: 1, 2, 4 or 8 */
+
+/* words between the planes r mod L of an LDS array: the warm-up before row
+ * 0, 64 lanes, the back substitution's warm-up after them */
+constexpr int spec_stride(int lg) { return kSpecWave + ((kSpecWF + kSpecWB) >> lg); }
+/* LDS position of row r (>= -kSpecWF) with 2^lg rows per lane */
+struct SpecMap {
+    int lg;
+    __device__ __forceinline__ int pos(int r) const
+    {
+        return ((r + kSpecWF) & ((1 << lg) - 1)) * (kSpecWave + ((kSpecWF + kSpecWB) >> lg)) + ((r + kSpecWF) >> lg);
+    }
+};
+/* words per LDS array of a sweep of at most n rows, and two more, at
+ * spec_words(n) - 2 and - 1, for the caller's own use; a multiple of 64, so
+ * that one instruction reads the same position of two arrays */
+constexpr int spec_words(int n)
+{
+    int lg = 0;
+    while ((kSpecWave << lg) < n) ++lg;
+    return (((spec_stride(lg) << lg) + 2 + 63) / 64) * 64;
+}
+__device__ __forceinline__ SpecMap spec_map(int n, int minlg = 0)
+{
+    const int lg = n <= 64 ? 0 : (n <= 128 ? 1 : (n <= 256 ? 2 : 3));
+    return SpecMap{lg < minlg ? minlg : lg};
+}
 
 struct Mx {
     double a, b, c, d, e, f, g; /* [[a b 0] [c d 0] [e f g]] */
@@ -86,22 +129,22 @@ __device__ __forceinline__ Mx mx_mul(const Mx& X, const Mx& Y)
 }
 
 /* Scale by a power of two (exact) so the largest entry lies in [0.5, 1):
- * only ratios of the composed state matter. */
+ * only ratios of the composed state matter.  A zero, infinite or NaN maximum
+ * has exponent 0 here and leaves X as it is. */
 __device__ __forceinline__ void mx_norm(Mx& X)
 {
-    double m = fmax(fmax(fmax(fabs(X.a), fabs(X.b)), fmax(fabs(X.c), fabs(X.d))),
-                    fmax(fmax(fabs(X.e), fabs(X.f)), fabs(X.g)));
-    if (m > 0 && m <= 1.7976931348623157e308) {
-        int ex;
-        frexp(m, &ex);
-        double s = ldexp(1.0, -ex);
-        X.a *= s; X.b *= s; X.c *= s; X.d *= s; X.e *= s; X.f *= s; X.g *= s;
-    }
+    const double m = fmax(fmax(fmax(fabs(X.a), fabs(X.b)), fmax(fabs(X.c), fabs(X.d))),
+                          fmax(fmax(fabs(X.e), fabs(X.f)), fabs(X.g)));
+    const int s = -__builtin_amdgcn_frexp_exp(m);
+    X.a = __builtin_amdgcn_ldexp(X.a, s); X.b = __builtin_amdgcn_ldexp(X.b, s);
+    X.c = __builtin_amdgcn_ldexp(X.c, s); X.d = __builtin_amdgcn_ldexp(X.d, s);
+    X.e = __builtin_amdgcn_ldexp(X.e, s); X.f = __builtin_amdgcn_ldexp(X.f, s);
+    X.g = __builtin_amdgcn_ldexp(X.g, s);
 }
 
-/* A 64-bit value moved across lanes by a DPP mode (row shifts within rows
- * of 16 lanes, row broadcasts to later rows): a lane the mode gives no source,
- * or whose row ROWMASK leaves out, gets `old`. */
+/* A 64-bit value moved across lanes by a DPP mode (shifts by one lane, row
+ * shifts within rows of 16 lanes, row broadcasts to later rows): a lane the
+ * mode gives no source, or whose row ROWMASK leaves out, gets `old`. */
 template <int CTRL, int ROWMASK>
 __device__ __forceinline__ double dpp_f64(double old, double src)
 {
@@ -110,29 +153,39 @@ __device__ __forceinline__ double dpp_f64(double old, double src)
     const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(v >> 32), CTRL, ROWMASK, 0xF, false);
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
+/* the same where lanes without a source may get anything */
+template <int CTRL>
+__device__ __forceinline__ double dpp_any(double src)
+{
+    const long long v = __double_as_longlong(src);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+/* the previous lane's value (lane 0 keeps its own) */
+__device__ __forceinline__ double lane_before(double v) { return dpp_f64<0x138, 0xF>(v, v); }
 
 /* One step of the wave's inclusive prefix scan of row matrices: X := X Y
- * with Y the matrix of the source lane, the identity where there is none. */
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ void mx_scan_step(Mx& X)
+ * with Y the matrix of the source lane, where there is one (`has`). */
+template <int CTRL>
+__device__ __forceinline__ void mx_scan_step(Mx& X, bool has)
 {
     Mx Y;
-    Y.a = dpp_f64<CTRL, ROWMASK>(1.0, X.a); Y.b = dpp_f64<CTRL, ROWMASK>(0.0, X.b);
-    Y.c = dpp_f64<CTRL, ROWMASK>(0.0, X.c); Y.d = dpp_f64<CTRL, ROWMASK>(1.0, X.d);
-    Y.e = dpp_f64<CTRL, ROWMASK>(0.0, X.e); Y.f = dpp_f64<CTRL, ROWMASK>(0.0, X.f);
-    Y.g = dpp_f64<CTRL, ROWMASK>(1.0, X.g);
-    X = mx_mul(X, Y);
-    mx_norm(X);
+    Y.a = dpp_any<CTRL>(X.a); Y.b = dpp_any<CTRL>(X.b); Y.c = dpp_any<CTRL>(X.c); Y.d = dpp_any<CTRL>(X.d);
+    Y.e = dpp_any<CTRL>(X.e); Y.f = dpp_any<CTRL>(X.f); Y.g = dpp_any<CTRL>(X.g);
+    if (has) X = mx_mul(X, Y);
 }
 
 /* The same for the affine maps x -> al x + be of back substitution: the
  * source lane's map is applied first. */
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ void aff_scan_step(double& al, double& be)
+template <int CTRL>
+__device__ __forceinline__ void aff_scan_step(double& al, double& be, bool has)
 {
-    const double a2 = dpp_f64<CTRL, ROWMASK>(1.0, al), b2 = dpp_f64<CTRL, ROWMASK>(0.0, be);
-    be = fma(al, b2, be);
-    al = al * a2;
+    const double a2 = dpp_any<CTRL>(al), b2 = dpp_any<CTRL>(be);
+    if (has) {
+        be = fma(al, b2, be);
+        al = al * a2;
+    }
 }
 
 /* v of lane `l` (wave-uniform l) through the scalar unit */
@@ -149,287 +202,372 @@ __device__ __forceinline__ bool same_bits(double x, double y)
 }
 
 /* One exact forward row, in the operation order of tridiag. */
-__device__ __forceinline__ void thomas_row(const double* sA, const double* sB, const double* sC, const double* sD,
-                                           int i, double& ap, double& bp)
+__device__ __forceinline__ void thomas_row(double A, double B, double C, double D, double& ap, double& bp)
 {
-    double A = sA[i], B = sB[i], C = sC[i], D = sD[i];
-    double e = A * ap + B;
-    double nap = -C / e;
-    double nbp = (D - (A * bp)) / e;
+    const double e = A * ap + B;
+    const double nap = -C / e;
+    const double nbp = (D - (A * bp)) / e;
     ap = nap;
     bp = nbp;
 }
 
-/* bp of one forward row when its divisor e and y = RN(1/e) are known
- * (Markstein's correction: q0 = RN(n y) is within an ulp of n / e, the
- * remainder n - q0 e is exact by FMA, and RN(q0 + r y) is then RN(n / e)):
- * the bits of (D - A bp) / e with a multiply and two FMAs instead of a
- * division, valid where no intermediate underflows or overflows (|n| >=
- * 2^-960, |q0| in [2^-1000, 2^1000]; e and y are checked by the caller).
- * Branch-free: `off` is set when a row leaves that range, and the caller
- * then redoes the rows with divisions. */
-__device__ __forceinline__ double bp_known_e(double A, double D, double bp, double e, double y, bool& off)
+/* bp of a row whose divisor e and refined reciprocal y are known: the
+ * numerator is scaled up and the quotient down again (both exact while the
+ * quotient is a normal number or zero), so that a bp that decays towards
+ * the end of the exponent range stays in reach of the reciprocal form. */
+__device__ __forceinline__ double bp_known_e(double A, double D, double bp, double e, double y, hd_div::Range& rg)
 {
-    const double n = D - (A * bp);
-    const double q0 = n * y;
-    const double an = fabs(n), aq = fabs(q0);
-    off = off || !(an >= 0x1p-960 && an <= 0x1p1000 && aq >= 0x1p-1000 && aq <= 0x1p1000);
-    const double r = fma(-q0, e, n);
-    return fma(r, y, q0);
+    const double q = hd_div::quot((D - (A * bp)) * 0x1p300, e, y);
+    rg.num(q);
+    return q * 0x1p-300;
 }
 
-/* Forward elimination of LDS rows g0 .. g1 (chunk-relative), entering with
- * the exact state (ap, bp) of row g0 - 1, which is left as the state of row
- * g1.  The factors ap / bp of the rows replace C / D (after every lane has
- * read them: speculating lanes keep their own rows' factors in registers
- * until the sweep is verified).  At most 64 * kSpecMaxL rows; one wave,
- * uniform control; ends with a barrier. */
-template <bool kFastRepair>
-__device__ __forceinline__ void spec_forward(const double* sA, double* sB, double* sC, double* sD, int g0,
-                                             int g1, double& ap, double& bp, int minL = 1, int* fails = nullptr)
+/* A warm-up row: the same bits in all but extreme cases (whatever it
+ * returns is verified before it counts). */
+__device__ __forceinline__ void thomas_row_warm(double A, double B, double C, double D, double& ap, double& bp)
 {
+    const double e = A * ap + B;
+    const double y = hd_div::rcp_refined(e);
+    ap = hd_div::quot(C, -e, -y);
+    bp = hd_div::quot(D - (A * bp), e, y);
+}
+
+/* The row of thomas_row with one reciprocal for both quotients: its bits
+ * while rows_ok holds of `rg` and of the results (hd_fastdiv.h), if C and D
+ * are not -0 (then neither numerator is) and C is in range. */
+__device__ __forceinline__ void thomas_row_rcp(double A, double B, double C, double D, double& ap, double& bp,
+                                               hd_div::Range& rg)
+{
+    const double e = A * ap + B;
+    const double y = hd_div::rcp_refined(e);
+    rg.den(e);
+    ap = hd_div::quot(C, -e, -y);
+    bp = bp_known_e(A, D, bp, e, y, rg);
+}
+
+/* whether the scaled quotients stood for normal numbers or zeros */
+__device__ __forceinline__ bool rows_ok(const hd_div::Range& rg, double ap, double bp)
+{
+    return rg.den_ok() && rg.lo >= -720 && hd_div::finite(ap) && hd_div::finite(bp);
+}
+
+template <int LG>
+__device__ __forceinline__ void spec_forward_lg(double* sA, double* sB, double* sC, double* sD, int n, double& ap,
+                                                double& bp, int* fails)
+{
+    constexpr int L = 1 << LG, S = spec_stride(LG), m = kSpecWF >> LG; /* m: lanes of warm-up */
+    constexpr SpecMap sm{LG};
     const int lane = threadIdx.x;
-    const int n = g1 - g0 + 1;
-    if (n <= 0) return;
-    if (n <= kSpecSerialF) {
-        /* short sweep: lane 0 alone, factors written in place */
-        double ca = ap, cb = bp;
-        if (lane == 0) {
-#pragma unroll 4
-            for (int i = g0; i <= g1; ++i) {
-                thomas_row(sA, sB, sC, sD, i, ca, cb);
-                sC[i] = ca;
-                sD[i] = cb;
-            }
+    const int kl = (n - 1) >> LG;       /* the last lane with rows */
+    const bool act = lane <= kl;
+    const int own = lane + m;           /* position of the lane's first row */
+    /* rows -16 .. -1 hand on the entry state, rows after n - 1 fill the last lane */
+    if (lane < kSpecWF) {
+        const int p = sm.pos(lane - kSpecWF);
+        sA[p] = 0.0; sB[p] = 1.0; sC[p] = -ap; sD[p] = bp;
+    } else {
+        const int r = n + lane - kSpecWF;
+        if (r < ((kl + 1) << LG)) {
+            const int p = sm.pos(r);
+            sA[p] = 0.0; sB[p] = 1.0; sC[p] = 0.0; sD[p] = 0.0;
         }
-        ap = __shfl(ca, 0, kSpecWave);
-        bp = __shfl(cb, 0, kSpecWave);
-        __syncthreads();
-        return;
     }
-    /* rows per lane, <= kSpecMaxL: at least minL (more rows per lane, fewer
-     * lanes, a shorter chain of lane-by-lane repairs when speculation fails;
-     * the result is the same for any L) */
-    const int L0 = (n + kSpecWave - 1) / kSpecWave;
-    const int L = L0 < minL ? minL : L0;
-    const int sk = g0 + lane * L;
-    const int ek = sk + L <= g1 + 1 ? sk + L : g1 + 1;
-    const bool act = sk <= g1;
-    const int m = (kSpecWF + L - 1) / L;
-    const int j = lane - m - 1;
-    /* prefix estimates */
-    Mx X{1, 0, 0, 1, 0, 0, 1};
-    for (int i = sk; i < ek; ++i) {
-        X = mx_row(sA[i], sB[i], sC[i], sD[i], X);
-        if (((i - sk) & 3) == 3) mx_norm(X);
-    }
-    mx_norm(X);
-    /* inclusive scan over the wave with DPP moves: shifts by 1, 2, 4, 8
-     * within rows of 16 lanes, then the end of row r to row r + 1 (rows 1
-     * and 3), then the end of row 1 to rows 2 and 3; the estimates need not
-     * match any particular rounding */
-    mx_scan_step<0x111, 0xF>(X);
-    mx_scan_step<0x112, 0xF>(X);
-    mx_scan_step<0x114, 0xF>(X);
-    mx_scan_step<0x118, 0xF>(X);
-    mx_scan_step<0x142, 0xA>(X);
-    mx_scan_step<0x143, 0xC>(X);
-    double ea, eb;
-    {
-        double p = fma(X.a, ap, X.b), q = fma(X.c, ap, X.d), r = fma(X.e, ap, fma(X.g, bp, X.f));
-        ea = __shfl(p / q, j < 0 ? 0 : j, kSpecWave);
-        eb = __shfl(r / q, j < 0 ? 0 : j, kSpecWave);
-    }
-    const bool exact = j < 0;
-    double ca = exact ? ap : ea, cb = exact ? bp : eb;
-    int i0 = exact ? g0 : g0 + (j + 1) * L;
-    if (!act) i0 = sk;
-    /* warm-up rows, then the lane's own rows */
-    for (int i = i0; i < sk; ++i) thomas_row(sA, sB, sC, sD, i, ca, cb);
-    const double wa = ca, wb = cb;
-    double ra[kSpecMaxL], rb[kSpecMaxL];
+    __syncthreads();
+    /* the lane's own rows, composed, and what the reciprocal form asks of C and D */
+    double A[L], B[L], C[L], D[L];
+    bool nz = false;
+    hd_div::Range rc;
 #pragma unroll
-    for (int q = 0; q < kSpecMaxL; ++q) {
-        if (sk + q < ek) {
-            thomas_row(sA, sB, sC, sD, sk + q, ca, cb);
+    for (int q = 0; q < L; ++q) {
+        const int p = q * S + own;
+        A[q] = sA[p]; B[q] = sB[p]; C[q] = sC[p]; D[q] = sD[p];
+    }
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+        nz = nz || hd_div::neg_zero(C[q]) || hd_div::neg_zero(D[q]);
+        rc.num(C[q]);
+    }
+    const bool cd = !nz && rc.lo >= -900;
+    bool plain = __any(act && !cd);
+    const bool exact = lane <= m;       /* starts from the entry state */
+    double a0 = ap, b0 = bp;
+    if (n > kSpecWF + L) {              /* some lane needs an estimate */
+        Mx X{0.0, -C[0], A[0], B[0], 0.0, D[0], -A[0]};
+#pragma unroll
+        for (int q = 1; q < L; ++q) X = mx_row(A[q], B[q], C[q], D[q], X);
+        mx_norm(X);
+        /* inclusive scan over the wave with DPP moves: shifts by 1, 2, 4, 8
+         * within rows of 16 lanes, then the end of row r to row r + 1 (rows 1
+         * and 3), then the end of row 1 to rows 2 and 3; the estimates need
+         * not match any particular rounding */
+        mx_scan_step<0x111>(X, (lane & 15) >= 1);
+        mx_scan_step<0x112>(X, (lane & 15) >= 2);
+        mx_scan_step<0x114>(X, (lane & 15) >= 4);
+        mx_scan_step<0x118>(X, (lane & 15) >= 8);
+        mx_scan_step<0x142>(X, (lane & 16) != 0);
+        mx_scan_step<0x143>(X, lane >= 32);
+        const double p = fma(X.a, ap, X.b), q = fma(X.c, ap, X.d), r = fma(X.e, ap, fma(X.g, bp, X.f));
+        const double y = hd_div::rcp_refined(q);
+        const int j = exact ? 0 : lane - m - 1;
+        const double ea = __shfl(p * y, j, kSpecWave), eb = __shfl(r * y, j, kSpecWave);
+        a0 = exact ? ap : ea;
+        b0 = exact ? bp : eb;
+    }
+    /* warm-up rows, then the lane's own */
+    double ca, cb, wa, wb, ra[L], rb[L];
+    if (!plain) {
+        hd_div::Range rg;
+        ca = a0;
+        cb = b0;
+        double A4[4], B4[4], C4[4], D4[4];
+        auto fetch = [&](int t0) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int t = t0 + u, p = (t & (L - 1)) * S + lane + (t >> LG);
+                A4[u] = sA[p]; B4[u] = sB[p]; C4[u] = sC[p]; D4[u] = sD[p];
+            }
+        };
+        fetch(0);
+#pragma unroll
+        for (int t0 = 0; t0 < kSpecWF; t0 += 4) { /* four rows, the next four on their way */
+            double A3[4], B3[4], C3[4], D3[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) { A3[u] = A4[u]; B3[u] = B4[u]; C3[u] = C4[u]; D3[u] = D4[u]; }
+            if (t0 + 4 < kSpecWF) fetch(t0 + 4);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) thomas_row_warm(A3[u], B3[u], C3[u], D3[u], ca, cb);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (lane == 0) { ca = ap; cb = bp; }
+        wa = ca;
+        wb = cb;
+#pragma unroll
+        for (int q = 0; q < L; ++q) {
+            thomas_row_rcp(A[q], B[q], C[q], D[q], ca, cb, rg);
             ra[q] = ca;
             rb[q] = cb;
+        }
+        plain = __any(act && !rows_ok(rg, ca, cb));
+    }
+    if (plain) {
+        ca = a0;
+        cb = b0;
+#pragma unroll 1
+        for (int t = 0; t < kSpecWF; ++t) {
+            const int p = (t & (L - 1)) * S + lane + (t >> LG);
+            if (lane * L - kSpecWF + t >= 0) thomas_row(sA[p], sB[p], sC[p], sD[p], ca, cb);
+        }
+        wa = ca;
+        wb = cb;
+#pragma unroll 1
+        for (int t = 0; t < L; ++t) {
+            const int p = t * S + own;
+            thomas_row(sA[p], sB[p], sC[p], sD[p], ca, cb);
+#pragma unroll
+            for (int q = 0; q < L; ++q)
+                if (q == t) { ra[q] = ca; rb[q] = cb; }
         }
     }
     /* exact verification against the predecessor's last row */
     {
-        double pa = __shfl_up(ca, 1, kSpecWave), pb = __shfl_up(cb, 1, kSpecWave);
-        bool ok = exact || !act || (same_bits(wa, pa) && same_bits(wb, pb));
+        const double pa = lane_before(ca), pb = lane_before(cb);
+        bool ok = lane == 0 || !act || (same_bits(wa, pa) && same_bits(wb, pb));
         unsigned long long bad = __ballot(!ok);
-        if (bad && fails && lane == 0) atomicAdd(fails, 1);
-        if constexpr (kFastRepair) {
-            /* Where the flow starts from rest every failure has the lane's
-             * ap bits right (ap depends on A, B, C only and merges; bp decays
-             * ahead of the waves as fast as the estimate's error), so the
-             * lane's rows' divisors e are exact: every lane takes A, D, e
-             * and 1/e of its rows into registers once a failure is seen, and
-             * the repair of such a lane runs bp's chain in the reciprocal
-             * form (bp_known_e) with no LDS access; the predecessor's state
-             * moves through the scalar unit. */
-            double rA[kSpecMaxL], rD[kSpecMaxL], re[kSpecMaxL], ry[kSpecMaxL];
-            bool mk = false;
-            if (bad) {
-                mk = true;
+        if (bad) {
+            if (fails && lane == 0) atomicAdd(fails, 1);
+            /* where a failing lane's ap was right (ap depends on A, B, C only
+             * and merges) its divisors are, and it redoes bp's chain alone */
+            double e[L], y[L];
+            hd_div::Range rd;
 #pragma unroll
-                for (int q = 0; q < kSpecMaxL; ++q) {
-                    rA[q] = 0.0; rD[q] = 0.0; re[q] = 1.0; ry[q] = 1.0;
-                    if (sk + q < ek) {
-                        rA[q] = sA[sk + q];
-                        rD[q] = sD[sk + q];
-                        re[q] = rA[q] * (q == 0 ? wa : ra[q - 1]) + sB[sk + q];
-                        ry[q] = 1.0 / re[q];
-                        const double ae = fabs(re[q]);
-                        mk = mk && ae >= 0x1p-1000 && ae <= 0x1p1000;
-                    }
-                }
+            for (int q = 0; q < L; ++q) {
+                e[q] = A[q] * (q == 0 ? wa : ra[q - 1]) + B[q];
+                y[q] = hd_div::rcp_refined(e[q]);
+                rd.den(e[q]);
             }
+            const bool mk = !nz && rd.den_ok();
             while (bad) {
-                const int f = __ffsll((long long)bad) - 1; /* >= 1: lane 0 starts exact */
-                double fa = readlane_f64(ca, f - 1), fb = readlane_f64(cb, f - 1);
+                const int f = __ffsll((long long)bad) - 1; /* >= 1 */
+                const double fa = readlane_f64(ca, f - 1), fb = readlane_f64(cb, f - 1);
                 if (lane == f) {
-                    if (mk && same_bits(wa, fa)) {
-                        /* ap of the lane's rows is exact already: bp only */
-                        bool off = false;
+                    if (same_bits(wa, fa)) {
+                        hd_div::Range rn;
                         cb = fb;
 #pragma unroll
-                        for (int q = 0; q < kSpecMaxL; ++q) {
-                            if (sk + q < ek) {
-                                cb = bp_known_e(rA[q], rD[q], cb, re[q], ry[q], off);
-                                rb[q] = cb;
-                            }
+                        for (int q = 0; q < L; ++q) {
+                            cb = bp_known_e(A[q], D[q], cb, e[q], y[q], rn);
+                            rb[q] = cb;
                         }
-                        if (off) { /* a row outside the reciprocal form's range: divide */
+                        if (!(mk && rn.lo >= -720 && hd_div::finite(cb))) { /* outside the reciprocal form's range */
                             cb = fb;
 #pragma unroll
-                            for (int q = 0; q < kSpecMaxL; ++q) {
-                                if (sk + q < ek) {
-                                    cb = (rD[q] - (rA[q] * cb)) / re[q];
-                                    rb[q] = cb;
-                                }
+                            for (int q = 0; q < L; ++q) {
+                                cb = (D[q] - (A[q] * cb)) / e[q];
+                                rb[q] = cb;
                             }
                         }
                     } else {
                         ca = fa;
                         cb = fb;
 #pragma unroll
-                        for (int q = 0; q < kSpecMaxL; ++q) {
-                            if (sk + q < ek) {
-                                thomas_row(sA, sB, sC, sD, sk + q, ca, cb);
-                                ra[q] = ca;
-                                rb[q] = cb;
-                            }
-                        }
-                    }
-                }
-                double na = readlane_f64(ca, f), nb = readlane_f64(cb, f);
-                if (lane == f) ok = true;
-                if (lane == f + 1) ok = exact || !act || (same_bits(wa, na) && same_bits(wb, nb));
-                bad = __ballot(!ok);
-            }
-        } else {
-            while (bad) {
-                const int f = __ffsll((long long)bad) - 1; /* >= 1: lane 0 starts exact */
-                double fa = __shfl(ca, f - 1, kSpecWave), fb = __shfl(cb, f - 1, kSpecWave);
-                if (lane == f) {
-                    ca = fa;
-                    cb = fb;
-#pragma unroll
-                    for (int q = 0; q < kSpecMaxL; ++q) {
-                        if (sk + q < ek) {
-                            thomas_row(sA, sB, sC, sD, sk + q, ca, cb);
+                        for (int q = 0; q < L; ++q) {
+                            thomas_row(A[q], B[q], C[q], D[q], ca, cb);
                             ra[q] = ca;
                             rb[q] = cb;
                         }
                     }
                 }
-                double na = __shfl(ca, f, kSpecWave), nb = __shfl(cb, f, kSpecWave);
+                const double na = readlane_f64(ca, f), nb = readlane_f64(cb, f);
                 if (lane == f) ok = true;
-                if (lane == f + 1) ok = exact || !act || (same_bits(wa, na) && same_bits(wb, nb));
+                if (lane == f + 1) ok = !act || (same_bits(wa, na) && same_bits(wb, nb));
                 bad = __ballot(!ok);
             }
         }
     }
-    const int klast = (n - 1) / L;
-    ap = __shfl(ca, klast, kSpecWave);
-    bp = __shfl(cb, klast, kSpecWave);
+    {
+        const int ql = (n - 1) & (L - 1);
+        double ea = ra[0], eb = rb[0];
+#pragma unroll
+        for (int q = 1; q < L; ++q)
+            if (q == ql) { ea = ra[q]; eb = rb[q]; }
+        ap = readlane_f64(ea, kl);
+        bp = readlane_f64(eb, kl);
+    }
     __syncthreads(); /* every lane has read C / D */
 #pragma unroll
-    for (int q = 0; q < kSpecMaxL; ++q) {
-        if (sk + q < ek) {
-            sC[sk + q] = ra[q];
-            sD[sk + q] = rb[q];
+    for (int q = 0; q < L; ++q) {
+        if (lane * L + q < n) {
+            sC[q * S + own] = ra[q];
+            sD[q * S + own] = rb[q];
         }
     }
     __syncthreads();
 }
 
-/* Back substitution over LDS rows hi down to 0 (chunk-relative) given x of
- * row hi + 1; x_i goes to sX[i].  Returns x of row 0 (x_in when hi < 0). */
-__device__ __forceinline__ double spec_backward(const double* sAp, const double* sBp, double* sX, int hi, double x_in)
+/* Forward elimination of the n rows of a sweep (at sm.pos(r) of the LDS
+ * arrays), entering with the exact state (ap, bp) of the row before, which
+ * is left as the state of row n - 1.  The factors ap / bp of the rows replace
+ * C / D (after every lane has read them: speculating lanes keep their own
+ * rows' factors in registers until the sweep is verified).  n <= 64 L; one
+ * wave, uniform control; ends with a barrier.  fails: counts sweeps that
+ * needed a repair. */
+template <int MAXLG>
+__device__ __forceinline__ void spec_forward(double* sA, double* sB, double* sC, double* sD, const SpecMap& sm, int n,
+                                             double& ap, double& bp, int* fails = nullptr)
 {
+    if (n <= 0) return;
+    if (sm.lg == 0) spec_forward_lg<0>(sA, sB, sC, sD, n, ap, bp, fails);
+    else if (sm.lg == 1) spec_forward_lg<1>(sA, sB, sC, sD, n, ap, bp, fails);
+    else if (MAXLG == 2 || sm.lg == 2) spec_forward_lg<2>(sA, sB, sC, sD, n, ap, bp, fails);
+    else spec_forward_lg<3>(sA, sB, sC, sD, n, ap, bp, fails);
+}
+
+template <int LG>
+__device__ __forceinline__ double spec_backward_lg(double* sAp, double* sBp, double* sX, int n, double x_in)
+{
+    constexpr int L = 1 << LG, S = spec_stride(LG), m = kSpecWB >> LG;
+    constexpr SpecMap sm{LG};
     const int lane = threadIdx.x;
-    const int n = hi + 1;
-    if (n <= 0) return x_in;
-    const int L = n <= kSpecSerialB ? n : (n + kSpecWave - 1) / kSpecWave;
-    const int top = hi - lane * L;
-    const int bot = top - L + 1 >= 0 ? top - L + 1 : 0;
-    const bool act = top >= 0;
-    const int m = (kSpecWB + L - 1) / L;
-    const int j = lane - m - 1;
+    const int kl = (n - 1) >> LG;
+    /* identity factors (x = -0 + 1 x) where the warm-up reads past row n - 1 */
+    if (n + lane < ((kl + 1) << LG) + kSpecWB) {
+        const int p = sm.pos(n + lane);
+        sAp[p] = 1.0;
+        sBp[p] = -0.0;
+    }
+    __syncthreads();
+    /* wave lane l takes the rows of forward lane kl - l, so that the chain
+     * runs up the lanes */
+    const bool act = lane <= kl;
+    const int k = (act ? kl - lane : 0) + (kSpecWF >> LG);
+    double oa[L], ob[L]; /* the lane's own factors */
+#pragma unroll
+    for (int q = 0; q < L; ++q) { oa[q] = sAp[q * S + k]; ob[q] = sBp[q * S + k]; }
+    const bool exact = lane <= m;
     double cx = x_in;
-    int i0 = hi;
-    if (n > kSpecSerialB) {
-        double al = 1, be = 0;
-        for (int i = top; i >= bot; --i) {
-            be = fma(sAp[i], be, sBp[i]);
-            al = sAp[i] * al;
+    if (n > kSpecWB + L) {
+        double al = oa[L - 1], be = ob[L - 1];
+#pragma unroll
+        for (int q = L - 2; q >= 0; --q) {
+            be = fma(oa[q], be, ob[q]);
+            al = oa[q] * al;
         }
-        /* inclusive scan of the affine maps, DPP moves as in spec_forward */
-        aff_scan_step<0x111, 0xF>(al, be);
-        aff_scan_step<0x112, 0xF>(al, be);
-        aff_scan_step<0x114, 0xF>(al, be);
-        aff_scan_step<0x118, 0xF>(al, be);
-        aff_scan_step<0x142, 0xA>(al, be);
-        aff_scan_step<0x143, 0xC>(al, be);
-        double est = fma(al, x_in, be);
-        est = __shfl(est, j < 0 ? 0 : j, kSpecWave);
-        if (j >= 0) { cx = est; i0 = hi - (j + 1) * L; }
+        /* inclusive scan of the affine maps, DPP moves as in the forward sweep */
+        aff_scan_step<0x111>(al, be, (lane & 15) >= 1);
+        aff_scan_step<0x112>(al, be, (lane & 15) >= 2);
+        aff_scan_step<0x114>(al, be, (lane & 15) >= 4);
+        aff_scan_step<0x118>(al, be, (lane & 15) >= 8);
+        aff_scan_step<0x142>(al, be, (lane & 16) != 0);
+        aff_scan_step<0x143>(al, be, lane >= 32);
+        const double est = __shfl(fma(al, x_in, be), exact ? 0 : lane - m - 1, kSpecWave);
+        cx = exact ? x_in : est;
     }
-    const bool exact = j < 0;
-    if (!act) i0 = top;
-    for (int i = i0; i > top; --i) cx = sBp[i] + (sAp[i] * cx);
+    /* warm-up: the 32 rows above the lane's, last first */
+    {
+        double a8[8], b8[8];
+        auto fetch = [&](int t0) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int t = kSpecWB - 1 - t0 - u, p = (t & (L - 1)) * S + k + 1 + (t >> LG);
+                a8[u] = sAp[p];
+                b8[u] = sBp[p];
+            }
+        };
+        fetch(0);
+#pragma unroll
+        for (int t0 = 0; t0 < kSpecWB; t0 += 8) { /* eight rows, the next eight on their way */
+            double a[8], b[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) { a[u] = a8[u]; b[u] = b8[u]; }
+            if (t0 + 8 < kSpecWB) fetch(t0 + 8);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) cx = b[u] + (a[u] * cx);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
     const double w = cx;
-#pragma unroll 8
-    for (int i = (top < i0 ? top : i0); i >= bot; --i) {
-        cx = sBp[i] + (sAp[i] * cx);
-        sX[i] = cx;
-    }
-    if (n > kSpecSerialB) {
-        double px = __shfl_up(cx, 1, kSpecWave);
+    auto rows = [&]() {
+#pragma unroll
+        for (int q = L - 1; q >= 0; --q) {
+            cx = ob[q] + (oa[q] * cx);
+            sX[q * S + k] = cx;
+        }
+    };
+    if (act) rows();
+    {
+        const double px = lane_before(cx);
         bool ok = exact || !act || same_bits(w, px);
         unsigned long long bad = __ballot(!ok);
         while (bad) {
             const int f = __ffsll((long long)bad) - 1;
-            __syncthreads();
+            const double fx = readlane_f64(cx, f - 1);
             if (lane == f) {
-                cx = sX[top + 1];
-                for (int i = top; i >= bot; --i) {
-                    cx = sBp[i] + (sAp[i] * cx);
-                    sX[i] = cx;
-                }
+                cx = fx;
+                rows();
             }
-            double nx = __shfl(cx, f, kSpecWave);
+            const double nx = readlane_f64(cx, f);
             if (lane == f) ok = true;
             if (lane == f + 1) ok = exact || !act || same_bits(w, nx);
             bad = __ballot(!ok);
         }
     }
-    return __shfl(cx, (n - 1) / L, kSpecWave);
+    const double x0 = readlane_f64(cx, kl);
+    __syncthreads();
+    return x0;
+}
+
+/* Back substitution over the n rows of a sweep, last first, given x of the
+ * row after them; x_r goes to sX[sm.pos(r)].  Returns x of row 0 (x_in when
+ * n <= 0). */
+template <int MAXLG>
+__device__ __forceinline__ double spec_backward(double* sAp, double* sBp, double* sX, const SpecMap& sm, int n,
+                                                double x_in)
+{
+    if (n <= 0) return x_in;
+    if (sm.lg == 0) return spec_backward_lg<0>(sAp, sBp, sX, n, x_in);
+    if (sm.lg == 1) return spec_backward_lg<1>(sAp, sBp, sX, n, x_in);
+    if (MAXLG == 2 || sm.lg == 2) return spec_backward_lg<2>(sAp, sBp, sX, n, x_in);
+    return spec_backward_lg<3>(sAp, sBp, sX, n, x_in);
 }
 
 } // namespace hd_spec
