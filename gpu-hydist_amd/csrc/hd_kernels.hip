@@ -3494,13 +3494,27 @@ void hd_launch_wet_count(const HdBatch& b, hipStream_t s)
     hipLaunchKernelGGL(k_wet_count, dim3(b.N + 3, 1, b.n), dim3(64), 0, s, b.dv);
 }
 
+/* One lane per system takes about 0.75 us per row of the mean system, one
+ * wave per system about 4.2 us for every 2048 systems (eight workgroups of
+ * 18 KB of LDS on each of 256 CUs): the lane form where the first is less.
+ * Measured, lane against wave form, us: 4 rows x 64 systems 3.4 / 4.2, 8 x 64
+ * 4.8 / 4.1, 8 x 2000 5.1 / 6.1, 12 x 2000 6.9 / 6.2, 16 x 2000 11 / 6.1, 24 x
+ * 20000 24 / 48, 32 x 20000 32 / 46, 64 x 20000 61 / 53, 64 x 2000 41 / 7.5. */
+static bool batch_lane_form(int nsys, int nrows)
+{
+    return ((long long)nsys + 2048) * nsys > 384LL * nrows;
+}
+
 int hd_thomas_batch_device(int nsys, const int* off, const int* sn, const double* A, const double* B,
                            const double* C, const double* D, double* x, double* Ap, double* Bp, int nrows,
                            hipStream_t s)
 {
-    if (nsys > 0)
+    if (nsys <= 0) return 0;
+    if (batch_lane_form(nsys, nrows))
         hipLaunchKernelGGL(k_thomas_batch, dim3((nsys + 63) / 64), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap,
                            Bp, nrows);
+    else
+        hipLaunchKernelGGL(k_thomas_spec, dim3(nsys), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap, Bp, nrows);
     return 0;
 }
 
