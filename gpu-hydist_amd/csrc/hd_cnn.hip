@@ -10,26 +10,27 @@
  * r][n = l%16] for r = 0..3 (checked by hd_cnn_mfma_check against a host
  * product).
  *
- * Forward conv: a workgroup of four waves covers four image rows of 64
- * pixels; a wave owns one row: 4 M-blocks (16 pixels) x COUT/16 N-blocks of
- * accumulators.  K runs over the 9 taps x CIN channels in chunks of 32; the
- * A fragment of a pixel is 8 consecutive channels (one 16-byte load, NHWC),
- * the B fragment 8 consecutive input channels of one output channel (one
- * 16-byte load, weights [tap][cout][cin]).  The data gradient is the same
- * kernel on the gradient image with the tap-flipped, transposed weights.
- * Weight gradient: K = pixels; 32-pixel chunks of the gradient and of the
- * three input rows are staged in LDS and read transposed.
+ * Convolution (forward and data gradient): A is the weights, B the pixels, so
+ * a lane's results are neighbouring channels of one pixel and leave in 16-byte
+ * stores.  A wave keeps the weights of its 32 output channels (all taps) in
+ * registers and walks down a strip of 16 columns: the fragments of an input
+ * row are loaded once, straight from memory in the operand's layout, and
+ * serve the three output rows they touch, each summed over the taps in their
+ * order.  Weight gradient: K = pixels; image rows pass through LDS once and
+ * both operands are read from there transposed.
  */
 #include "hd_internal.h"
 #include "../../include/hydist_cnn.h"
 
 #include <cmath>
 #include <cstring>
+#include <utility>
 #include <string>
 #include <vector>
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 /* hd_api.hip: device view and stream of a context (same library) */
@@ -40,6 +41,8 @@ namespace {
 constexpr int kCinPad = 32;   /* input channels after padding */
 constexpr int kWidth = 64;    /* hidden channels */
 constexpr int kOutPad = 32;   /* output channels after padding */
+constexpr int kNarrow = 8;    /* stored channels of input images and output gradients (the rest are zero) */
+constexpr int kOut4 = 4;      /* stored channels of the network's output */
 
 enum { EPI_RELU = 0, EPI_RESRELU = 1, EPI_LINEAR = 2, EPI_BWD_SET = 3, EPI_BWD_ADD = 4 };
 
@@ -48,256 +51,402 @@ __device__ __forceinline__ f32x4 mfma(const bf16x8& a, const bf16x8& b, const f3
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-/* Y = conv3x3(X) (+ bias) with epilogue EPI; images [nimg][H][W][C]. */
-/* With a tile list (tl != nullptr) workgroup k covers tile tl[k] for k <
- * *tn and does nothing beyond; without one, workgroup k covers tile k.
- * The tile's input window (rows h0 - 1 .. h0 + 4, columns w0 - 1 .. w0 + 64,
- * zero outside the image) is staged in LDS once, pixel pitch padded by 16
- * bytes against bank conflicts, and the nine taps' A fragments are read
- * from there; each tap's weights ([cout][cin]) pass through a double-buffered
- * LDS slot, the next tap's loaded into registers while the current one is
- * multiplied. */
-template <int CIN, int COUT, int EPI>
-__global__ void __launch_bounds__(256) k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt,
-                                              const float* __restrict__ bias, int nimg, int H, int W,
-                                              const bf16* __restrict__ res, bf16* __restrict__ Y,
-                                              bf16* __restrict__ R, float* __restrict__ Yf,
-                                              const int* __restrict__ tl, const int* __restrict__ tn)
+/* base[row elements + lane's byte offset]: the row (wave-uniform, kept from
+ * being turned into a pointer per lane and per use) in scalar registers */
+template <typename T, typename E>
+__device__ __forceinline__ T ld_row(const E* base, size_t row, unsigned off)
 {
-    constexpr int NB = COUT / 16;
-    constexpr int CP = CIN + 8;      /* padded channels per pixel in LDS */
-    constexpr int WR = 6, WC = 66;   /* window rows and columns */
-    constexpr int C8 = CIN / 8;      /* 16-byte chunks per pixel */
-    constexpr int TW = COUT * CIN;   /* weights of one tap */
-    constexpr int NW = (TW / 8 + 255) / 256;
-    __shared__ bf16 sx[WR * WC * CP];
-    __shared__ bf16 sw[2][TW];
-    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int tilesW = (W + 63) >> 6, tilesH = (H + 3) >> 2;
-    int t = blockIdx.x;
-    if (tl) {
-        if ((int)blockIdx.x >= *tn) return;
-        t = tl[blockIdx.x];
+    return *(const T*)((const char*)(base + row) + off);
+}
+template <typename T, typename E>
+__device__ __forceinline__ void st_row(E* base, size_t row, unsigned off, T v)
+{
+    *(T*)((char*)(base + row) + off) = v;
+}
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+/* The work of one convolution launch, in items of a strip of rows: item k
+ * covers rows [r0, r0 + R) of 16 * (strips per workgroup) columns.  Dense: k
+ * counts columns of items first, then row blocks, then images.  With a tile
+ * list (tl != nullptr) the items are the 4 x 64 tiles tl[0 .. *tn). */
+struct ConvItems {
+    int H, W, R, rows, cols, total;
+    const int *tl, *tn;
+};
+
+/* Y = conv3x3(X) (+ bias) with epilogue EPI; images [nimg][H][W][C].
+ *
+ * Bound: the matrix cores and the traffic of the images about evenly (64
+ * channels in and out: 74 kflop and 256 to 776 bytes a pixel).  A 16 x 16
+ * block of a row costs 36 MFMAs per wave (half of the output channels) and
+ * six 1-KB loads; weights cost none (144 registers), LDS and barriers are not
+ * used, and two waves per SIMD cover each other's loads and epilogues.  With
+ * the input window and each tap's weights staged in LDS every MFMA needed an
+ * LDS read of half its own time, and a workgroup lived for one 4 x 64 tile.
+ *
+ * Workgroups stay for as many items as there are; a wave's three
+ * accumulators are the output rows above, at and below the input row at
+ * hand.  gate: a bit per channel and pixel, whether the layer's ReLU passed
+ * (written forward when given; read backward for the layer below: dZ is
+ * bf16(dA) where it did). */
+template <int EPI>
+__global__ void __launch_bounds__(256, 2)
+k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __restrict__ bias, ConvItems it,
+       const bf16* __restrict__ res, bf16* __restrict__ Y, unsigned char* __restrict__ gate, float* __restrict__ Yf,
+       int store_f)
+{
+    constexpr bool NARROW = EPI == EPI_RELU || EPI == EPI_BWD_SET; /* stored input channels: 8 of 32, else 64 */
+    constexpr int KC = NARROW ? 1 : 2;                             /* 32-channel chunks of a tap */
+    constexpr int NB = EPI == EPI_LINEAR ? 1 : 2;                  /* 16-channel blocks of a wave's output */
+    constexpr int NH = NB;                                         /* waves that share a strip */
+    constexpr int CS = NARROW ? kNarrow : kWidth, CP = 32 * KC, CO = EPI == EPI_LINEAR ? kOutPad : kWidth;
+    constexpr int SW = 4 / NH;                                     /* strips per workgroup */
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int half = wv % NH, strip = wv / NH;
+    const int n = l & 15, g = l >> 4;
+    /* lane group g's results are channels cb .. cb + 4 NB - 1 */
+    const int cb = NB == 2 ? 32 * half + 8 * g : 4 * g;
+    bf16x8 wf[9][KC][NB];
+    {
+        const int co = NB == 2 ? 32 * half + 8 * (n >> 2) + (n & 3) : n;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    wf[tap][kc][nb] = *(const bf16x8*)(Wt + ((size_t)tap * CO + co + 4 * nb) * CP + kc * 32 + 8 * g);
     }
-    const int tw = t % tilesW;
-    t /= tilesW;
-    const int th = t % tilesH;
-    const int b = t / tilesH;
-    if (b >= nimg) return;               /* uniform over the workgroup */
-    const int h0 = th * 4, w0 = tw * 64;
-    const size_t img = (size_t)b * H * W;
-    for (int k = threadIdx.x; k < WR * WC * C8; k += 256) {
-        const int r = k / (WC * C8), rem = k - r * (WC * C8);
-        const int c = rem / C8, c8 = rem - c * C8;
-        const int hh = h0 - 1 + r, ww = w0 - 1 + c;
-        bf16x8 v = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (hh >= 0 && hh < H && ww >= 0 && ww < W) v = *(const bf16x8*)(X + (img + (size_t)hh * W + ww) * CIN + c8 * 8);
-        *(bf16x8*)(sx + (r * WC + c) * CP + c8 * 8) = v;
+    float bv[4 * NB];
+    if (EPI == EPI_RELU || EPI == EPI_RESRELU || EPI == EPI_LINEAR) {
+#pragma unroll
+        for (int q = 0; q < 4 * NB; ++q) bv[q] = bias[cb + q];
     }
-    for (int k = threadIdx.x; k < TW / 8; k += 256) *(bf16x8*)(sw[0] + k * 8) = *(const bf16x8*)(Wt + k * 8);
-    __syncthreads();
-    const int h = h0 + wv;
-    const bool live = h < H;   /* every wave stays for the barriers */
-    f32x4 acc[4][NB];
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int kq = 8 * (l >> 4);
-    for (int tap = 0; tap < 9; ++tap) {
-        const int r = wv + tap / 3, dx = tap % 3 - 1;
-        const bf16* swt = sw[tap & 1];
-        bf16x8 nw[NW];
-        if (tap < 8) {
-#pragma unroll
-            for (int q = 0; q < NW; ++q) {
-                const int k = threadIdx.x + 256 * q;
-                if (k < TW / 8) nw[q] = *(const bf16x8*)(Wt + (size_t)(tap + 1) * TW + k * 8);
-            }
+    const bf16x8 zero8 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    const int H = it.H, W = it.W;
+    constexpr int PER = 64 / (16 * SW); /* items per tile of the list */
+    const int total = it.tl ? it.tn[0] * PER : it.total;
+    for (int k = blockIdx.x; k < total; k += gridDim.x) {
+        int w0, r0, r1;
+        size_t img = 0;
+        if (it.tl) {
+            const int tilesW = (W + 63) >> 6, t = it.tl[k / PER];
+            w0 = (t % tilesW) * 64 + (k % PER) * 16 * SW;
+            r0 = (t / tilesW) * 4;
+            r1 = r0 + 4;
+        } else {
+            w0 = (k % it.cols) * 16 * SW;
+            const int t = k / it.cols;
+            r0 = (t % it.rows) * it.R;
+            r1 = r0 + it.R;
+            img = (size_t)(t / it.rows) * H * W;
         }
+        w0 = __builtin_amdgcn_readfirstlane(w0 + strip * 16);
+        r0 = __builtin_amdgcn_readfirstlane(r0);
+        r1 = __builtin_amdgcn_readfirstlane(r1 < H ? r1 : H);
+        if (w0 >= W) continue; /* the wave's strip lies right of the image */
+        const int col = w0 + n;
+        /* byte offsets of the lane's operands of the three taps of a row; a
+         * column outside the image (or a channel that is not stored) reads
+         * some other one and is zeroed before use */
+        unsigned vo[3];
+        bool in[3];
 #pragma unroll
-        for (int c0 = 0; c0 < CIN; c0 += 32) {
-            bf16x8 bf[NB];
+        for (int dx = 0; dx < 3; ++dx) {
+            const int c = col + dx - 1, cc = c < 0 ? 0 : (c < W ? c : W - 1);
+            in[dx] = c >= 0 && c < W && (!NARROW || g == 0);
+            vo[dx] = 2u * ((unsigned)cc * CS + (NARROW ? 0 : 8 * g));
+        }
+        const bool inside = !NARROW && w0 > 0 && w0 + 16 < W;
+        const bool out = col < W;
+        const unsigned oe = (unsigned)(out ? col : W - 1) * kWidth + cb; /* the lane's results in a row of 64 channels */
+        auto load = [&](int i, bf16x8(&f)[3][KC]) {
+            if (i < 0 || i >= H) {
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc) f[dx][kc] = zero8;
+                return;
+            }
+            const size_t row = (img + (size_t)uniform(i * W)) * CS;
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                for (int kc = 0; kc < KC; ++kc) f[dx][kc] = ld_row<bf16x8>(X, row, vo[dx] + 64 * kc);
+        };
+        /* input row i: its products for the output rows i - 1 (below it in
+         * the order of the taps: their last three), i and i + 1, then the
+         * epilogue of row i - 1 */
+        auto step = [&](int i, f32x4(&above)[NB], f32x4(&at)[NB], f32x4(&below)[NB], bf16x8(&f)[3][KC]) {
+            const int y = i - 1;
+            const bool done = y >= r0;
+            const size_t p = img + (size_t)uniform(y * W); /* the row's first pixel */
+            bf16x8 rs = zero8;
+            f32x4 o0, o1;
+            unsigned gt = 0;
+            if (done) { /* the epilogue's operands travel behind the products */
+                if (EPI == EPI_RESRELU) rs = ld_row<bf16x8>(res, p * kWidth, 2 * oe);
+                if (EPI == EPI_BWD_ADD) {
+                    o0 = ld_row<f32x4>(Yf, p * kWidth, 4 * oe);
+                    o1 = ld_row<f32x4>(Yf, p * kWidth, 4 * oe + 16);
+                }
+                if (EPI == EPI_BWD_SET || EPI == EPI_BWD_ADD) gt = ld_row<unsigned char>(gate, p * 8, oe >> 3);
+            }
+            if (!inside) {
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc)
+                        if (!in[dx]) f[dx][kc] = zero8;
+            }
+            auto taps = [&](int t0, f32x4(&acc)[NB]) {
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma(wf[t0 + dx][kc][nb], f[dx][kc], acc[nb]);
+            };
+            if (done) taps(6, above);
+            if (i >= r0 && i < r1) taps(3, at);
+            if (i + 1 < r1) {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) below[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+                taps(0, below);
+            }
+            if (!done || !out) return;
+            if (EPI == EPI_LINEAR) {
+                if (g == 0) {
+                    f32x4 v;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = above[0][r] + bv[r];
+                    st_row(Yf, p * kOut4, 16u * col, v);
+                }
+                return;
+            }
+            bf16x8 yv;
+            if (EPI == EPI_RELU || EPI == EPI_RESRELU) {
+                unsigned bits = 0;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const float v = fmaxf(above[NB == 2 ? q >> 2 : 0][q & 3] + bv[q % (4 * NB)], 0.f);
+                    yv[q] = (bf16)(EPI == EPI_RESRELU ? (float)rs[q] + v : v);
+                    /* the rounded value is positive (the smallest bf16 is 2^-133) */
+                    bits |= v > 0x1p-134f ? 1u << q : 0u;
+                }
+                st_row(Y, p * kWidth, 2 * oe, yv);
+                if (gate) st_row(gate, p * 8, oe >> 3, (unsigned char)bits);
+            } else {
+                f32x4 d0 = above[0], d1 = above[NB - 1];
+                if (EPI == EPI_BWD_ADD) { d0 = o0 + d0; d1 = o1 + d1; }
+                if (store_f) {
+                    st_row(Yf, p * kWidth, 4 * oe, d0);
+                    st_row(Yf, p * kWidth, 4 * oe + 16, d1);
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q) yv[q] = (gt >> q) & 1 ? (bf16)(q < 4 ? d0[q & 3] : d1[q & 3]) : (bf16)0.f;
+                st_row(Y, p * kWidth, 2 * oe, yv);
+            }
+        };
+        f32x4 above[NB], at[NB], below[NB];
+        bf16x8 f[3][KC], fn[3][KC];
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) above[nb] = at[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        load(r0 - 1, f);
+#pragma unroll 1
+        for (int i = r0 - 1; i <= r1; ++i) {
+            load(i < r1 ? i + 1 : H, fn);
+            step(i, above, at, below, f);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
-                const int co = nb * 16 + (l & 15);
-                bf[nb] = *(const bf16x8*)(swt + co * CIN + c0 + kq);
+                above[nb] = at[nb];
+                at[nb] = below[nb];
             }
 #pragma unroll
-            for (int mb = 0; mb < 4; ++mb) {
-                const int c = mb * 16 + (l & 15) + dx + 1;
-                const bf16x8 af = *(const bf16x8*)(sx + (r * WC + c) * CP + c0 + kq);
+            for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mfma(af, bf[nb], acc[mb][nb]);
-            }
+                for (int kc = 0; kc < KC; ++kc) f[dx][kc] = fn[dx][kc];
         }
-        if (tap < 8) {
-            /* the other slot was last read in the previous tap, which every
-             * wave finished before the barrier that ended it */
+    }
+}
+
+/* 16 channels x 8 pixels of an LDS image row as an MFMA operand (lane l:
+ * channel l % 16, pixels 8 (l / 16) ..): two transposing reads.  p: the
+ * lane's address of the first, pixel 8 (l / 16) + (l % 16) / 4, channel
+ * 4 (l % 4); S: channels between pixels. */
+template <int S>
+__device__ __forceinline__ bf16x8 ld_tr(const bf16* p)
+{
+    typedef __attribute__((address_space(3))) s16x4* lp;
+    union {
+        s16x4 h[2];
+        bf16x8 v;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)p);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p + 4 * S));
+    return u.v;
+}
+
+/* dW[tap][co][ci] += sum over pixels p of dZ[p][co] * X[p + off(tap)][ci],
+ * db[co] += sum of dZ[p][co].  MB, NBI: 16-channel blocks of dZ and of X (1
+ * where 8 channels are stored).
+ *
+ * Bound: the matrix cores, then LDS.  A workgroup walks down 64 columns: each
+ * row of dZ and of X comes to LDS once (the X rows in a ring of four, the next
+ * row's loads behind this row's products, one barrier a row) and is read from
+ * there transposed.  A wave takes 16 input channels, all output channels and
+ * all taps: 13 operands for 36 MFMAs, 0.7 of the LDS rate.  Pixels are 160
+ * bytes apart, so that the four rows of a transposing read lie in different
+ * banks.  The bias gradient is one more product, with ones.  Sums stay in
+ * registers until the workgroup has no rows left. */
+template <int MB, int NBI>
+__global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ,
+                                                  ConvItems it, float* __restrict__ dw, float* __restrict__ db)
+{
+    constexpr int SZ = MB == 4 ? 80 : 16, SX = NBI == 4 ? 80 : 16;
+    constexpr int CZ = MB == 4 ? 64 : kNarrow, CX = NBI == 4 ? 64 : kNarrow; /* stored channels */
+    constexpr int COP = MB == 4 ? kWidth : kOutPad, CIP = NBI == 4 ? kWidth : kCinPad;
+    constexpr int QZ = 64 * CZ / 8, QX = 66 * CX / 8;                        /* 16-byte pieces of a row */
+    constexpr int NZ = (QZ + 255) / 256, NX = (QX + 255) / 256;
+    constexpr int MW = NBI == 4 ? MB : 1;                                    /* dZ blocks of a wave */
+    __shared__ __attribute__((aligned(16))) bf16 sZ[2][64 * SZ];
+    __shared__ __attribute__((aligned(16))) bf16 sX[4][66 * SX];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int H = it.H, W = it.W;
+    const bf16x8 zero8 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    const bf16x8 ones = bf16x8{1, 1, 1, 1, 1, 1, 1, 1};
+    if (MB == 1)
+        for (int q = threadIdx.x; q < 128; q += 256) *(bf16x8*)(sZ[q >> 6] + (q & 63) * SZ + 8) = zero8;
+    if (NBI == 1)
+        for (int q = threadIdx.x; q < 4 * 66; q += 256) *(bf16x8*)(sX[q / 66] + (q % 66) * SX + 8) = zero8;
+    f32x4 acc[9][MW], accb = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int q = 0; q < NW; ++q) {
-                const int k = threadIdx.x + 256 * q;
-                if (k < TW / 8) *(bf16x8*)(sw[(tap + 1) & 1] + k * 8) = nw[q];
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int m = 0; m < MW; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int mb0 = NBI == 4 ? 0 : wv, nb0 = NBI == 4 ? wv : 0; /* the wave's first blocks */
+    const int px = 8 * (l >> 4) + ((l & 15) >> 2), ch = 4 * (l & 3);
+    for (int k = blockIdx.x; k < it.total; k += gridDim.x) {
+        const int w0 = (k % it.cols) * 64, t = k / it.cols;
+        const int r0 = (t % it.rows) * it.R, r1 = r0 + it.R < H ? r0 + it.R : H;
+        const size_t img = (size_t)(t / it.rows) * H * W;
+        bf16x8 zr[NZ], xr[NX];
+        auto ld_z = [&](int h) {
+#pragma unroll
+            for (int q = 0; q < NZ; ++q) {
+                const int e = threadIdx.x + 256 * q, c = w0 + e / (CZ / 8);
+                zr[q] = zero8;
+                if (e < QZ && c < W) zr[q] = *(const bf16x8*)(dZ + (img + (size_t)h * W + c) * CZ + e % (CZ / 8) * 8);
+            }
+        };
+        auto st_z = [&](int h) {
+#pragma unroll
+            for (int q = 0; q < NZ; ++q) {
+                const int e = threadIdx.x + 256 * q;
+                if (e < QZ) *(bf16x8*)(sZ[h & 1] + e / (CZ / 8) * SZ + e % (CZ / 8) * 8) = zr[q];
+            }
+        };
+        auto ld_x = [&](int h) {
+#pragma unroll
+            for (int q = 0; q < NX; ++q) {
+                const int e = threadIdx.x + 256 * q, c = w0 - 1 + e / (CX / 8);
+                xr[q] = zero8;
+                if (e < QX && c >= 0 && c < W && h >= 0 && h < H)
+                    xr[q] = *(const bf16x8*)(X + (img + (size_t)h * W + c) * CX + e % (CX / 8) * 8);
+            }
+        };
+        auto st_x = [&](int h) {
+#pragma unroll
+            for (int q = 0; q < NX; ++q) {
+                const int e = threadIdx.x + 256 * q;
+                if (e < QX) *(bf16x8*)(sX[h & 3] + e / (CX / 8) * SX + e % (CX / 8) * 8) = xr[q];
+            }
+        };
+        __syncthreads(); /* the item before has read its last rows */
+        for (int h = r0 - 1; h <= r0 + 1; ++h) {
+            ld_x(h);
+            st_x(h);
+        }
+        ld_z(r0);
+        st_z(r0);
+        __syncthreads();
+        for (int h = r0; h < r1; ++h) {
+            const bool more = h + 1 < r1;
+            if (more) {
+                ld_x(h + 2);
+                ld_z(h + 1);
+            }
+#pragma unroll
+            for (int kc = 0; kc < 2; ++kc) {
+                bf16x8 af[MW];
+#pragma unroll
+                for (int m = 0; m < MW; ++m)
+                    af[m] = ld_tr<SZ>(sZ[h & 1] + (kc * 32 + px) * SZ + (mb0 + m) * 16 + ch);
+#pragma unroll
+                for (int tap = 0; tap < 9; ++tap) {
+                    const bf16x8 bf =
+                        ld_tr<SX>(sX[(h - 1 + tap / 3) & 3] + (kc * 32 + px + tap % 3) * SX + nb0 * 16 + ch);
+#pragma unroll
+                    for (int m = 0; m < MW; ++m) acc[tap][m] = mfma(af[m], bf, acc[tap][m]);
+                }
+                if (MW == 4) {
+#pragma unroll
+                    for (int m = 0; m < MW; ++m)
+                        if (m == wv) accb = mfma(af[m], ones, accb);
+                } else if (NBI == 1 || wv == 0) {
+                    accb = mfma(af[0], ones, accb);
+                }
+            }
+            if (more) {
+                st_x(h + 2);
+                st_z(h + 1);
             }
             __syncthreads();
         }
     }
-    if (!live) return;
-    const int w0e = w0;
+    const int ci = nb0 * 16 + (l & 15), c4 = 4 * (l >> 4);
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
+    for (int tap = 0; tap < 9; ++tap)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int w = w0e + mb * 16 + 4 * (l >> 4) + r;
-            if (w >= W) continue;
-            const size_t p = img + (size_t)h * W + w;
+        for (int m = 0; m < MW; ++m)
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                const int co = nb * 16 + (l & 15);
-                float y = acc[mb][nb][r];
-                const size_t q = p * COUT + co;
-                if (EPI == EPI_RELU) {
-                    Y[q] = (bf16)fmaxf(y + bias[co], 0.f);
-                } else if (EPI == EPI_RESRELU) {
-                    float rr = fmaxf(y + bias[co], 0.f);
-                    R[q] = (bf16)rr;
-                    Y[q] = (bf16)((float)res[q] + rr);
-                } else if (EPI == EPI_LINEAR) {
-                    Yf[q] = y + bias[co];
-                } else if (EPI == EPI_BWD_SET) {
-                    Yf[q] = y;
-                } else {
-                    Yf[q] += y;
-                }
-            }
-        }
-}
-
-/* dW[tap][co][ci] += sum over pixels p of dZ[p][co] * X[p + off(tap)][ci];
- * chunks of 32 pixels of one image row, workgroups stride over chunks. */
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(256) k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ, int nimg,
-                                               int H, int W, float* __restrict__ dw)
-{
-    constexpr int NBI = CIN / 16, MB = COUT / 16, PAIRS = 9 * NBI, PPW = (PAIRS + 3) / 4;
-    __shared__ __attribute__((aligned(16))) bf16 sZ[32][COUT];
-    __shared__ __attribute__((aligned(16))) bf16 sX[3][34][CIN];
-    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int cpr = (W + 31) >> 5;
-    const long nchunks = (long)nimg * H * cpr;
-    f32x4 acc[PPW][MB];
+            for (int r = 0; r < 4; ++r)
+                unsafeAtomicAdd(&dw[((size_t)tap * COP + (mb0 + m) * 16 + c4 + r) * CIP + ci], acc[tap][m][r]);
+    if ((l & 15) == 0 && (MB == 4 || wv == 0)) {
 #pragma unroll
-    for (int q = 0; q < PPW; ++q)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) acc[q][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int kq = 8 * (l >> 4);
-    for (long ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-        const int cw = (int)(ch % cpr);
-        const long rest = ch / cpr;
-        const int h = (int)(rest % H);
-        const int b = (int)(rest / H);
-        const int p0 = cw * 32;
-        const size_t img = (size_t)b * H * W;
-        __syncthreads();
-        for (int v = threadIdx.x; v < 32 * COUT / 8; v += 256) {
-            const int k = v / (COUT / 8), c8 = (v % (COUT / 8)) * 8;
-            bf16x8 z = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (p0 + k < W) z = *(const bf16x8*)(dZ + (img + (size_t)h * W + p0 + k) * COUT + c8);
-            *(bf16x8*)&sZ[k][c8] = z;
-        }
-        for (int v = threadIdx.x; v < 3 * 34 * CIN / 8; v += 256) {
-            const int c8 = (v % (CIN / 8)) * 8;
-            const int q = v / (CIN / 8);
-            const int k = q % 34, r = q / 34;
-            const int hh = h + r - 1, ww = p0 + k - 1;
-            bf16x8 x = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (hh >= 0 && hh < H && ww >= 0 && ww < W) x = *(const bf16x8*)(X + (img + (size_t)hh * W + ww) * CIN + c8);
-            *(bf16x8*)&sX[r][k][c8] = x;
-        }
-        __syncthreads();
-        bf16x8 af[MB];
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) af[mb][e] = sZ[kq + e][mb * 16 + (l & 15)];
-#pragma unroll
-        for (int q = 0; q < PPW; ++q) {
-            const int pair = wv + 4 * q;
-            if (pair < PAIRS) {
-                const int tap = pair / NBI, nb = pair % NBI;
-                const int r = tap / 3, dx = tap % 3 - 1;
-                bf16x8 bfr;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) bfr[e] = sX[r][kq + e + dx + 1][nb * 16 + (l & 15)];
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) acc[q][mb] = mfma(af[mb], bfr, acc[q][mb]);
-            }
-        }
+        for (int r = 0; r < 4; ++r) unsafeAtomicAdd(&db[(MB == 4 ? wv * 16 : 0) + c4 + r], accb[r]);
     }
-#pragma unroll
-    for (int q = 0; q < PPW; ++q) {
-        const int pair = wv + 4 * q;
-        if (pair >= PAIRS) continue;
-        const int tap = pair / NBI, nb = pair % NBI;
-        const int ci = nb * 16 + (l & 15);
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int co = mb * 16 + 4 * (l >> 4) + r;
-                atomicAdd(&dw[((size_t)tap * COUT + co) * CIN + ci], acc[q][mb][r]);
-            }
-    }
-}
-
-/* db[co] += sum over pixels of dZ[p][co] (C channels, 256 threads: 4 pixel
- * groups of 64 channels each, channels beyond C idle). */
-template <int C>
-__global__ void __launch_bounds__(256) k_bias_grad(const bf16* __restrict__ dZ, long npix, float* __restrict__ db)
-{
-    __shared__ float part[4][64];
-    const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-    float s = 0.f;
-    if (c < C)
-        for (long p = blockIdx.x * 4L + g; p < npix; p += gridDim.x * 4L) s += (float)dZ[p * C + c];
-    part[g][c] = s;
-    __syncthreads();
-    if (g == 0 && c < C) atomicAdd(&db[c], part[0][c] + part[1][c] + part[2][c] + part[3][c]);
-}
-
-/* dZ = bf16(dA * (gate > 0)) over npix * 64 elements */
-__global__ void __launch_bounds__(256) k_relu_grad(const float* __restrict__ dA, const bf16* __restrict__ gate,
-                                                   long n, bf16* __restrict__ dZ)
-{
-    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L)
-        dZ[i] = (float)gate[i] > 0.f ? (bf16)dA[i] : (bf16)0.f;
 }
 
 /* prediction = base + out[0..2]; masked squared error and its gradient
- * dOut (bf16, kOutPad channels) = 2 m (pred - tgt) * inv_norm. */
+ * dOut (bf16, kNarrow channels) = 2 m (pred - tgt) / (3 sum m), the sum of
+ * the mask at *nmask. */
 __global__ void __launch_bounds__(256) k_loss(const float* __restrict__ out, const float* __restrict__ base,
                                               const float* __restrict__ tgt, const float* __restrict__ msk,
-                                              long npix, float inv_norm, hd_cnn_scales sc, float* __restrict__ pred,
-                                              bf16* __restrict__ dOut, double* __restrict__ loss)
+                                              long npix, const double* __restrict__ nmask, hd_cnn_scales sc,
+                                              float* __restrict__ pred, bf16* __restrict__ dOut,
+                                              double* __restrict__ loss)
 {
     __shared__ double red[256];
     double s = 0;
     const float dsc[3] = {sc.d_u, sc.d_v, sc.d_z};
+    const float nm = (float)nmask[0];
+    const float inv_norm = nm > 0 ? 1.f / (3.f * nm) : 0.f;
     for (long p = blockIdx.x * 256L + threadIdx.x; p < npix; p += gridDim.x * 256L) {
         const float m = msk[p];
-        for (int c = 0; c < kOutPad; ++c) {
-            bf16 g = (bf16)0.f;
-            if (c < 3) {
-                const float pr = base[p * 3 + c] + dsc[c] * out[p * kOutPad + c];
-                pred[p * 3 + c] = pr;
-                if (m != 0.f) {   /* pixels outside the mask neither add loss nor gradient */
-                    const float d = (pr - tgt[p * 3 + c]) / dsc[c];   /* increment error in d units */
-                    s += (double)(m * d * d);
-                    g = (bf16)(2.f * m * d * inv_norm);
-                }
+        const f32x4 o = *(const f32x4*)(out + p * kOut4);
+        bf16x8 g = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float pr = base[p * 3 + c] + dsc[c] * o[c];
+            pred[p * 3 + c] = pr;
+            if (m != 0.f) {   /* pixels outside the mask neither add loss nor gradient */
+                const float d = (pr - tgt[p * 3 + c]) / dsc[c];   /* increment error in d units */
+                s += (double)(m * d * d);
+                g[c] = (bf16)(2.f * m * d * inv_norm);
             }
-            if (dOut) dOut[p * kOutPad + c] = g;
         }
+        if (dOut) *(bf16x8*)(dOut + p * kNarrow) = g;
     }
     red[threadIdx.x] = s;
     __syncthreads();
@@ -308,20 +457,43 @@ __global__ void __launch_bounds__(256) k_loss(const float* __restrict__ out, con
     if (threadIdx.x == 0) atomicAdd(loss, red[0] * (double)inv_norm);
 }
 
-/* Adam on n parameters; writes the BF16 copy (and, for weights, the
- * tap-flipped transposed BF16 copy used by the data gradient). */
-__global__ void __launch_bounds__(256) k_adam(float* __restrict__ w, const float* __restrict__ g,
-                                              float* __restrict__ m, float* __restrict__ v, long n, float lr,
-                                              float bc1, float bc2)
+/* One layer's parameters on the device. */
+struct LayerDev {
+    float *w, *dw, *mw, *vw, *b, *db, *mb, *vb;
+    bf16 *w16, *wT16;
+    int cin, cout;
+};
+
+__device__ __forceinline__ float adam_one(float* w, const float* g, float* m, float* v, long i, float lr, float bc1,
+                                          float bc2)
 {
+    const float gi = g[i];
+    const float mi = 0.9f * m[i] + 0.1f * gi;
+    const float vi = 0.999f * v[i] + 0.001f * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    const float x = w[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + 1e-8f);
+    w[i] = x;
+    return x;
+}
+
+/* Adam on every layer's weights and biases (grid.y: the layer), with the
+ * BF16 copies of the weights as k_wcast writes them: one launch for the
+ * network. */
+__global__ void __launch_bounds__(256) k_adam(const LayerDev* __restrict__ layers, float lr, float bc1, float bc2)
+{
+    const LayerDev& y = layers[blockIdx.y];
+    const int cin = y.cin, cout = y.cout;
+    const long n = 9L * cin * cout;
     for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
-        const float gi = g[i];
-        const float mi = 0.9f * m[i] + 0.1f * gi;
-        const float vi = 0.999f * v[i] + 0.001f * gi * gi;
-        m[i] = mi;
-        v[i] = vi;
-        w[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + 1e-8f);
+        const int ci = (int)(i % cin);
+        const long q = i / cin;
+        const int co = (int)(q % cout), tap = (int)(q / cout);
+        const bf16 x = (bf16)adam_one(y.w, y.dw, y.mw, y.vw, i, lr, bc1, bc2);
+        y.w16[i] = x;
+        y.wT16[((size_t)(8 - tap) * cin + ci) * cout + co] = x;
     }
+    if (blockIdx.x == 0 && (int)threadIdx.x < cout) adam_one(y.b, y.db, y.mb, y.vb, threadIdx.x, lr, bc1, bc2);
 }
 
 /* w16[tap][co][ci] = bf16(w32), wT16[8 - tap][ci][co] = bf16(w32) */
@@ -339,21 +511,40 @@ __global__ void __launch_bounds__(256) k_wcast(const float* __restrict__ w32, in
     }
 }
 
-/* FP32 host images -> BF16 input (channels padded) and the FP32 base u, v, z */
+/* FP32 host images -> BF16 input and the FP32 base u, v, z */
 __global__ void __launch_bounds__(256) k_load_x(const float* __restrict__ x8, long npix, bf16* __restrict__ x0,
                                                 float* __restrict__ base)
 {
     for (long p = blockIdx.x * 256L + threadIdx.x; p < npix; p += gridDim.x * 256L) {
-        for (int c = 0; c < kCinPad; ++c) x0[p * kCinPad + c] = (bf16)(c < HD_CNN_CIN ? x8[p * HD_CNN_CIN + c] : 0.f);
+        for (int c = 0; c < HD_CNN_CIN; ++c) x0[p * kNarrow + c] = (bf16)x8[p * HD_CNN_CIN + c];
         for (int c = 0; c < 3; ++c) base[p * 3 + c] = x8[p * HD_CNN_CIN + c];
     }
 }
 
-/* Sample store (8 BF16 channels per pixel) -> batch input image */
-__global__ void __launch_bounds__(256) k_expand_x(const bf16* __restrict__ xs, long npix, bf16* __restrict__ x0)
+/* One sample of the store -> image d of the batch, its mask's sum added to
+ * *nmask (whole numbers: the order does not matter) */
+__global__ void __launch_bounds__(256) k_gather(const bf16* __restrict__ sx, const float* __restrict__ sbase,
+                                                const float* __restrict__ stgt, const float* __restrict__ smsk,
+                                                long npix, bf16* __restrict__ x0, float* __restrict__ base,
+                                                float* __restrict__ tgt, float* __restrict__ msk,
+                                                double* __restrict__ nmask)
 {
-    for (long p = blockIdx.x * 256L + threadIdx.x; p < npix; p += gridDim.x * 256L)
-        for (int c = 0; c < kCinPad; ++c) x0[p * kCinPad + c] = c < HD_CNN_CIN ? xs[p * HD_CNN_CIN + c] : (bf16)0.f;
+    __shared__ double red[4];
+    double s = 0;
+    for (long p = blockIdx.x * 256L + threadIdx.x; p < npix; p += gridDim.x * 256L) {
+        *(bf16x8*)(x0 + p * kNarrow) = *(const bf16x8*)(sx + p * kNarrow);
+        for (int c = 0; c < 3; ++c) {
+            base[p * 3 + c] = sbase[p * 3 + c];
+            tgt[p * 3 + c] = stgt[p * 3 + c];
+        }
+        const float m = smsk[p];
+        msk[p] = m;
+        s += (double)m;
+    }
+    for (int k = 32; k > 0; k >>= 1) s += __shfl_down(s, k, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(nmask, red[0] + red[1] + red[2] + red[3]);
 }
 
 /* A context's state -> sample input (8 BF16 channels), FP32 base, mask */
@@ -404,9 +595,9 @@ __global__ void __launch_bounds__(256) k_unpack(const HdDev* __restrict__ dv, hd
     for (long p = blockIdx.x * 256L + threadIdx.x; p < npix; p += gridDim.x * 256L) {
         const int i = (int)(p / W), j = (int)(p % W);
         if (i < 1 || i > N || j < 1 || j > M || d.khouot[p] != 0) continue;
-        d.u[p] += (double)s.s_u * (double)s.d_u * (double)out[p * kOutPad + 0];
-        d.v[p] += (double)s.s_v * (double)s.d_v * (double)out[p * kOutPad + 1];
-        d.z[p] += (double)s.s_z * (double)s.d_z * (double)out[p * kOutPad + 2];
+        d.u[p] += (double)s.s_u * (double)s.d_u * (double)out[p * kOut4 + 0];
+        d.v[p] += (double)s.s_v * (double)s.d_v * (double)out[p * kOut4 + 1];
+        d.z[p] += (double)s.s_z * (double)s.d_z * (double)out[p * kOut4 + 2];
     }
 }
 
@@ -425,15 +616,11 @@ __global__ void __launch_bounds__(64) k_active_tiles(const HdDev* __restrict__ d
     if (th * 4 >= H) return;
     const int i0 = max(th * 4 - rad, 1), i1 = min(th * 4 + 3 + rad, N);
     const int j0 = max(tw * 64 - rad, 1), j1 = min(tw * 64 + 63 + rad, M);
-    bool any = false;
-    if (i0 <= i1 && j0 <= j1) {
-        const int wj = j1 - j0 + 1;
-        const long n = (long)(i1 - i0 + 1) * wj;
-        for (long k = threadIdx.x; k < n && !any; k += 64) {
-            const int i = i0 + (int)(k / wj), j = j0 + (int)(k % wj);
-            any = d.khouot[(long)i * W + j] == 0;
-        }
-    }
+    /* a lane per column, every load on its own */
+    int any = 0;
+    for (int j = j0 + (int)threadIdx.x; j <= j1; j += 64)
+#pragma unroll 6
+        for (int i = i0; i <= i1; ++i) any |= d.khouot[(long)i * W + j] == 0;
     if (__any(any) && threadIdx.x == 0) list[atomicAdd(count, 1)] = t;
 }
 
@@ -472,17 +659,21 @@ struct hd_cnn {
     std::vector<Layer> layer;
     hd_cnn_scales sc{1, 1, 1, 1, 1, 1, 1, 1, 1};
     std::vector<void*> allocs;
-    bf16* x0 = nullptr;                 /* [B][P][32] */
+    bf16* x0 = nullptr;                 /* [B][P][8] */
     float* base = nullptr;              /* [B][P][3] */
     float *tgt = nullptr, *msk = nullptr, *pred = nullptr;
     std::vector<bf16*> act;             /* act[1..L-1]: [B][P][64] */
-    std::vector<bf16*> rel;             /* rel[1..L-2]: ReLU outputs of the residual layers */
-    float* out = nullptr;               /* [B][P][32] */
+    std::vector<unsigned char*> gate;   /* gate[0..L-2]: which channels the layer's ReLU passed, [B][P][8] bytes */
+    float* out = nullptr;               /* [B][P][4] */
     float* dA = nullptr;                /* [B][P][64] */
-    bf16* dZ = nullptr;                 /* [B][P][64] */
+    bf16 *dZ = nullptr, *dZ2 = nullptr; /* [B][P][64]: a layer's gradient and the one below's */
+    bf16* dOut = nullptr;               /* [B][P][8] */
+    float* grads = nullptr;             /* every layer's dw and db */
+    size_t ngrads = 0;
+    LayerDev* ldev = nullptr;
     double* loss = nullptr;
     int nb = 0;                         /* images in the batch */
-    float nmask = 0;
+    double* nmask = nullptr;            /* sum of the batch's mask */
     int step = 0;
     /* sample store */
     int nsamp = 0;
@@ -542,73 +733,98 @@ static int refresh_layer(hd_cnn* n, int l)
     return HD_OK;
 }
 
-template <int CIN, int COUT, int EPI>
-static void conv(hd_cnn* n, const bf16* X, const Layer& y, bool transposed, int nimg, const bf16* res, bf16* Y,
-                 bf16* R, float* Yf)
+/* Rows per item such that the items fill the 512 resident workgroups (two on
+ * each CU) in whole rounds, weighing the rows an item reads beyond its own. */
+static ConvItems conv_items(const hd_cnn* n, int nimg, int width)
 {
-    int tiles = ((n->W + 63) / 64) * ((n->H + 3) / 4) * nimg;
-    hipLaunchKernelGGL((k_conv<CIN, COUT, EPI>), dim3(tiles), dim3(256), 0, n->stream, X, transposed ? y.wT16 : y.w16,
-                       y.b32, nimg, n->H, n->W, res, Y, R, Yf, n->tl, n->tcount);
+    ConvItems c{};
+    c.H = n->H;
+    c.W = n->W;
+    c.cols = (n->W + width - 1) / width;
+    double best = 0;
+    for (int R = 4; R <= 64; ++R) {
+        const int rows = (n->H + R - 1) / R;
+        const long items = (long)nimg * rows * c.cols;
+        const double cost = (double)((items + 511) / 512) * (R + 1.5);
+        if (c.R == 0 || cost < best) {
+            best = cost;
+            c.R = R;
+            c.rows = rows;
+            c.total = (int)items;
+        }
+    }
+    return c;
 }
 
-template <int CIN, int COUT>
+template <int EPI>
+static void conv(hd_cnn* n, const bf16* X, const Layer& y, bool transposed, int nimg, const bf16* res, bf16* Y,
+                 unsigned char* gate, float* Yf, bool store_f = true)
+{
+    ConvItems it = conv_items(n, nimg, EPI == EPI_LINEAR ? 64 : 32);
+    int grid = it.total < 512 ? it.total : 512;
+    if (n->tl) {
+        it.tl = n->tl;
+        it.tn = n->tcount;
+        grid = 512;
+    }
+    hipLaunchKernelGGL((k_conv<EPI>), dim3(grid), dim3(256), 0, n->stream, X, transposed ? y.wT16 : y.w16, y.b32, it,
+                       res, Y, gate, Yf, store_f ? 1 : 0);
+}
+
+template <int MB, int NBI>
 static void wgrad(hd_cnn* n, const bf16* X, const bf16* dZ, const Layer& y, int nimg)
 {
-    long chunks = (long)nimg * n->H * ((n->W + 31) / 32);
-    int grid = (int)(chunks < 1024 ? chunks : 1024);
-    hipLaunchKernelGGL((k_wgrad<CIN, COUT>), dim3(grid), dim3(256), 0, n->stream, X, dZ, nimg, n->H, n->W, y.dw);
-    long npix = (long)nimg * n->P;
-    hipLaunchKernelGGL((k_bias_grad<COUT>), dim3(nblk(npix / 4 + 1) < 1024 ? nblk(npix / 4 + 1) : 1024), dim3(256), 0,
-                       n->stream, dZ, npix, y.db);
+    const ConvItems it = conv_items(n, nimg, 64);
+    hipLaunchKernelGGL((k_wgrad<MB, NBI>), dim3(it.total < 512 ? it.total : 512), dim3(256), 0, n->stream, X, dZ, it,
+                       y.dw, y.db);
 }
 
-static int forward(hd_cnn* n, int nimg)
+/* gates: whether a backward pass may follow */
+static int forward(hd_cnn* n, int nimg, bool gates)
 {
     const int L = n->L;
-    conv<kCinPad, kWidth, EPI_RELU>(n, n->x0, n->layer[0], false, nimg, nullptr, n->act[1], nullptr, nullptr);
+    conv<EPI_RELU>(n, n->x0, n->layer[0], false, nimg, nullptr, n->act[1], gates ? n->gate[0] : nullptr, nullptr);
     for (int l = 1; l <= L - 2; ++l)
-        conv<kWidth, kWidth, EPI_RESRELU>(n, n->act[l], n->layer[l], false, nimg, n->act[l], n->act[l + 1], n->rel[l],
-                                          nullptr);
-    conv<kWidth, kOutPad, EPI_LINEAR>(n, n->act[L - 1], n->layer[L - 1], false, nimg, nullptr, nullptr, nullptr,
-                                      n->out);
+        conv<EPI_RESRELU>(n, n->act[l], n->layer[l], false, nimg, n->act[l], n->act[l + 1],
+                          gates ? n->gate[l] : nullptr, nullptr);
+    conv<EPI_LINEAR>(n, n->act[L - 1], n->layer[L - 1], false, nimg, nullptr, nullptr, nullptr, n->out);
     CHK(n, hipGetLastError());
     return HD_OK;
 }
 
-static int loss_and_grad(hd_cnn* n, int nimg, bool grad, double* loss)
+/* the loss of the last forward (and dOut), left at n->loss */
+static int loss_and_grad(hd_cnn* n, int nimg, bool grad)
 {
     long npix = (long)nimg * n->P;
     CHK(n, hipMemsetAsync(n->loss, 0, sizeof(double), n->stream));
-    float inv = n->nmask > 0 ? 1.f / (3.f * n->nmask) : 0.f;
     hipLaunchKernelGGL(k_loss, dim3(nblk(npix) < 2048 ? nblk(npix) : 2048), dim3(256), 0, n->stream, n->out, n->base,
-                       n->tgt, n->msk, npix, inv, n->sc, n->pred, grad ? n->dZ : nullptr, n->loss);
+                       n->tgt, n->msk, npix, n->nmask, n->sc, n->pred, grad ? n->dOut : nullptr, n->loss);
     CHK(n, hipGetLastError());
-    if (loss) {
-        CHK(n, hipMemcpyAsync(loss, n->loss, sizeof(double), hipMemcpyDeviceToHost, n->stream));
-        CHK(n, hipStreamSynchronize(n->stream));
-    }
+    return HD_OK;
+}
+
+/* waits for the stream, the loss in *loss */
+static int finish(hd_cnn* n, double* loss)
+{
+    if (loss) CHK(n, hipMemcpyAsync(loss, n->loss, sizeof(double), hipMemcpyDeviceToHost, n->stream));
+    CHK(n, hipStreamSynchronize(n->stream));
     return HD_OK;
 }
 
 static int backward(hd_cnn* n, int nimg)
 {
     const int L = n->L;
-    long npix = (long)nimg * n->P;
-    for (auto& y : n->layer) {
-        CHK(n, hipMemsetAsync(y.dw, 0, y.nw() * 4, n->stream));
-        CHK(n, hipMemsetAsync(y.db, 0, (size_t)y.cout * 4, n->stream));
-    }
-    /* output layer: dZ holds dOut (kOutPad channels) */
-    wgrad<kWidth, kOutPad>(n, n->act[L - 1], n->dZ, n->layer[L - 1], nimg);
-    conv<kOutPad, kWidth, EPI_BWD_SET>(n, n->dZ, n->layer[L - 1], true, nimg, nullptr, nullptr, nullptr, n->dA);
+    CHK(n, hipMemsetAsync(n->grads, 0, n->ngrads * 4, n->stream));
+    wgrad<1, 4>(n, n->act[L - 1], n->dOut, n->layer[L - 1], nimg);
+    conv<EPI_BWD_SET>(n, n->dOut, n->layer[L - 1], true, nimg, nullptr, n->dZ, n->gate[L - 2], n->dA);
+    bf16 *z = n->dZ, *zn = n->dZ2;
     for (int l = L - 2; l >= 1; --l) {
-        hipLaunchKernelGGL(k_relu_grad, dim3(nblk(npix * kWidth) < 4096 ? nblk(npix * kWidth) : 4096), dim3(256), 0,
-                           n->stream, n->dA, n->rel[l], npix * kWidth, n->dZ);
-        wgrad<kWidth, kWidth>(n, n->act[l], n->dZ, n->layer[l], nimg);
-        conv<kWidth, kWidth, EPI_BWD_ADD>(n, n->dZ, n->layer[l], true, nimg, nullptr, nullptr, nullptr, n->dA);
+        wgrad<4, 4>(n, n->act[l], z, n->layer[l], nimg);
+        /* dA itself is not read below layer 1 */
+        conv<EPI_BWD_ADD>(n, z, n->layer[l], true, nimg, nullptr, zn, n->gate[l - 1], n->dA, l > 1);
+        std::swap(z, zn);
     }
-    hipLaunchKernelGGL(k_relu_grad, dim3(4096), dim3(256), 0, n->stream, n->dA, n->act[1], npix * kWidth, n->dZ);
-    wgrad<kCinPad, kWidth>(n, n->x0, n->dZ, n->layer[0], nimg);
+    wgrad<4, 1>(n, n->x0, z, n->layer[0], nimg);
     CHK(n, hipGetLastError());
     return HD_OK;
 }
@@ -617,15 +833,7 @@ static int adam(hd_cnn* n, float lr)
 {
     n->step += 1;
     float bc1 = 1.f - std::pow(0.9f, (float)n->step), bc2 = 1.f - std::pow(0.999f, (float)n->step);
-    for (int l = 0; l < n->L; ++l) {
-        Layer& y = n->layer[l];
-        hipLaunchKernelGGL(k_adam, dim3(nblk((long)y.nw())), dim3(256), 0, n->stream, y.w32, y.dw, y.mw, y.vw,
-                           (long)y.nw(), lr, bc1, bc2);
-        hipLaunchKernelGGL(k_adam, dim3(1), dim3(256), 0, n->stream, y.b32, y.db, y.mb, y.vb, (long)y.cout, lr, bc1,
-                           bc2);
-        int rc = refresh_layer(n, l);
-        if (rc) return rc;
-    }
+    hipLaunchKernelGGL(k_adam, dim3(36, n->L), dim3(256), 0, n->stream, n->ldev, lr, bc1, bc2);
     CHK(n, hipGetLastError());
     return HD_OK;
 }
@@ -649,16 +857,30 @@ int hd_cnn_create(int device, int H, int W, int batch, int layers, uint64_t seed
     int rc;
     const size_t PB = (size_t)n->P * batch;
     n->layer.resize(layers);
-    uint64_t s = seed;
     for (int l = 0; l < layers; ++l) {
         Layer& y = n->layer[l];
         y.cin = l == 0 ? kCinPad : kWidth;
         y.cout = l == layers - 1 ? kOutPad : kWidth;
+        n->ngrads += y.nw() + y.cout;
+    }
+    if ((rc = calloc_dev(n, (void**)&n->grads, n->ngrads * 4)) ||
+        (rc = calloc_dev(n, (void**)&n->ldev, layers * sizeof(LayerDev)))) {
+        hd_cnn_destroy(n);
+        return rc;
+    }
+    float* grad = n->grads;
+    std::vector<LayerDev> ld(layers);
+    uint64_t s = seed;
+    for (int l = 0; l < layers; ++l) {
+        Layer& y = n->layer[l];
         size_t nw = y.nw();
-        void** f32[] = {(void**)&y.w32, (void**)&y.dw, (void**)&y.mw, (void**)&y.vw};
+        y.dw = grad;
+        y.db = grad + nw;
+        grad += nw + y.cout;
+        void** f32[] = {(void**)&y.w32, (void**)&y.mw, (void**)&y.vw};
         for (auto p : f32)
             if ((rc = calloc_dev(n, p, nw * 4))) { hd_cnn_destroy(n); return rc; }
-        void** fb[] = {(void**)&y.b32, (void**)&y.db, (void**)&y.mb, (void**)&y.vb};
+        void** fb[] = {(void**)&y.b32, (void**)&y.mb, (void**)&y.vb};
         for (auto p : fb)
             if ((rc = calloc_dev(n, p, (size_t)y.cout * 4))) { hd_cnn_destroy(n); return rc; }
         if ((rc = calloc_dev(n, (void**)&y.w16, nw * 2)) || (rc = calloc_dev(n, (void**)&y.wT16, nw * 2))) {
@@ -680,17 +902,24 @@ int hd_cnn_create(int device, int H, int W, int batch, int layers, uint64_t seed
             return cfail(nullptr, HD_EHIP, "hipMemcpy weights");
         }
         if ((rc = refresh_layer(n, l))) { hd_cnn_destroy(n); return rc; }
+        ld[l] = LayerDev{y.w32, y.dw, y.mw, y.vw, y.b32, y.db, y.mb, y.vb, y.w16, y.wT16, y.cin, y.cout};
+    }
+    if (hipMemcpy(n->ldev, ld.data(), layers * sizeof(LayerDev), hipMemcpyHostToDevice) != hipSuccess) {
+        hd_cnn_destroy(n);
+        return cfail(nullptr, HD_EHIP, "hipMemcpy layer table");
     }
     n->act.assign(layers, nullptr);
-    n->rel.assign(layers, nullptr);
+    n->gate.assign(layers, nullptr);
     for (int l = 1; l <= layers - 1; ++l)
         if ((rc = calloc_dev(n, (void**)&n->act[l], PB * kWidth * 2))) { hd_cnn_destroy(n); return rc; }
-    for (int l = 1; l <= layers - 2; ++l)
-        if ((rc = calloc_dev(n, (void**)&n->rel[l], PB * kWidth * 2))) { hd_cnn_destroy(n); return rc; }
-    if ((rc = calloc_dev(n, (void**)&n->x0, PB * kCinPad * 2)) || (rc = calloc_dev(n, (void**)&n->base, PB * 3 * 4)) ||
+    for (int l = 0; l <= layers - 2; ++l)
+        if ((rc = calloc_dev(n, (void**)&n->gate[l], PB * (kWidth / 8)))) { hd_cnn_destroy(n); return rc; }
+    if ((rc = calloc_dev(n, (void**)&n->x0, PB * kNarrow * 2)) || (rc = calloc_dev(n, (void**)&n->base, PB * 3 * 4)) ||
         (rc = calloc_dev(n, (void**)&n->tgt, PB * 3 * 4)) || (rc = calloc_dev(n, (void**)&n->msk, PB * 4)) ||
-        (rc = calloc_dev(n, (void**)&n->pred, PB * 3 * 4)) || (rc = calloc_dev(n, (void**)&n->out, PB * kOutPad * 4)) ||
+        (rc = calloc_dev(n, (void**)&n->pred, PB * 3 * 4)) || (rc = calloc_dev(n, (void**)&n->out, PB * kOut4 * 4)) ||
         (rc = calloc_dev(n, (void**)&n->dA, PB * kWidth * 4)) || (rc = calloc_dev(n, (void**)&n->dZ, PB * kWidth * 2)) ||
+        (rc = calloc_dev(n, (void**)&n->dZ2, PB * kWidth * 2)) || (rc = calloc_dev(n, (void**)&n->dOut, PB * kNarrow * 2)) ||
+        (rc = calloc_dev(n, (void**)&n->nmask, 8)) ||
         (rc = calloc_dev(n, (void**)&n->loss, 8)) ||
         (rc = calloc_dev(n, (void**)&n->tlist, (size_t)((W + 63) / 64) * ((H + 3) / 4) * 4)) ||
         (rc = calloc_dev(n, (void**)&n->tcount, 4))) {
@@ -791,7 +1020,7 @@ int hd_cnn_load_batch(hd_cnn* n, int b, const float* host_x, const float* host_y
         CHK(n, hipMemcpy(n->msk, host_m, (size_t)npix * 4, hipMemcpyHostToDevice));
         for (long p = 0; p < npix; ++p) ms += host_m[p];
     }
-    n->nmask = (float)ms;
+    CHK(n, hipMemcpy(n->nmask, &ms, sizeof(double), hipMemcpyHostToDevice));
     n->nb = b;
     return HD_OK;
 }
@@ -799,9 +1028,9 @@ int hd_cnn_load_batch(hd_cnn* n, int b, const float* host_x, const float* host_y
 int hd_cnn_forward(hd_cnn* n, float* host_out)
 {
     if (!n || n->nb < 1) return cfail(n, HD_ESTATE, "hd_cnn_forward: no batch loaded");
-    int rc = forward(n, n->nb);
+    int rc = forward(n, n->nb, true);
     if (rc) return rc;
-    if ((rc = loss_and_grad(n, n->nb, false, nullptr))) return rc;
+    if ((rc = loss_and_grad(n, n->nb, false))) return rc;
     if (host_out) {
         CHK(n, hipStreamSynchronize(n->stream));
         CHK(n, hipMemcpy(host_out, n->pred, (size_t)n->nb * n->P * 3 * 4, hipMemcpyDeviceToHost));
@@ -812,27 +1041,29 @@ int hd_cnn_forward(hd_cnn* n, float* host_out)
 int hd_cnn_backward(hd_cnn* n, double* loss)
 {
     if (!n || n->nb < 1) return cfail(n, HD_ESTATE, "hd_cnn_backward: no batch loaded");
-    int rc = loss_and_grad(n, n->nb, true, loss);
-    if (rc) return rc;
-    if ((rc = backward(n, n->nb))) return rc;
-    CHK(n, hipStreamSynchronize(n->stream));
-    return HD_OK;
+    int rc = loss_and_grad(n, n->nb, true);
+    if (!rc) rc = backward(n, n->nb);
+    if (!rc) rc = finish(n, loss);
+    return rc;
 }
 
 int hd_cnn_adam(hd_cnn* n, float lr)
 {
     if (!n) return HD_EINVAL;
     int rc = adam(n, lr);
-    if (rc) return rc;
-    CHK(n, hipStreamSynchronize(n->stream));
-    return HD_OK;
+    if (!rc) rc = finish(n, nullptr);
+    return rc;
 }
 
+/* one wait for the whole step */
 int hd_cnn_train_step(hd_cnn* n, float lr, double* loss)
 {
-    int rc = hd_cnn_forward(n, nullptr);
-    if (!rc) rc = hd_cnn_backward(n, loss);
-    if (!rc) rc = hd_cnn_adam(n, lr);
+    if (!n || n->nb < 1) return cfail(n, HD_ESTATE, "hd_cnn_forward: no batch loaded");
+    int rc = forward(n, n->nb, true);
+    if (!rc) rc = loss_and_grad(n, n->nb, true);
+    if (!rc) rc = backward(n, n->nb);
+    if (!rc) rc = adam(n, lr);
+    if (!rc) rc = finish(n, loss);
     return rc;
 }
 
@@ -873,22 +1104,16 @@ int hd_cnn_capture(hd_cnn* n, int idx, int role, hd_ctx* c, float q, float zb)
 static int gather(hd_cnn* n, const int* idx, int b)
 {
     if (!idx || b < 1 || b > n->B) return cfail(n, HD_EINVAL, "sample list");
-    double ms = 0;
-    std::vector<float> hm;
-    for (int k = 0; k < b; ++k) {
+    for (int k = 0; k < b; ++k)
         if (idx[k] < 0 || idx[k] >= n->nsamp) return cfail(n, HD_EINVAL, "sample index out of range");
-        size_t o = (size_t)idx[k] * n->P, d = (size_t)k * n->P;
-        hipLaunchKernelGGL(k_expand_x, dim3(nblk(n->P)), dim3(256), 0, n->stream, n->sx + o * HD_CNN_CIN, n->P,
-                           n->x0 + d * kCinPad);
-        CHK(n, hipMemcpyAsync(n->base + d * 3, n->sbase + o * 3, (size_t)n->P * 12, hipMemcpyDeviceToDevice, n->stream));
-        CHK(n, hipMemcpyAsync(n->tgt + d * 3, n->stgt + o * 3, (size_t)n->P * 12, hipMemcpyDeviceToDevice, n->stream));
-        CHK(n, hipMemcpyAsync(n->msk + d, n->smsk + o, (size_t)n->P * 4, hipMemcpyDeviceToDevice, n->stream));
+    CHK(n, hipMemsetAsync(n->nmask, 0, sizeof(double), n->stream));
+    for (int k = 0; k < b; ++k) {
+        const size_t o = (size_t)idx[k] * n->P, d = (size_t)k * n->P;
+        hipLaunchKernelGGL(k_gather, dim3(nblk(n->P) < 1024 ? nblk(n->P) : 1024), dim3(256), 0, n->stream,
+                           n->sx + o * kNarrow, n->sbase + o * 3, n->stgt + o * 3, n->smsk + o, n->P,
+                           n->x0 + d * kNarrow, n->base + d * 3, n->tgt + d * 3, n->msk + d, n->nmask);
     }
-    hm.resize((size_t)b * n->P);
-    CHK(n, hipMemcpyAsync(hm.data(), n->msk, hm.size() * 4, hipMemcpyDeviceToHost, n->stream));
-    CHK(n, hipStreamSynchronize(n->stream));
-    for (float m : hm) ms += m;
-    n->nmask = (float)ms;
+    CHK(n, hipGetLastError());
     n->nb = b;
     return HD_OK;
 }
@@ -905,8 +1130,9 @@ int hd_cnn_eval_samples(hd_cnn* n, const int* host_idx, int b, double* loss)
 {
     if (!n) return HD_EINVAL;
     int rc = gather(n, host_idx, b);
-    if (!rc) rc = forward(n, b);
-    if (!rc) rc = loss_and_grad(n, b, false, loss);
+    if (!rc) rc = forward(n, b, true);
+    if (!rc) rc = loss_and_grad(n, b, false);
+    if (!rc) rc = finish(n, loss);
     return rc;
 }
 
@@ -921,9 +1147,7 @@ int hd_cnn_predict_into_ctx(hd_cnn* n, hd_ctx* c, float q, float zb)
     if ((long)(hd.N + 3) * (hd.M + 3) != n->P || hd.N + 3 != n->H) return cfail(n, HD_ESHAPE, "grid mismatch");
     if (st != 0) return cfail(n, HD_ESTATE, "context between half-steps");
     CHK(n, hipStreamSynchronize(cs));
-    bf16* xs = (bf16*)n->dZ;   /* scratch for the 8-channel sample (the gradient buffer is free here) */
-    hipLaunchKernelGGL(k_pack, dim3(nblk(n->P)), dim3(256), 0, n->stream, dv, n->sc, q, zb, xs, n->base, nullptr);
-    hipLaunchKernelGGL(k_expand_x, dim3(nblk(n->P)), dim3(256), 0, n->stream, xs, n->P, n->x0);
+    hipLaunchKernelGGL(k_pack, dim3(nblk(n->P)), dim3(256), 0, n->stream, dv, n->sc, q, zb, n->x0, n->base, nullptr);
     if (n->sparse) {
         /* Only the tiles within L - 1 cells of a wet cell: the first layer
          * reads the whole input image, and a layer's value at a cell is the
@@ -935,7 +1159,7 @@ int hd_cnn_predict_into_ctx(hd_cnn* n, hd_ctx* c, float q, float zb)
         hipLaunchKernelGGL(k_active_tiles, dim3(tiles), dim3(64), 0, n->stream, dv, n->L - 1, n->tlist, n->tcount);
         n->tl = n->tlist;
     }
-    int rc = forward(n, 1);
+    int rc = forward(n, 1, false);
     n->tl = nullptr;
     if (rc) return rc;
     hipLaunchKernelGGL(k_unpack, dim3(nblk(n->P)), dim3(256), 0, n->stream, dv, n->sc, n->out);
