@@ -77,23 +77,29 @@ struct ConvItems {
 /* Y = conv3x3(X) (+ bias) with epilogue EPI; images [nimg][H][W][C].
  *
  * Bound: the matrix cores and the traffic of the images about evenly (64
- * channels in and out: 74 kflop and 256 to 776 bytes a pixel).  A 16 x 16
- * block of a row costs 36 MFMAs per wave (half of the output channels) and
- * six 1-KB loads; weights cost none (144 registers), LDS and barriers are not
- * used, and two waves per SIMD cover each other's loads and epilogues.  With
- * the input window and each tap's weights staged in LDS every MFMA needed an
- * LDS read of half its own time, and a workgroup lived for one 4 x 64 tile.
+ * channels in and out: 74 kflop and 256 to 776 bytes a pixel), if the loads
+ * are far enough ahead: a row of a strip is 0.5 us of MFMAs and a load takes
+ * up to 2 us.  So a workgroup's rows travel three ahead in registers and wait
+ * in an LDS ring of four, one barrier a row; weights cost nothing (144
+ * registers, half of the output channels a wave, two waves per SIMD).  A
+ * row's fragments serve the three output rows it touches, 36 MFMAs for six
+ * LDS reads; pixels are 144 bytes apart there, free of bank conflicts.
+ * Staging each tap's weights in LDS instead, for 4 x 64 tiles, needed an LDS
+ * read of half its time for every MFMA: 224 us per 64 -> 64 layer at 983 x
+ * 1051, against 107 now
+ * (dZ and dA of the data gradient: 242 + 158 for the ReLU pass, against 190,
+ * 4.2 TB/s).
  *
  * Workgroups stay for as many items as there are; a wave's three
  * accumulators are the output rows above, at and below the input row at
  * hand.  gate: a bit per channel and pixel, whether the layer's ReLU passed
  * (written forward when given; read backward for the layer below: dZ is
- * bf16(dA) where it did). */
+ * bf16(dA) where it did).  The layer adds its input to its output (RESRELU)
+ * from the ring. */
 template <int EPI>
 __global__ void __launch_bounds__(256, 2)
 k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __restrict__ bias, ConvItems it,
-       const bf16* __restrict__ res, bf16* __restrict__ Y, unsigned char* __restrict__ gate, float* __restrict__ Yf,
-       int store_f)
+       bf16* __restrict__ Y, unsigned char* __restrict__ gate, float* __restrict__ Yf, int store_f)
 {
     constexpr bool NARROW = EPI == EPI_RELU || EPI == EPI_BWD_SET; /* stored input channels: 8 of 32, else 64 */
     constexpr int KC = NARROW ? 1 : 2;                             /* 32-channel chunks of a tap */
@@ -101,7 +107,13 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
     constexpr int NH = NB;                                         /* waves that share a strip */
     constexpr int CS = NARROW ? kNarrow : kWidth, CP = 32 * KC, CO = EPI == EPI_LINEAR ? kOutPad : kWidth;
     constexpr int SW = 4 / NH;                                     /* strips per workgroup */
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    constexpr int PX = 16 * SW + 2;                                /* columns of a row in LDS */
+    constexpr int PS = NARROW ? 8 : 72;                            /* channels between them there */
+    /* a row in 16-byte pieces: NL per thread, and for 64 channels the last
+     * two columns as a word each of 64 threads */
+    constexpr int NL = NARROW ? 1 : SW / 2;
+    __shared__ __attribute__((aligned(16))) bf16 ring[4][PX * PS];
+    const int wv = uniform(threadIdx.x >> 6), l = threadIdx.x & 63;
     const int half = wv % NH, strip = wv / NH;
     const int n = l & 15, g = l >> 4;
     /* lane group g's results are channels cb .. cb + 4 NB - 1 */
@@ -126,6 +138,8 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
     const int H = it.H, W = it.W;
     constexpr int PER = 64 / (16 * SW); /* items per tile of the list */
     const int total = it.tl ? it.tn[0] * PER : it.total;
+    /* the lane's fragments of a row: column 16 strip + n + dx, channels 8 g .. */
+    const int fo = (16 * strip + n) * PS + (NARROW ? 0 : 8 * g);
     for (int k = blockIdx.x; k < total; k += gridDim.x) {
         int w0, r0, r1;
         size_t img = 0;
@@ -141,64 +155,78 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
             r1 = r0 + it.R;
             img = (size_t)(t / it.rows) * H * W;
         }
-        w0 = __builtin_amdgcn_readfirstlane(w0 + strip * 16);
-        r0 = __builtin_amdgcn_readfirstlane(r0);
-        r1 = __builtin_amdgcn_readfirstlane(r1 < H ? r1 : H);
-        if (w0 >= W) continue; /* the wave's strip lies right of the image */
-        const int col = w0 + n;
-        /* byte offsets of the lane's operands of the three taps of a row; a
-         * column outside the image (or a channel that is not stored) reads
-         * some other one and is zeroed before use */
-        unsigned vo[3];
-        bool in[3];
+        w0 = uniform(w0);
+        r0 = uniform(r0);
+        r1 = uniform(r1 < H ? r1 : H);
+        /* the thread's pieces of a row: byte offsets; outside the image they
+         * read some other column and are zeroed on their way to LDS */
+        struct Piece {
+            bf16x8 q[NL];
+            unsigned last;
+        };
+        unsigned vo[NL], vl = 0;
+        bool oq[NL], ol = false;
 #pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-            const int c = col + dx - 1, cc = c < 0 ? 0 : (c < W ? c : W - 1);
-            in[dx] = c >= 0 && c < W && (!NARROW || g == 0);
-            vo[dx] = 2u * ((unsigned)cc * CS + (NARROW ? 0 : 8 * g));
+        for (int q = 0; q < NL; ++q) {
+            const int e = threadIdx.x + 256 * q, c = w0 - 1 + e / (CS / 8);
+            oq[q] = c >= 0 && c < W;
+            vo[q] = 2u * ((unsigned)(c < 0 ? 0 : (c < W ? c : W - 1)) * CS + e % (CS / 8) * 8);
         }
-        const bool inside = !NARROW && w0 > 0 && w0 + 16 < W;
-        const bool out = col < W;
-        const unsigned oe = (unsigned)(out ? col : W - 1) * kWidth + cb; /* the lane's results in a row of 64 channels */
-        auto load = [&](int i, bf16x8(&f)[3][KC]) {
-            if (i < 0 || i >= H) {
-#pragma unroll
-                for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-                    for (int kc = 0; kc < KC; ++kc) f[dx][kc] = zero8;
-                return;
-            }
+        if (!NARROW) {
+            const int c = w0 - 1 + PX - 2 + (l >> 5);
+            ol = c < W;
+            vl = 2u * (unsigned)(c < W ? c : W - 1) * CS + 4u * (l & 31);
+        }
+        auto load = [&](int i, Piece& r) {
+            if (i < 0 || i >= H) return;
             const size_t row = (img + (size_t)uniform(i * W)) * CS;
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
+            for (int q = 0; q < NL; ++q) r.q[q] = ld_row<bf16x8>(X, row, vo[q]);
+            if (!NARROW) r.last = ld_row<unsigned>(X, row, vl);
+        };
+        auto store = [&](int i, const Piece& r) {
+            const bool in = i >= 0 && i < H;
+            bf16* to = ring[i & 3];
 #pragma unroll
-                for (int kc = 0; kc < KC; ++kc) f[dx][kc] = ld_row<bf16x8>(X, row, vo[dx] + 64 * kc);
+            for (int q = 0; q < NL; ++q) {
+                const int e = threadIdx.x + 256 * q;
+                if (!NARROW || e < PX) *(bf16x8*)(to + e / (CS / 8) * PS + e % (CS / 8) * 8) = in && oq[q] ? r.q[q] : zero8;
+            }
+            if (!NARROW && wv == 0) *(unsigned*)(to + (PX - 2 + (l >> 5)) * PS + 2 * (l & 31)) = in && ol ? r.last : 0u;
+        };
+        const int col = w0 + 16 * strip + n;
+        const bool live = w0 + 16 * strip < W, out = col < W;
+        const unsigned oe = (unsigned)(out ? col : W - 1) * kWidth + cb; /* the lane's results in a row of 64 channels */
+        /* old dA and the gate of an output row, loaded a row ahead */
+        struct Old {
+            f32x4 a, b;
+            unsigned gate;
+        };
+        auto load_old = [&](int y, Old& o) {
+            if (EPI != EPI_BWD_SET && EPI != EPI_BWD_ADD) return;
+            if (y < r0 || y >= r1) return;
+            const size_t p = img + (size_t)uniform(y * W);
+            if (EPI == EPI_BWD_ADD) {
+                o.a = ld_row<f32x4>(Yf, p * kWidth, 4 * oe);
+                o.b = ld_row<f32x4>(Yf, p * kWidth, 4 * oe + 16);
+            }
+            o.gate = ld_row<unsigned char>(gate, p * 8, oe >> 3);
         };
         /* input row i: its products for the output rows i - 1 (below it in
          * the order of the taps: their last three), i and i + 1, then the
          * epilogue of row i - 1 */
-        auto step = [&](int i, f32x4(&above)[NB], f32x4(&at)[NB], f32x4(&below)[NB], bf16x8(&f)[3][KC]) {
+        auto step = [&](int i, f32x4(&above)[NB], f32x4(&at)[NB], f32x4(&below)[NB], const Old& o) {
+            if (!live) return;
             const int y = i - 1;
             const bool done = y >= r0;
-            const size_t p = img + (size_t)uniform(y * W); /* the row's first pixel */
-            bf16x8 rs = zero8;
-            f32x4 o0, o1;
-            unsigned gt = 0;
-            if (done) { /* the epilogue's operands travel behind the products */
-                if (EPI == EPI_RESRELU) rs = ld_row<bf16x8>(res, p * kWidth, 2 * oe);
-                if (EPI == EPI_BWD_ADD) {
-                    o0 = ld_row<f32x4>(Yf, p * kWidth, 4 * oe);
-                    o1 = ld_row<f32x4>(Yf, p * kWidth, 4 * oe + 16);
+            bf16x8 f[3][KC];
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                for (int kc = 0; kc < KC; ++kc) {
+                    f[dx][kc] = *(const bf16x8*)(ring[i & 3] + fo + dx * PS + 32 * kc);
+                    if (NARROW && g != 0) f[dx][kc] = zero8;
                 }
-                if (EPI == EPI_BWD_SET || EPI == EPI_BWD_ADD) gt = ld_row<unsigned char>(gate, p * 8, oe >> 3);
-            }
-            if (!inside) {
-#pragma unroll
-                for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-                    for (int kc = 0; kc < KC; ++kc)
-                        if (!in[dx]) f[dx][kc] = zero8;
-            }
             auto taps = [&](int t0, f32x4(&acc)[NB]) {
 #pragma unroll
                 for (int dx = 0; dx < 3; ++dx)
@@ -215,6 +243,7 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
                 taps(0, below);
             }
             if (!done || !out) return;
+            const size_t p = img + (size_t)uniform(y * W); /* the row's first pixel */
             if (EPI == EPI_LINEAR) {
                 if (g == 0) {
                     f32x4 v;
@@ -227,6 +256,8 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
             bf16x8 yv;
             if (EPI == EPI_RELU || EPI == EPI_RESRELU) {
                 unsigned bits = 0;
+                bf16x8 rs = zero8;
+                if (EPI == EPI_RESRELU) rs = *(const bf16x8*)(ring[y & 3] + (16 * strip + n + 1) * PS + cb);
 #pragma unroll
                 for (int q = 0; q < 8; ++q) {
                     const float v = fmaxf(above[NB == 2 ? q >> 2 : 0][q & 3] + bv[q % (4 * NB)], 0.f);
@@ -238,34 +269,45 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
                 if (gate) st_row(gate, p * 8, oe >> 3, (unsigned char)bits);
             } else {
                 f32x4 d0 = above[0], d1 = above[NB - 1];
-                if (EPI == EPI_BWD_ADD) { d0 = o0 + d0; d1 = o1 + d1; }
+                if (EPI == EPI_BWD_ADD) { d0 = o.a + d0; d1 = o.b + d1; }
                 if (store_f) {
                     st_row(Yf, p * kWidth, 4 * oe, d0);
                     st_row(Yf, p * kWidth, 4 * oe + 16, d1);
                 }
 #pragma unroll
-                for (int q = 0; q < 8; ++q) yv[q] = (gt >> q) & 1 ? (bf16)(q < 4 ? d0[q & 3] : d1[q & 3]) : (bf16)0.f;
+                for (int q = 0; q < 8; ++q)
+                    yv[q] = (o.gate >> q) & 1 ? (bf16)(q < 4 ? d0[q & 3] : d1[q & 3]) : (bf16)0.f;
                 st_row(Y, p * kWidth, 2 * oe, yv);
             }
         };
-        f32x4 above[NB], at[NB], below[NB];
-        bf16x8 f[3][KC], fn[3][KC];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) above[nb] = at[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        load(r0 - 1, f);
+        f32x4 a0[NB], a1[NB], a2[NB];
+        Piece p0, p1, p2;
+        Old o0, o1, o2;
+        int i = r0 - 1;
+        load(i, p0);
+        load(i + 1, p1);
+        load(i + 2, p2);
+        __syncthreads(); /* the item before has read its last rows */
+        store(i, p0);
+        load(i + 3, p0);
+        __syncthreads();
+        /* three steps a round: accumulators, pieces and old values change
+         * roles without moving.  Step i: row i + 1 to LDS, row i + 4 on its way */
+        auto round = [&](f32x4(&above)[NB], f32x4(&at)[NB], f32x4(&below)[NB], Piece& pc, const Old& o, Old& on) {
+            if (i < r1) store(i + 1, pc);
+            if (i + 4 <= r1) load(i + 4, pc);
+            load_old(i, on);
+            step(i, above, at, below, o);
+            __syncthreads();
+        };
 #pragma unroll 1
-        for (int i = r0 - 1; i <= r1; ++i) {
-            load(i < r1 ? i + 1 : H, fn);
-            step(i, above, at, below, f);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                above[nb] = at[nb];
-                at[nb] = below[nb];
-            }
-#pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-                for (int kc = 0; kc < KC; ++kc) f[dx][kc] = fn[dx][kc];
+        for (;;) {
+            round(a0, a1, a2, p1, o0, o1);
+            if (++i > r1) break;
+            round(a1, a2, a0, p2, o1, o2);
+            if (++i > r1) break;
+            round(a2, a0, a1, p0, o2, o0);
+            if (++i > r1) break;
         }
     }
 }
@@ -757,8 +799,8 @@ static ConvItems conv_items(const hd_cnn* n, int nimg, int width)
 }
 
 template <int EPI>
-static void conv(hd_cnn* n, const bf16* X, const Layer& y, bool transposed, int nimg, const bf16* res, bf16* Y,
-                 unsigned char* gate, float* Yf, bool store_f = true)
+static void conv(hd_cnn* n, const bf16* X, const Layer& y, bool transposed, int nimg, bf16* Y, unsigned char* gate,
+                 float* Yf, bool store_f = true)
 {
     ConvItems it = conv_items(n, nimg, EPI == EPI_LINEAR ? 64 : 32);
     int grid = it.total < 512 ? it.total : 512;
@@ -767,8 +809,8 @@ static void conv(hd_cnn* n, const bf16* X, const Layer& y, bool transposed, int 
         it.tn = n->tcount;
         grid = 512;
     }
-    hipLaunchKernelGGL((k_conv<EPI>), dim3(grid), dim3(256), 0, n->stream, X, transposed ? y.wT16 : y.w16, y.b32, it,
-                       res, Y, gate, Yf, store_f ? 1 : 0);
+    hipLaunchKernelGGL((k_conv<EPI>), dim3(grid), dim3(256), 0, n->stream, X, transposed ? y.wT16 : y.w16, y.b32, it, Y,
+                       gate, Yf, store_f ? 1 : 0);
 }
 
 template <int MB, int NBI>
@@ -783,11 +825,10 @@ static void wgrad(hd_cnn* n, const bf16* X, const bf16* dZ, const Layer& y, int 
 static int forward(hd_cnn* n, int nimg, bool gates)
 {
     const int L = n->L;
-    conv<EPI_RELU>(n, n->x0, n->layer[0], false, nimg, nullptr, n->act[1], gates ? n->gate[0] : nullptr, nullptr);
+    conv<EPI_RELU>(n, n->x0, n->layer[0], false, nimg, n->act[1], gates ? n->gate[0] : nullptr, nullptr);
     for (int l = 1; l <= L - 2; ++l)
-        conv<EPI_RESRELU>(n, n->act[l], n->layer[l], false, nimg, n->act[l], n->act[l + 1],
-                          gates ? n->gate[l] : nullptr, nullptr);
-    conv<EPI_LINEAR>(n, n->act[L - 1], n->layer[L - 1], false, nimg, nullptr, nullptr, nullptr, n->out);
+        conv<EPI_RESRELU>(n, n->act[l], n->layer[l], false, nimg, n->act[l + 1], gates ? n->gate[l] : nullptr, nullptr);
+    conv<EPI_LINEAR>(n, n->act[L - 1], n->layer[L - 1], false, nimg, nullptr, nullptr, n->out);
     CHK(n, hipGetLastError());
     return HD_OK;
 }
@@ -816,12 +857,12 @@ static int backward(hd_cnn* n, int nimg)
     const int L = n->L;
     CHK(n, hipMemsetAsync(n->grads, 0, n->ngrads * 4, n->stream));
     wgrad<1, 4>(n, n->act[L - 1], n->dOut, n->layer[L - 1], nimg);
-    conv<EPI_BWD_SET>(n, n->dOut, n->layer[L - 1], true, nimg, nullptr, n->dZ, n->gate[L - 2], n->dA);
+    conv<EPI_BWD_SET>(n, n->dOut, n->layer[L - 1], true, nimg, n->dZ, n->gate[L - 2], n->dA);
     bf16 *z = n->dZ, *zn = n->dZ2;
     for (int l = L - 2; l >= 1; --l) {
         wgrad<4, 4>(n, n->act[l], z, n->layer[l], nimg);
         /* dA itself is not read below layer 1 */
-        conv<EPI_BWD_ADD>(n, z, n->layer[l], true, nimg, nullptr, zn, n->gate[l - 1], n->dA, l > 1);
+        conv<EPI_BWD_ADD>(n, z, n->layer[l], true, nimg, zn, n->gate[l - 1], n->dA, l > 1);
         std::swap(z, zn);
     }
     wgrad<4, 1>(n, n->x0, z, n->layer[0], nimg);
