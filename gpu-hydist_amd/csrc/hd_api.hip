@@ -306,6 +306,8 @@ int hd_create(int device, const hd_params* p, int N, int M, int series_len, int 
     std::memset(&d, 0, sizeof(d));
     d.N = N; d.M = M; d.W = M + 3; d.SL = c->SL; d.total_time = total_time; d.series_len = series_len;
     d.P = c->P;
+    d.Dxr_m03 = hd_pow(d.P.Dxr, -0.3);
+    d.Qb_c = 0.053 * hd_pow((d.P.Sx - 1) * d.P.g, 0.5) * hd_pow(d.P.dm, 1.5);
     size_t F = (size_t)(N + 3) * (M + 3);
     double** f2d[] = {&d.h, &d.hsnham, &d.VISCOIDX, &d.u, &d.v, &d.z, &d.t_u, &d.t_v, &d.t_z, &d.Htdu, &d.Htdv,
                       &d.H_moi, &d.htaiz, &d.htaiz_bd, &d.Kx1, &d.Ky1, &d.Tsxw, &d.Tsyw, &d.FS, &d.tFS, &d.VTH,

@@ -29,7 +29,9 @@
  * read from dv[blockIdx.z],
  * so that loads and stores through these pointers are global instructions
  * rather than flat ones (a pointer loaded from memory is otherwise generic).
- * Layouts are identical.  Fields: the reference's Argument_Pointers arrays;
+ * Layouts are identical.  Dxr_m03 = Dxr^-0.3 and Qb_c = 0.053
+ * ((Sx - 1) g)^0.5 dm^1.5: powers of case constants that the sediment
+ * formulas hold.  Fields: the reference's Argument_Pointers arrays;
  * hmax[4]; tmp_u / tmp_v, the smoothing ping-pong partners of t_u / t_v;
  * AA..Bp line-major rows and factors; seg_end / seg_sn per-run side tables;
  * runs_u / runs_v packed wet runs (line, first, last, 0) of the UZ / VZ
@@ -46,6 +48,7 @@
 #define HD_DEV_MEMBERS(G) \
     int N, M, W, SL, total_time, series_len; \
     hd_params P; \
+    double Dxr_m03, Qb_c; \
     G double *h, *hsnham, *VISCOIDX, *u, *v, *z, *t_u, *t_v, *t_z, *Htdu, *Htdv, *H_moi, *htaiz, *htaiz_bd; \
     G double *Kx1, *Ky1, *Tsxw, *Tsyw, *FS, *tFS, *VTH, *Kx, *Ky, *Fw, *Qbx, *Qby, *dH; \
     G int* khouot; \
@@ -89,6 +92,17 @@ static_assert(sizeof(HdDev) == sizeof(HdDevG), "device view layout");
 __device__ __forceinline__ const HdDevG& dev_view(const HdDev* dv)
 {
     return reinterpret_cast<const HdDevG*>(dv)[blockIdx.z];
+}
+
+/* p[base + lane's byte offset]: a wave-uniform element base and a 32-bit
+ * per-lane offset, so that the load takes its base from scalar registers */
+__device__ __forceinline__ double ld_off(HD_GLOBAL_AS const double* p, long base, unsigned off)
+{
+    return *(HD_GLOBAL_AS const double*)((HD_GLOBAL_AS const char*)(p + base) + off);
+}
+__device__ __forceinline__ void st_off(HD_GLOBAL_AS double* p, long base, unsigned off, double v)
+{
+    *(HD_GLOBAL_AS double*)((HD_GLOBAL_AS char*)(p + base) + off) = v;
 }
 
 /* The entries of a packed run table (cnt of them) that this workgroup of a

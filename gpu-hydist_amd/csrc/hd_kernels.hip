@@ -1244,17 +1244,6 @@ __device__ __forceinline__ Pre shfl_pre(const Pre& a, int src)
     return b;
 }
 
-/* p[base + lane's byte offset]: a wave-uniform element base and a 32-bit
- * per-lane offset, so that the load takes its base from scalar registers */
-__device__ __forceinline__ double ld_off(HD_GLOBAL_AS const double* p, long base, unsigned off)
-{
-    return *(HD_GLOBAL_AS const double*)((HD_GLOBAL_AS const char*)(p + base) + off);
-}
-__device__ __forceinline__ void st_off(HD_GLOBAL_AS double* p, long base, unsigned off, double v)
-{
-    *(HD_GLOBAL_AS double*)((HD_GLOBAL_AS char*)(p + base) + off) = v;
-}
-
 /* pre_uz_ld / pre_vz_ld at element base + off / 8 */
 template <bool isU>
 __device__ __forceinline__ PreRaw pre_ld_off(const HdDevG& d, long b, unsigned o)

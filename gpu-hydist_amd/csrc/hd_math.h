@@ -21,7 +21,11 @@
  *
  * Every function uses only +, -, *, /, fma, comparisons and bit casts, so with
  * floating-point contraction disabled (-ffp-contract=off on both compilers) the
- * host and the device evaluate exactly the same operation sequence.
+ * host and the device evaluate exactly the same operation sequence.  Where the
+ * part has an instruction for an exact step (frexp, ldexp, the quotient of
+ * operands near 1) the device takes it; the values are the same.  The _core
+ * functions leave out the special arguments, which a kernel may test for a
+ * whole wave at once.
  */
 #ifndef HD_MATH_H
 #define HD_MATH_H
@@ -31,6 +35,7 @@
 
 #if defined(__HIP__)
 #include <hip/hip_runtime.h>
+#include "hd_fastdiv.h"
 #define HD_FN __host__ __device__ static inline
 #else
 #define HD_FN static inline
@@ -45,6 +50,9 @@ HD_FN double hd_exp2i(int k) { return hd_from_bits((uint64_t)(k + 1023) << 52); 
 /* x * 2^k without intermediate overflow/underflow for |k| <= 2098. */
 HD_FN double hd_ldexp(double x, int k)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_ldexp(x, k); /* as below, one rounding */
+#endif
     if (k > 1023) { x *= hd_exp2i(1023); k -= 1023; if (k > 1023) { x *= hd_exp2i(1023); k -= 1023; if (k > 1023) k = 1023; } }
     else if (k < -1022) { x *= hd_exp2i(-1022 + 53); k += 1022 - 53; if (k < -1022) { x *= hd_exp2i(-1022 + 53); k += 1022 - 53; if (k < -1022) k = -1022; } }
     return x * hd_exp2i(k);
@@ -59,7 +67,13 @@ HD_FN double hd_ldexp(double x, int k)
 /* log(1+f) for f = m - 1, m in [sqrt(2)/2, sqrt(2)); returns f - s*(f - R). */
 HD_FN double hd_log1p_reduced(double f)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
+    /* f is 0 or 2^-53 .. 0.42 in size, 2 + f within [1.7, 2.5]: no scaling */
+    const double e = 2.0 + f;
+    double s = hd_div::quot(f, e, hd_div::rcp_refined(e));
+#else
     double s = f / (2.0 + f);
+#endif
     double z = s * s;
     /* R = sum_{n>=1} 2 z^n / (2n+1), Horner form, 12 terms (z <= 0.0295). */
     double r = 2.0 / 25.0;
@@ -82,6 +96,12 @@ HD_FN double hd_log1p_reduced(double f)
 /* Split a positive finite x into 2^k * m with m in [sqrt(2)/2, sqrt(2)). */
 HD_FN double hd_reduce_log_arg(double x, int* kout)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double h = __builtin_amdgcn_frexp_mant(x); /* [1/2, 1) */
+    const int low = h <= HD_SQRT2 * 0.5;
+    *kout = __builtin_amdgcn_frexp_exp(x) - low;
+    return __builtin_ldexp(h, low);
+#endif
     int k = 0;
     uint64_t b = hd_bits(x);
     if ((b >> 52) == 0) { /* subnormal */
@@ -96,12 +116,12 @@ HD_FN double hd_reduce_log_arg(double x, int* kout)
     return m;
 }
 
-HD_FN double hd_log(double x)
+/* x is positive and normal */
+HD_FN int hd_is_normal_pos(double x) { return hd_bits(x) - 0x0010000000000000ULL < 0x7fe0000000000000ULL; }
+
+/* log(x), x positive and finite */
+HD_FN double hd_log_core(double x)
 {
-    if (x != x) return x;
-    if (x < 0.0) return __builtin_nan("");
-    if (x == 0.0) return -__builtin_inf();
-    if (x == __builtin_inf()) return x;
     int k;
     double m = hd_reduce_log_arg(x, &k);
     double lp = hd_log1p_reduced(m - 1.0);
@@ -109,15 +129,25 @@ HD_FN double hd_log(double x)
     return dk * HD_LN2_HI + (dk * HD_LN2_LO + lp);
 }
 
-/* exp(x) * (1 + xlo): exp of the double-double x + xlo, |xlo| << ulp(x). */
-HD_FN double hd_exp_dd(double x, double xlo)
+HD_FN double hd_log(double x)
 {
-    if (x != x) return x;
-    if (x > 709.782712893384) return __builtin_inf();
-    if (x < -745.2) return 0.0;
+    if (!hd_is_normal_pos(x)) {
+        if (x != x) return x;
+        if (x < 0.0) return __builtin_nan("");
+        if (x == 0.0) return -__builtin_inf();
+        if (x == __builtin_inf()) return x;
+    }
+    return hd_log_core(x);
+}
+
+/* exp(x) * (1 + xlo): exp of the double-double x + xlo, |xlo| << ulp(x),
+ * for x in [-745.2, 709.78] */
+HD_FN double hd_exp_core(double x, double xlo)
+{
     double kd = x * HD_LOG2E;
-    kd = (kd >= 0.0) ? (double)(int64_t)(kd + 0.5) : -(double)(int64_t)(0.5 - kd);
-    int k = (int)kd;
+    int k = (int)((kd < 0.0 ? -kd : kd) + 0.5); /* to nearest, ties away */
+    if (kd < 0.0) k = -k;
+    kd = (double)k;
     double r = (x - kd * HD_LN2_HI) - kd * HD_LN2_LO;
     /* exp(r) - 1 - r = r^2 (1/2 + r/6 + ...), Taylor to degree 14 (|r| <= 0.347). */
     double p = 1.0 / 87178291200.0;          /* 1/14! */
@@ -138,7 +168,41 @@ HD_FN double hd_exp_dd(double x, double xlo)
     return hd_ldexp(e, k);
 }
 
+HD_FN double hd_exp_dd(double x, double xlo)
+{
+    if (!(x >= -745.2 && x <= 709.782712893384)) {
+        if (x != x) return x;
+        return x < 0.0 ? 0.0 : __builtin_inf();
+    }
+    return hd_exp_core(x, xlo);
+}
+
 HD_FN double hd_exp(double x) { return hd_exp_dd(x, 0.0); }
+
+/* y log(x) as a double-double hi (returned) + *lo, x positive and finite */
+HD_FN double hd_ylog_core(double x, double y, double* lo)
+{
+    int k;
+    double m = hd_reduce_log_arg(x, &k);
+    double lp = hd_log1p_reduced(m - 1.0);
+    double dk = (double)k;
+    /* log x as hi + lo */
+    double a = dk * HD_LN2_HI;               /* exact */
+    double lhi = a + lp;
+    double llo = ((a - lhi) + lp) + dk * HD_LN2_LO;
+    /* y * log x as phi + plo (two-product with fma) */
+    double phi = y * lhi;
+    *lo = fma(y, lhi, -phi) + y * llo;
+    return phi;
+}
+
+/* pow(x, y) for x positive and finite, y finite and |y log x| < 700 (x = 1
+ * gives 1) */
+HD_FN double hd_pow_core(double x, double y)
+{
+    double lo, hi = hd_ylog_core(x, y, &lo);
+    return hd_exp_core(hi, lo);
+}
 
 /* pow(x, y) for the domains the ADI/sediment formulas use (x >= 0, or x < 0
  * with integral y).  Special values follow C99 Annex F. */
@@ -150,37 +214,29 @@ HD_FN double hd_pow(double x, double y)
     if (y == 1.0) return x;
     if (y == 2.0) return x * x;
     double ay = y < 0.0 ? -y : y;
-    int yint = 0, yodd = 0;
-    if (ay < 0x1p53) {
-        double yi = (double)(int64_t)ay;
-        if (yi == ay) { yint = 1; yodd = ((int64_t)ay) & 1; }
-    } else {
-        yint = 1;
-    }
     double sign = 1.0;
-    if (x < 0.0) {
-        if (!yint) return __builtin_nan("");
-        if (yodd) sign = -1.0;
-        x = -x;
+    if (!hd_is_normal_pos(x) || ay == __builtin_inf()) {
+        int yint = 0, yodd = 0;
+        if (ay < 0x1p53) {
+            double yi = (double)(int64_t)ay;
+            if (yi == ay) { yint = 1; yodd = ((int64_t)ay) & 1; }
+        } else {
+            yint = 1;
+        }
+        if (x < 0.0) {
+            if (!yint) return __builtin_nan("");
+            if (yodd) sign = -1.0;
+            x = -x;
+        }
+        if (x == 0.0) return (y > 0.0) ? sign * 0.0 : sign * __builtin_inf();
+        if (x == __builtin_inf()) return (y > 0.0) ? sign * __builtin_inf() : sign * 0.0;
+        if (ay == __builtin_inf()) {
+            if (x < 1.0) return (y > 0.0) ? 0.0 : __builtin_inf();
+            return (y > 0.0) ? __builtin_inf() : 0.0;
+        }
     }
-    if (x == 0.0) return (y > 0.0) ? sign * 0.0 : sign * __builtin_inf();
-    if (x == __builtin_inf()) return (y > 0.0) ? sign * __builtin_inf() : sign * 0.0;
-    if (ay == __builtin_inf()) {
-        if (x < 1.0) return (y > 0.0) ? 0.0 : __builtin_inf();
-        return (y > 0.0) ? __builtin_inf() : 0.0;
-    }
-    int k;
-    double m = hd_reduce_log_arg(x, &k);
-    double lp = hd_log1p_reduced(m - 1.0);
-    double dk = (double)k;
-    /* log x as hi + lo */
-    double a = dk * HD_LN2_HI;               /* exact */
-    double lhi = a + lp;
-    double llo = ((a - lhi) + lp) + dk * HD_LN2_LO;
-    /* y * log x as phi + plo (two-product with fma) */
-    double phi = y * lhi;
-    double plo = fma(y, lhi, -phi) + y * llo;
-    return sign * hd_exp_dd(phi, plo);
+    double lo, hi = hd_ylog_core(x, y, &lo);
+    return sign * hd_exp_dd(hi, lo);
 }
 
 /* pi/2 split into three 33-bit parts: k*P1, k*P2 exact for |k| < 2^20. */

@@ -45,16 +45,101 @@ __device__ double source_chs(const hd_params& P, double wsm, double Zf, double f
     return S;
 }
 
-/* source_nchs, Sediment_Transport.cu:52-60. */
-__device__ double source_nchs(const hd_params& P, double wsm, double Zf, double Uf, double h_moi, double fs)
+/* The fast forms of the rows below take each quotient from the refined
+ * reciprocal of its divisor (hd_fastdiv.h) and the powers and logarithms
+ * without their special arguments; FsGuard collects what that takes for
+ * granted, and a wave in which a lane fails it evaluates the plain forms. */
+struct FsGuard {
+    hd_div::Range g;
+    bool bad = false;
+    __device__ __forceinline__ bool ok() const { return !bad && g.lo >= -800 && g.den_ok(); }
+};
+
+/* wave-uniform values of the rows: reciprocals of the case constants */
+struct FsConst {
+    double sqrtg, Ufr2, hT, cd;              /* sqrt(g), Ufr^2, dT/2, 0.015 dm */
+    double yKs, yUfr2, yhT, ydX2, ydY2;      /* refined reciprocals */
+    bool ok;                                 /* constants positive, within 2^-50 .. 2^50 */
+};
+
+__device__ __forceinline__ FsConst fs_const(const HdDevG& d)
 {
-    double gamac = 0.434 + 5.975 * Zf + 2.888 * Zf * Zf;
-    double Tx = fmax(0.0, (Uf * Uf - P.Ufr * P.Ufr) / (P.Ufr * P.Ufr));
-    double Cac = 0.015 * P.dm * hd_pow(Tx, 1.5) * hd_pow(P.Dxr, (-0.3)) / (0.05 * h_moi);
+    const hd_params& P = d.P;
+    FsConst k;
+    k.sqrtg = sqrt(P.g);
+    k.Ufr2 = P.Ufr * P.Ufr;
+    k.hT = P.dT * 0.5;
+    k.cd = 0.015 * P.dm;
+    k.yKs = hd_div::rcp_refined(P.Ks);
+    k.yUfr2 = hd_div::rcp_refined(k.Ufr2);
+    k.yhT = hd_div::rcp_refined(k.hT);
+    k.ydX2 = hd_div::rcp_refined(P.dX2);
+    k.ydY2 = hd_div::rcp_refined(P.dY2);
+    const double c[] = {P.Ks, k.Ufr2, k.hT, P.dX2, P.dY2, P.dXbp, P.dYbp, P.wss, P.g, k.cd, d.Dxr_m03};
+    k.ok = true;
+#pragma unroll
+    for (double v : c) k.ok = k.ok && v > 0x1p-50 && v < 0x1p50;
+    return k;
+}
+
+template <bool FAST>
+__device__ __forceinline__ double fs_div(double n, double e, double y)
+{
+    return FAST ? hd_div::quot_pos(n, e, y) : n / e;
+}
+template <bool FAST>
+__device__ __forceinline__ double fs_rcp(double e)
+{
+    return FAST ? hd_div::rcp_refined(e) : 0.0;
+}
+
+/* The source term S of a cell with depth hm, concentration fs and speed vth
+ * (source_chs, or source_nchs, Sediment_Transport.cu:52-60) and its Zf (0
+ * unless fs > thr), as the rows (Sediment_Transport.cu:90-100) and the bed
+ * change (:490-500) evaluate them.  The fast form's quotients are in range
+ * for constants within 2^-50 .. 2^50, divisors within 2^-100 .. 2^100 and
+ * the numerators that the guard takes; the clamp of Tx at 0 would hide a
+ * NaN, so its numerator is tested by itself. */
+template <bool FAST>
+__device__ __forceinline__ double fs_source(const HdDevG& d, const FsConst& K, int ketdinh, double thr, double hm,
+                                            double fs, double vth, double fw, double& Zf, FsGuard& G)
+{
+    const hd_params& P = d.P;
+    const double xl = fs_div<FAST>(12 * hm, P.Ks, K.yKs);
+    const double c = 18 * (FAST ? hd_log_core(xl) : hd_log(xl));
+    const double nu = K.sqrtg * fabs(vth);
+    const double Uf = FAST ? hd_div::quot(nu, c, hd_div::rcp_refined(c)) : nu / c;
+    const double z = 1 - fs;
+    const double wsm = P.wss * (FAST ? hd_pow_core(fabs(z), 4) : hd_pow(z, 4));
+    Zf = 0;
+    const double ez = 0.4 * (Uf + 2 * wsm);
+    if (fs > thr) Zf = fs_div<FAST>(wsm, ez, fs_rcp<FAST>(ez));
+    if (FAST) {
+        G.bad = G.bad || !(hm > 0) || z == 0;
+        G.g.den(hm); G.g.den(c); G.g.den(z); G.g.den(ez);
+        G.g.num(vth);
+    }
+    if (ketdinh) return source_chs(P, wsm, Zf, fs, fw, vth, hm);
+    const double gamac = 0.434 + 5.975 * Zf + 2.888 * Zf * Zf;
+    const double nt = Uf * Uf - K.Ufr2;
+    const double Tx = fmax(0.0, fs_div<FAST>(nt, K.Ufr2, K.yUfr2));
+    double pt = 0.0;
+    if (FAST) {
+        G.bad = G.bad || !(nt < 0x1p200);
+        G.g.den(Tx);
+        if (__any(Tx > 0)) pt = Tx > 0 ? hd_pow_core(Tx, 1.5) : 0.0;
+    } else {
+        pt = hd_pow(Tx, 1.5);
+    }
+    const double e5 = 0.05 * hm;
+    const double Cac = fs_div<FAST>(K.cd * pt * d.Dxr_m03, e5, fs_rcp<FAST>(e5));
     return wsm * (Cac - gamac * fs);
 }
 
-/* Find_VTH (Sediment_Transport.cu:541-568) and hesoK (:508-539). */
+/* Find_VTH (Sediment_Transport.cu:541-568) and hesoK (:508-539).  Bound by
+ * the chain of its loads (view, tile, fields): all fields are loaded at
+ * once, 5.7 us on a 980 x 1048 river grid against 7.1 with the loads behind
+ * the tests. */
 __global__ void __launch_bounds__(256) k_vth_hesok(const HdDev* __restrict__ dv, int tiled)
 {
     const HdDevG& d = dev_view(dv);
@@ -67,27 +152,31 @@ __global__ void __launch_bounds__(256) k_vth_hesok(const HdDev* __restrict__ dv,
     }
     int N = d.N, M = d.M, W = d.W;
     const hd_params& P = d.P;
-    if (j > M || i > N) return;
-    int pos = i * W + j;
+    if (i < 1 || j < 1 || j > M || i > N) return;
+    const int pos = i * W + j;
+    /* one round of loads */
+    const double u0 = d.t_u[pos], um = d.t_u[pos - W], v0 = d.t_v[pos], vm = d.t_v[pos - 1];
+    const double hu = d.Htdu[pos], hv = d.Htdv[pos], hm = d.H_moi[pos], hz = d.htaiz[pos];
+    const double h0 = d.h[pos], hx = d.h[pos - 1], hy = d.h[pos - W];
     if (i >= 2 && j >= 2) {
-        if ((d.htaiz[pos] > P.NANGDAY) && (d.H_moi[pos] > P.H_TINH)) {
-            double ut = (d.t_u[pos] + d.t_u[pos - W]) * 0.5;
-            double vt = (d.t_v[pos] + d.t_v[pos - 1]) * 0.5;
-            d.VTH[pos] = sqrt(ut * ut + vt * vt);
-        } else d.VTH[pos] = 0;
+        double vth = 0;
+        if ((hz > P.NANGDAY) && (hm > P.H_TINH)) {
+            double ut = (u0 + um) * 0.5;
+            double vt = (v0 + vm) * 0.5;
+            vth = sqrt(ut * ut + vt * vt);
+        }
+        d.VTH[pos] = vth;
     }
-    if (i >= 1 && j >= 1) {
-        double Cz;
-        if (d.Htdu[pos] > 0) {
-            Cz = 18 * hd_log(12 * d.Htdu[pos] / P.Ks);
-            double kx = 5.93 * sqrt(P.g) * (d.h[pos - 1] + d.h[pos]) * 0.25 * fabs(d.t_u[pos]) / Cz;
-            d.Kx[pos] = fmin(100.0, fmax(5.0, kx));
-        }
-        if (d.Htdv[pos] > 0) {
-            Cz = 18 * hd_log(12 * d.Htdv[pos] / P.Ks);
-            double ky = 5.93 * sqrt(P.g) * (d.h[pos - W] + d.h[pos]) * 0.25 * fabs(d.t_v[pos]) / Cz;
-            d.Ky[pos] = fmin(100.0, fmax(5.0, ky));
-        }
+    const double sg = 5.93 * sqrt(P.g);
+    if (hu > 0) {
+        double Cz = 18 * hd_log(12 * hu / P.Ks);
+        double kx = sg * (hx + h0) * 0.25 * fabs(u0) / Cz;
+        d.Kx[pos] = fmin(100.0, fmax(5.0, kx));
+    }
+    if (hv > 0) {
+        double Cz = 18 * hd_log(12 * hv / P.Ks);
+        double ky = sg * (hy + h0) * 0.25 * fabs(v0) / Cz;
+        d.Ky[pos] = fmin(100.0, fmax(5.0, ky));
     }
 }
 
@@ -109,74 +198,181 @@ struct FsRow {
     double A, B, C, D;
 };
 
-/* One concentration row at cell (i, j) of run [first, last]:
- * _FSj_calculate__mactrix_coeff (Sediment_Transport.cu:205-302, column lines,
- * gamav before Zf and && at the last row, as written) or
- * _FSi_calculate__mactrix_coeff (:62-165, row lines). */
+/* What a row reads: along the line the velocity, the face depth and K at the
+ * cell and the one before (u, hu, k; suffix m), across it the same (v, hv,
+ * kv) and the depth and concentration at the neighbours. */
+struct FsRaw {
+    double u0, um, hu0, hum, k0, km;
+    double v0, vm, hv0, hvm, kv0, kvm;
+    double h0, hp1, hp2, hm1, hm2;
+    double f0, fp, fm;
+    double vth, fw;
+};
+
+/* The run's ends: the first / last row takes its end cell's coefficient into
+ * B (wall, or no flow there), else its concentration into D. */
+struct FsEnds {
+    bool w1, w2, c2; /* c2: the end copy's test at the last cell */
+    double f1, f2;
+};
+
+template <bool isJ>
+__device__ __forceinline__ FsEnds fs_ends(const HdDevG& d, int line, int first, int last, bool br1, bool br2)
+{
+    const int W = d.W;
+    const double* tq = isJ ? d.t_u : d.t_v;
+    const int p1 = isJ ? first * W + line : line * W + first, p2 = isJ ? last * W + line : line * W + last;
+    FsEnds e;
+    const double q1 = tq[p1], q2 = tq[p2];
+    e.f1 = d.FS[p1];
+    e.f2 = d.FS[p2];
+    e.w1 = br1 || q1 == 0;
+    e.c2 = br2 || q2 == 0;
+    e.w2 = isJ ? (br2 && q2 == 0) : e.c2; /* as written */
+    return e;
+}
+
+template <bool isJ>
+__device__ __forceinline__ FsRaw fs_load(const HdDevG& d, int i, int j)
+{
+    const int W = d.W, pos = i * W + j, s = isJ ? W : 1, t = isJ ? 1 : W;
+    const double *u = isJ ? d.t_u : d.t_v, *v = isJ ? d.t_v : d.t_u;
+    const double *hu = isJ ? d.Htdu : d.Htdv, *hv = isJ ? d.Htdv : d.Htdu;
+    const double *ku = isJ ? d.Kx : d.Ky, *kv = isJ ? d.Ky : d.Kx;
+    const double *H = d.H_moi, *F = d.FS;
+    FsRaw r;
+    r.u0 = u[pos]; r.um = u[pos - s]; r.hu0 = hu[pos]; r.hum = hu[pos - s]; r.k0 = ku[pos]; r.km = ku[pos - s];
+    r.v0 = v[pos]; r.vm = v[pos - t]; r.hv0 = hv[pos]; r.hvm = hv[pos - t]; r.kv0 = kv[pos]; r.kvm = kv[pos - t];
+    r.h0 = H[pos]; r.hp1 = H[pos + t]; r.hp2 = H[pos + 2 * t]; r.hm1 = H[pos - t]; r.hm2 = H[pos - 2 * t];
+    r.f0 = F[pos]; r.fp = F[pos + t]; r.fm = F[pos - t];
+    r.vth = d.VTH[pos];
+    r.fw = d.Fw[pos];
+    return r;
+}
+
+/* two neighbouring elements in one load, aligned to 8 bytes */
+typedef double hd_pair __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ hd_pair ld2_off(HD_GLOBAL_AS const double* p, long base, unsigned off)
+{
+    return *(HD_GLOBAL_AS const hd_pair*)((HD_GLOBAL_AS const char*)(p + base) + off);
+}
+
+/* fs_load of 64 successive cells, lane l's at element base + off / 8 (off
+ * the lane's offset along the line); before: the base of the cell before
+ * lane 0's.  A column's cells lie in 64 cache lines, and a load of 64 lines
+ * keeps the address unit for 64 cycles: its values along the line come from
+ * the lane before, and neighbours across it in pairs, 12 loads in place of
+ * 22. */
+template <bool isJ>
+__device__ __forceinline__ FsRaw fs_load_off(const HdDevG& d, int ketdinh, long b, long before, unsigned o)
+{
+    const long W = d.W;
+    FsRaw r;
+    r.fw = 0;
+    if (isJ) {
+        r.u0 = ld_off(d.t_u, b, o); r.hu0 = ld_off(d.Htdu, b, o); r.k0 = ld_off(d.Kx, b, o);
+        const double xu = ld_off(d.t_u, before, 0), xh = ld_off(d.Htdu, before, 0), xk = ld_off(d.Kx, before, 0);
+        const hd_pair v = ld2_off(d.t_v, b - 1, o), hv = ld2_off(d.Htdv, b - 1, o), kv = ld2_off(d.Ky, b - 1, o);
+        const hd_pair ha = ld2_off(d.H_moi, b - 2, o), hb = ld2_off(d.H_moi, b, o);
+        const hd_pair f = ld2_off(d.FS, b - 1, o);
+        r.hp2 = ld_off(d.H_moi, b + 2, o);
+        r.fp = ld_off(d.FS, b + 1, o);
+        r.vth = ld_off(d.VTH, b, o);
+        if (ketdinh) r.fw = ld_off(d.Fw, b, o);
+        r.vm = v.x; r.v0 = v.y; r.hvm = hv.x; r.hv0 = hv.y; r.kvm = kv.x; r.kv0 = kv.y;
+        r.hm2 = ha.x; r.hm1 = ha.y; r.h0 = hb.x; r.hp1 = hb.y;
+        r.fm = f.x; r.f0 = f.y;
+        r.um = xu; r.hum = xh; r.km = xk; /* lane 0's; fs_before gives the others theirs */
+    } else {
+        const hd_pair u = ld2_off(d.t_v, b - 1, o), hu = ld2_off(d.Htdv, b - 1, o), ku = ld2_off(d.Ky, b - 1, o);
+        r.v0 = ld_off(d.t_u, b, o); r.vm = ld_off(d.t_u, b - W, o);
+        r.hv0 = ld_off(d.Htdu, b, o); r.hvm = ld_off(d.Htdu, b - W, o);
+        r.kv0 = ld_off(d.Kx, b, o); r.kvm = ld_off(d.Kx, b - W, o);
+        r.h0 = ld_off(d.H_moi, b, o);
+        r.hp1 = ld_off(d.H_moi, b + W, o); r.hp2 = ld_off(d.H_moi, b + 2 * W, o);
+        r.hm1 = ld_off(d.H_moi, b - W, o); r.hm2 = ld_off(d.H_moi, b - 2 * W, o);
+        r.f0 = ld_off(d.FS, b, o); r.fp = ld_off(d.FS, b + W, o); r.fm = ld_off(d.FS, b - W, o);
+        r.vth = ld_off(d.VTH, b, o);
+        if (ketdinh) r.fw = ld_off(d.Fw, b, o);
+        r.um = u.x; r.u0 = u.y; r.hum = hu.x; r.hu0 = hu.y; r.km = ku.x; r.k0 = ku.y;
+    }
+    return r;
+}
+
+template <bool isJ>
+__device__ __forceinline__ void fs_before(FsRaw& r)
+{
+    if (!isJ) return;
+    r.um = hd_spec::dpp_f64<0x138, 0xF>(r.um, r.u0);
+    r.hum = hd_spec::dpp_f64<0x138, 0xF>(r.hum, r.hu0);
+    r.km = hd_spec::dpp_f64<0x138, 0xF>(r.km, r.k0);
+}
+
+/* One concentration row from its loads: _FSj_calculate__mactrix_coeff
+ * (Sediment_Transport.cu:205-302, column lines, gamav before Zf, as written)
+ * or _FSi_calculate__mactrix_coeff (:62-165, row lines); is1 / is2: the
+ * run's first / last row.  Quotients that differ in sign only are taken
+ * once; every other operation is the reference's, in its order. */
+template <bool isJ, bool FAST>
+__device__ __forceinline__ FsRow fs_eval(const HdDevG& d, const FsConst& K, const FsRaw& r, const FsEnds& E, bool src,
+                                         int ketdinh, bool is1, bool is2, FsGuard& G)
+{
+    const hd_params& P = d.P;
+    const double dL2 = isJ ? P.dX2 : P.dY2, dLb = isJ ? P.dXbp : P.dYbp;
+    const double dC2 = isJ ? P.dY2 : P.dX2, dCb = isJ ? P.dYbp : P.dXbp;
+    const double yL2 = isJ ? K.ydX2 : K.ydY2, yC2 = isJ ? K.ydY2 : K.ydX2;
+    double Zf;
+    double S = fs_source<FAST>(d, K, ketdinh, 0.00001, r.h0, r.f0, r.vth, r.fw, Zf, G);
+    if (!src) S = 0;
+    const double Zg = isJ ? 0.0 : Zf;
+    const double gamav = 0.98 - 0.198 * Zg + 0.032 * Zg * Zg;
+    const double na = gamav * 0.5 * (r.u0 + r.um);
+    const double qa = fs_div<FAST>(na, dL2, yL2);
+    const double e1 = r.h0 * dLb, y1 = fs_rcp<FAST>(e1);
+    const double n0 = r.hu0 * r.k0, nm = r.hum * r.km;
+    const double A = -qa - fs_div<FAST>(nm, e1, y1);
+    const double C = qa - fs_div<FAST>(n0, e1, y1);
+    double B = P.HaiChiadT + fs_div<FAST>(n0 + nm, e1, y1);
+    double p = 0, q = 0;
+    if (r.hm1 > P.H_TINH && r.hp2 > P.H_TINH) p = r.fp - r.f0;
+    if (r.hm2 > P.H_TINH && r.hp1 > P.H_TINH) q = r.f0 - r.fm;
+    const double e2 = r.h0 * dCb;
+    p = fs_div<FAST>(1.0, e2, fs_rcp<FAST>(e2)) * (r.hv0 * r.kv0 * p - r.hvm * r.kvm * q);
+    q = 0;
+    const double nq = r.fp - r.fm;
+    if (r.hm2 > P.H_TINH && r.hp2 > P.H_TINH) q = (r.v0 + r.vm) * 0.5 * fs_div<FAST>(nq, dC2, yC2) * gamav;
+    double D = fs_div<FAST>(r.f0, K.hT, K.yhT) - q + p + fs_div<FAST>(S, r.h0, fs_rcp<FAST>(r.h0));
+    if (is1) {
+        if (E.w1) B += A;
+        else D -= A * E.f1;
+    }
+    if (is2) {
+        if (E.w2) B += C;
+        else D -= C * E.f2;
+    }
+    if (FAST) {
+        G.g.num(na); G.g.num(n0); G.g.num(nm); G.g.num(nq); G.g.num(r.f0); G.g.num(S);
+        G.bad = G.bad || !hd_div::finite(A) || !hd_div::finite(B) || !hd_div::finite(C) || !hd_div::finite(D);
+    }
+    FsRow w;
+    w.A = A; w.B = B; w.C = C; w.D = D;
+    return w;
+}
+
+/* The row of cell (i, j) of run [first, last], plain. */
 template <bool isJ>
 __device__ FsRow fs_row(const HdDevG& d, double t, double s_start, int ketdinh, int i, int j, int first, int last,
                         bool br1, bool br2)
 {
-    const hd_params& P = d.P;
-    int W = d.W;
-    const double *FS = d.FS, *Hm = d.H_moi, *t_u = d.t_u, *t_v = d.t_v, *VTH = d.VTH, *Htdu = d.Htdu, *Htdv = d.Htdv,
-                 *Fw = d.Fw, *Kx = d.Kx, *Ky = d.Ky;
-        int pos = i * W + j;
-        double c = 18 * hd_log(12 * Hm[pos] / P.Ks);
-        double Uf = sqrt(P.g) * fabs(VTH[pos]) / c;
-        double wsm = P.wss * hd_pow((1 - FS[pos]), 4);
-        double Zf = 0, S = 0, gamav;
-        if (isJ) gamav = 0.98 - 0.198 * Zf + 0.032 * Zf * Zf;
-        if (FS[pos] > 0.00001) Zf = wsm / (0.4 * (Uf + 2 * wsm));
-        if (ketdinh) S = source_chs(P, wsm, Zf, FS[pos], Fw[pos], VTH[pos], Hm[pos]);
-        else S = source_nchs(P, wsm, Zf, Uf, Hm[pos], FS[pos]);
-        if (t < s_start) S = 0;
-        if (!isJ) gamav = 0.98 - 0.198 * Zf + 0.032 * Zf * Zf;
-        double A, B, C, D, p = 0, q = 0;
-        if (isJ) {
-            A = -gamav * 0.5 * (t_u[pos] + t_u[pos - W]) / P.dX2 - Htdu[pos - W] * Kx[pos - W] / (Hm[pos] * (P.dXbp));
-            C = gamav * 0.5 * (t_u[pos] + t_u[pos - W]) / P.dX2 - Htdu[pos] * Kx[pos] / (Hm[pos] * (P.dXbp));
-            B = P.HaiChiadT + (Htdu[pos] * Kx[pos] + Htdu[pos - W] * Kx[pos - W]) / (Hm[pos] * (P.dXbp));
-            if ((Hm[pos - 1] > P.H_TINH) && (Hm[pos + 2] > P.H_TINH)) p = (FS[pos + 1] - FS[pos]);
-            if ((Hm[pos - 2] > P.H_TINH) && (Hm[pos + 1] > P.H_TINH)) q = (FS[pos] - FS[pos - 1]);
-            p = (1 / (Hm[pos] * P.dYbp)) * (Htdv[pos] * Ky[pos] * p - Htdv[pos - 1] * Ky[pos - 1] * q);
-            if ((Hm[pos - 2] > P.H_TINH) && (Hm[pos + 2] > P.H_TINH)) {
-                q = (FS[pos + 1] - FS[pos - 1]) / P.dY2;
-                q = (t_v[pos] + t_v[pos - 1]) * 0.5 * q * gamav;
-            } else q = 0;
-            D = FS[pos] / (P.dT * 0.5) - q + p + (S / Hm[pos]);
-            if (i == first + 1) {
-                if ((br1) || (t_u[first * W + j] == 0)) B += A;
-                else D -= A * FS[first * W + j];
-            }
-            if (i == last - 1) {
-                if ((br2) && (t_u[last * W + j] == 0)) B += C;
-                else D -= C * FS[last * W + j];
-            }
-        } else {
-            A = -gamav * 0.5 * (t_v[pos - 1] + t_v[pos]) / P.dY2 - Htdv[pos - 1] * Ky[pos - 1] / (Hm[pos] * P.dYbp);
-            C = gamav * 0.5 * (t_v[pos - 1] + t_v[pos]) / P.dY2 - Htdv[pos] * Ky[pos] / (Hm[pos] * P.dYbp);
-            B = P.HaiChiadT + (Htdv[pos] * Ky[pos] + Htdv[pos - 1] * Ky[pos - 1]) / (Hm[pos] * P.dYbp);
-            if ((Hm[pos + 2 * W] > P.H_TINH) && (Hm[pos - W] > P.H_TINH)) p = (FS[pos + W] - FS[pos]);
-            if (Hm[pos - 2 * W] > P.H_TINH && Hm[pos + W] > P.H_TINH) q = (FS[pos] - FS[pos - W]);
-            p = (1 / (Hm[pos] * P.dXbp)) * (Htdu[pos] * Kx[pos] * p - Htdu[pos - W] * Kx[pos - W] * q);
-            if (Hm[pos + 2 * W] > P.H_TINH && Hm[pos - 2 * W] > P.H_TINH) {
-                q = (FS[pos + W] - FS[pos - W]) / P.dX2;
-                q = (t_u[pos] + t_u[pos - W]) * 0.5 * q * gamav;
-            } else q = 0;
-            D = FS[pos] / (P.dT * 0.5) - q + p + (S / Hm[pos]);
-            if (j == first + 1) {
-                if ((br1) || (t_v[i * W + first] == 0)) B = B + A;
-                else D = D - A * FS[i * W + first];
-            }
-            if (j == last - 1) {
-                if ((br2) || (t_v[i * W + last] == 0)) B = B + C;
-                else D = D - C * FS[i * W + last];
-            }
-        }
-    FsRow w;
-    w.A = A; w.B = B; w.C = C; w.D = D;
-    return w;
+    const int k = isJ ? i : j, line = isJ ? j : i;
+    FsConst K;
+    K.sqrtg = sqrt(d.P.g);
+    K.Ufr2 = d.P.Ufr * d.P.Ufr;
+    K.hT = d.P.dT * 0.5;
+    K.cd = 0.015 * d.P.dm;
+    FsGuard G;
+    return fs_eval<isJ, false>(d, K, fs_load<isJ>(d, i, j), fs_ends<isJ>(d, line, first, last, br1, br2),
+                               !(t < s_start), ketdinh, k == first + 1, k == last - 1, G);
 }
 
 /* Concentration rows: _FSj_calculate__mactrix_coeff (Sediment_Transport.cu:205-302,
@@ -523,7 +719,14 @@ __global__ void __launch_bounds__(64) k_fs_run(const HdDev* __restrict__ dv, dou
  * the back substitution run on all 64 lanes with exact verification, so the
  * bits are those of the serial solve (tridiagSolver with jump 1,
  * UVZSolver_multithread.cu:203-262, via the FS rows of Sediment_Transport.cu:
- * 62-338). */
+ * 62-338).
+ * One wave per run leaves a SIMD with a wave or two, which issue an
+ * instruction every 5 to 7 cycles: the rows' instruction count bounds it.
+ * The rows' loads are issued together (the next round's before this one is
+ * evaluated), powers of case constants come from the device view, and the
+ * rows take the fast form unless a lane's values leave its range: 25-27 us
+ * per launch with the plain rows, 18 us with these, on a 980 x 1048 river
+ * grid of about 2000 runs. */
 template <bool isJ>
 __global__ void __launch_bounds__(64) k_fs_spec(const HdDev* __restrict__ dv, double s_start, int ketdinh)
 {
@@ -534,7 +737,6 @@ __global__ void __launch_bounds__(64) k_fs_spec(const HdDev* __restrict__ dv, do
      * last two words */
     constexpr int kW = hd_spec::spec_words(RW), kRow0 = kW - 2, kRowN = kW - 1;
     __shared__ double sA[kW], sB[kW], sC[kW], sD[kW];
-    __shared__ double sV[2]; /* clamped x of the first and last row */
     const int N = d.N, M = d.M, W = d.W;
     const int lane = threadIdx.x;
     const int tw = 2 * (N > M ? N : M) + 4;
@@ -542,17 +744,28 @@ __global__ void __launch_bounds__(64) k_fs_spec(const HdDev* __restrict__ dv, do
     const int cap = (isJ ? M + 3 : N + 3) * d.SL;
     const int cnt = d.run_cnt[isJ ? 0 : 1] < cap ? d.run_cnt[isJ ? 0 : 1] : cap;
     const int4* runs = isJ ? d.runs_u : d.runs_v;
-    const double t = d.tdev[0];
+    const bool src = !(d.tdev[0] < s_start);
+    const FsConst K = fs_const(d);
     const RunSlice sl = run_slice(cnt);
     for (int ri = sl.start; ri < sl.end; ri += sl.step) {
         const int4 rn = runs[ri];
-        const int line = rn.x, first = rn.y, last = rn.z;
+        const int line = __builtin_amdgcn_readfirstlane(rn.x), first = __builtin_amdgcn_readfirstlane(rn.y),
+                  last = __builtin_amdgcn_readfirstlane(rn.z);
         if (line < 3 || line > lmax || last < first + 2) continue;
         auto at = [&](int k) -> size_t { return isJ ? (size_t)k * W + line : (size_t)line * W + k; };
-        bool br1, br2;
-        wall_flags2(d, isJ, line, first, last, br1, br2);
         const int sn = last - first - 2;
         const int k0 = first + 1;
+        const unsigned step = isJ ? 8u * W : 8u;
+        auto base = [&](int k) -> long { return isJ ? (long)k * W + line : (long)line * W + k; };
+        /* the cells of rows ra .. (64 of them, at most up to row re) */
+        auto load = [&](int ra, int re) {
+            return fs_load_off<isJ>(d, ketdinh, base(k0 + ra), base(k0 + ra - 1),
+                                    (unsigned)(lane < re - ra ? lane : re - ra) * step);
+        };
+        FsRaw raw = load(0, sn < RW ? sn : RW - 1);
+        bool br1, br2;
+        wall_flags2(d, isJ, line, first, last, br1, br2);
+        const FsEnds E = fs_ends<isJ>(d, line, first, last, br1, br2);
         double* gAp = d.Ap + (size_t)line * tw + k0;
         double* gBp = d.Bp + (size_t)line * tw + k0;
         const int nch = sn / RW + 1;
@@ -569,12 +782,22 @@ __global__ void __launch_bounds__(64) k_fs_spec(const HdDev* __restrict__ dv, do
             chunk_rows(c, rb, n);
             const hd_spec::SpecMap sm = hd_spec::spec_map(n);
             const int ra = RW * c, re = ra + RW - 1 < sn ? ra + RW - 1 : sn; /* assembled rows */
-            for (int r = ra + lane; r <= re; r += 64) {
-                const int k = k0 + r;
-                const int i = isJ ? k : line, j = isJ ? line : k;
-                const FsRow w = fs_row<isJ>(d, t, s_start, ketdinh, i, j, first, last, br1, br2);
-                const int p = r == 0 ? kRow0 : (r == sn ? kRowN : sm.pos(r - rb));
-                sA[p] = w.A; sB[p] = w.B; sC[p] = w.C; sD[p] = w.D;
+            if (c > 0) raw = load(ra, re);
+            for (int r0 = ra; r0 <= re; r0 += 64) {
+                const int r = r0 + lane;
+                FsRaw x = raw;
+                if (r0 + 64 <= re) raw = load(r0 + 64, re);
+                fs_before<isJ>(x);
+                FsGuard G;
+                FsRow w = fs_eval<isJ, true>(d, K, x, E, src, ketdinh, r == 0, r == sn, G);
+                if (__any(!(K.ok && G.ok()))) {
+                    FsGuard G2;
+                    w = fs_eval<isJ, false>(d, K, x, E, src, ketdinh, r == 0, r == sn, G2);
+                }
+                if (r <= re) {
+                    const int p = r == 0 ? kRow0 : (r == sn ? kRowN : sm.pos(r - rb));
+                    sA[p] = w.A; sB[p] = w.B; sC[p] = w.C; sD[p] = w.D;
+                }
             }
             __syncthreads();
             if (c == 0) {
@@ -617,18 +840,16 @@ __global__ void __launch_bounds__(64) k_fs_spec(const HdDev* __restrict__ dv, do
             for (int r = r0 + lane; r <= r1; r += 64) {
                 double v = r == sn ? xs : (r == 0 ? xc : sA[sm.pos(r - rb)]);
                 if (v < 0) v = d.P.NDnen;
-                d.tFS[at(k0 + r)] = v;
-                if (r == 0) sV[0] = v;
-                if (r == sn) sV[1] = v;
+                st_off(d.tFS, base(k0 + r0), (unsigned)(r - r0) * step, v);
             }
         }
-        __syncthreads();
+        /* the end cells: the neighbour's value, or their own */
         if (lane == 0) {
-            const double* tqq = isJ ? d.t_u : d.t_v;
-            if ((br1) || (tqq[at(first)] == 0)) d.tFS[at(first)] = sV[0];
-            else d.tFS[at(first)] = d.FS[at(first)];
-            if ((br2) || (tqq[at(last)] == 0)) d.tFS[at(last)] = sV[1];
-            else d.tFS[at(last)] = d.FS[at(last)];
+            double v1 = sn == 0 ? xs : xc, v2 = xs;
+            if (v1 < 0) v1 = d.P.NDnen;
+            if (v2 < 0) v2 = d.P.NDnen;
+            d.tFS[at(first)] = E.w1 ? v1 : E.f1;
+            d.tFS[at(last)] = E.c2 ? v2 : E.f2;
         }
         __syncthreads();
     }
@@ -651,7 +872,10 @@ __global__ void __launch_bounds__(256) k_update_fs(const HdDev* __restrict__ dv,
 }
 
 /* Calculate_Qb, Sediment_Transport.cu:341-414 (qb_mode REFERENCE keeps the
- * `!VTH` test as written, FIXED uses VTH != 0; corner copies braced). */
+ * `!VTH` test as written, FIXED uses VTH != 0; corner copies braced).  Two
+ * fluxes share one power; the other two are of case constants and come from
+ * the device view: 5.0 us on a 980 x 1048 river grid, 10.7 with eight
+ * powers per cell. */
 __global__ void __launch_bounds__(256) k_calc_qb(const HdDev* __restrict__ dv, int qb_mode, int tiled)
 {
     const HdDevG& d = dev_view(dv);
@@ -670,21 +894,23 @@ __global__ void __launch_bounds__(256) k_calc_qb(const HdDev* __restrict__ dv, i
     double* Qby = d.Qby;
     int pos = i * W + j;
     double Tob, Toee = P.Toe, Tx = 0;
-    double vth = d.VTH[pos];
-    bool sel = (qb_mode == HD_QB_REFERENCE) ? (!vth) : (vth != 0);
-    if (sel && (d.khouot[pos] == 0)) {
-        Tob = P.ro * d.Fw[pos] * (vth * vth);
-        if (d.H_moi[pos] > P.ghtoe) Toee = P.Toe * (1 + P.hstoe * ((d.H_moi[pos] - P.ghtoe)));
+    /* one round of loads */
+    const double vth = d.VTH[pos], fw = d.Fw[pos], hm = d.H_moi[pos];
+    const double us = d.t_u[pos] + d.t_u[pos - W], vs = d.t_v[pos] + d.t_v[pos - 1];
+    const int kh = d.khouot[pos];
+    const bool sel = (qb_mode == HD_QB_REFERENCE) ? (!vth) : (vth != 0);
+    double qx = 0, qy = 0;
+    if (sel && (kh == 0)) {
+        Tob = P.ro * fw * (vth * vth);
+        if (hm > P.ghtoe) Toee = P.Toe * (1 + P.hstoe * ((hm - P.ghtoe)));
         if (Tob > Toee) Tx = Tob / Toee - 1;
-        Qbx[pos] = 0.053 * hd_pow((P.Sx - 1) * P.g, 0.5) * hd_pow(P.dm, 1.5) * hd_pow(Tx, 2.1) * hd_pow(P.Dxr, -0.3)
-                   * (d.t_u[pos] + d.t_u[pos - W]) * 0.5 / vth;
-        Qby[pos] = 0.053 * hd_pow((P.Sx - 1) * P.g, 0.5) * hd_pow(P.dm, 1.5) * hd_pow(Tx, 2.1) * hd_pow(P.Dxr, -0.3)
-                   * (d.t_v[pos] + d.t_v[pos - 1]) * 0.5 / vth;
-    } else {
-        Qbx[pos] = 0;
-        Qby[pos] = 0;
+        /* 0.053 ((Sx - 1) g)^0.5 dm^1.5 Tx^2.1 Dxr^-0.3, the factors of both directions */
+        const double c = d.Qb_c * hd_pow(Tx, 2.1) * d.Dxr_m03;
+        qx = c * us * 0.5 / vth;
+        qy = c * vs * 0.5 / vth;
     }
-    double qx = Qbx[pos], qy = Qby[pos];
+    Qbx[pos] = qx;
+    Qby[pos] = qy;
     if (i == 2) { Qbx[pos - W] = qx; Qby[pos - W] = qy; }
     if (i == N) { Qbx[pos + W] = qx; Qby[pos + W] = qy; }
     if (j == 2) {
@@ -701,7 +927,9 @@ __global__ void __launch_bounds__(256) k_calc_qb(const HdDev* __restrict__ dv, i
 
 /* _bed_load via BedLoad, Sediment_Transport.cu:416-506 / 630-639: rows
  * [sidx, eidx-1], cells of row runs with last - first >= 2 (t_u[pos > 0]
- * reads t_u[1], as written). */
+ * reads t_u[1], as written).  The loads do not wait for the tests that
+ * choose among them, and the source term takes the rows' fast form: 7.7 us
+ * on a 980 x 1048 river grid, 12 without. */
 __global__ void __launch_bounds__(256) k_bedload(const HdDev* __restrict__ dv, int ketdinh, int slo, int eoff, int tiled)
 {
     const HdDevG& d = dev_view(dv);
@@ -734,46 +962,46 @@ __global__ void __launch_bounds__(256) k_bedload(const HdDev* __restrict__ dv, i
     }
     if (!found || last - first < 2) return;
     const hd_params& P = d.P;
-    const double *FS = d.FS, *Hm = d.H_moi, *t_u = d.t_u, *t_v = d.t_v, *VTH = d.VTH, *Htdu = d.Htdu, *Htdv = d.Htdv,
-                 *Fw = d.Fw, *Kx = d.Kx, *Ky = d.Ky, *Qbx = d.Qbx, *Qby = d.Qby;
+    const int pos = i * W + j;
+    /* one round of loads: the cell, and its neighbours up to two away */
+    const double *FS = d.FS, *Qbx = d.Qbx, *Qby = d.Qby;
     const int* kh = d.khouot;
-    int pos = i * W + j;
-    double p = 0, q = 0;
-    if (kh[pos - W] == 1) {
-        if (t_u[pos] < 0) p = (-3 * Qbx[pos] + 4 * Qbx[pos + W] - Qbx[pos + 2 * W]) / P.dX2;
-    } else {
-        if (kh[pos + W] == 1) {
-            if (t_u[1]) p = (3 * Qbx[pos] - 4 * Qbx[pos - W] + Qbx[pos - 2 * W]) / P.dX2;
-        } else p = (Qbx[pos + W] - Qbx[pos - W]) / P.dX2;
-    }
-    if (kh[pos - 1] == 1) {
-        if (t_v[pos] < 0) q = (-3 * Qby[pos] + 4 * Qby[pos + 1] - Qby[pos + 2]) / P.dY2;
-    } else {
-        if (kh[pos + 1] == 1) {
-            if (t_v[pos] > 0) q = (3 * Qby[pos] - 4 * Qby[pos - 1] + Qby[pos - 2]) / P.dY2;
-        } else q = (Qby[pos + 1] - Qby[pos - 1]) / P.dY2;
-    }
+    const double x0 = Qbx[pos], xp1 = Qbx[pos + W], xp2 = Qbx[pos + 2 * W], xm1 = Qbx[pos - W], xm2 = Qbx[pos - 2 * W];
+    const double y0 = Qby[pos], yp1 = Qby[pos + 1], yp2 = Qby[pos + 2], ym1 = Qby[pos - 1], ym2 = Qby[pos - 2];
+    const bool kxp1 = kh[pos + W] == 1, kxp2 = kh[pos + 2 * W] == 1, kxm1 = kh[pos - W] == 1, kxm2 = kh[pos - 2 * W] == 1;
+    const bool kyp1 = kh[pos + 1] == 1, kyp2 = kh[pos + 2] == 1, kym1 = kh[pos - 1] == 1, kym2 = kh[pos - 2] == 1;
+    const double f0 = FS[pos], fxp = FS[pos + W], fxm = FS[pos - W], fyp = FS[pos + 1], fym = FS[pos - 1];
+    const double hu0 = d.Htdu[pos], hum = d.Htdu[pos - W], hv0 = d.Htdv[pos], hvm = d.Htdv[pos - 1];
+    const double kx0 = d.Kx[pos], kxm = d.Kx[pos - W], ky0 = d.Ky[pos], kym = d.Ky[pos - 1];
+    const double u0 = d.t_u[pos], u1 = d.t_u[1], v0 = d.t_v[pos];
+    const double hm = d.H_moi[pos], vth = d.VTH[pos], fw = d.Fw[pos], dH = d.dH[pos];
+    /* the bed-load gradients: one-sided at a wall and only for flow away
+     * from it, else central */
+    double p = kxm1 ? -3 * x0 + 4 * xp1 - xp2 : kxp1 ? 3 * x0 - 4 * xm1 + xm2 : xp1 - xm1;
+    const bool onx = kxm1 ? u0 < 0 : (kxp1 ? u1 != 0 : true);
+    p = onx ? p / P.dX2 : 0.0;
+    double q = kym1 ? -3 * y0 + 4 * yp1 - yp2 : kyp1 ? 3 * y0 - 4 * ym1 + ym2 : yp1 - ym1;
+    const bool ony = kym1 ? v0 < 0 : (kyp1 ? v0 > 0 : true);
+    q = ony ? q / P.dY2 : 0.0;
     double tH = p + q;
-    p = FS[pos + W] - FS[pos];
-    if ((kh[pos + 2 * W] == 1 || kh[pos - W] == 1) && (i < N)) p = 0;
-    q = FS[pos] - FS[pos - W];
-    if ((i > 2) && (kh[pos - 2 * W] == 1 || kh[pos + W] == 1)) q = 0;
-    p = 1 / P.dXbp * (Htdu[pos] * Kx[pos] * p - Htdu[pos - W] * Kx[pos - W] * q);
+    p = fxp - f0;
+    if ((kxp2 || kxm1) && (i < N)) p = 0;
+    q = f0 - fxm;
+    if ((i > 2) && (kxm2 || kxp1)) q = 0;
+    p = 1 / P.dXbp * (hu0 * kx0 * p - hum * kxm * q);
     tH = tH + p;
-    p = FS[pos + 1] - FS[pos];
-    if (((last < M) && (kh[pos - 1] == 1 || kh[pos + 2] == 1)) || (last == M && (kh[pos - 1] == 1))) p = 0;
-    q = FS[pos] - FS[pos - 1];
-    if (((first > 2) && (kh[pos - 2] == 1 || kh[pos + 1] == 1)) || (first == 2 && kh[pos + 1] == 1)) q = 0;
-    p = 1 / (P.dYbp) * (Htdv[pos] * Ky[pos] * p - Htdv[pos - 1] * Ky[pos - 1] * q);
+    p = fyp - f0;
+    if (((last < M) && (kym1 || kyp2)) || (last == M && kym1)) p = 0;
+    q = f0 - fym;
+    if (((first > 2) && (kym2 || kyp1)) || (first == 2 && kyp1)) q = 0;
+    p = 1 / (P.dYbp) * (hv0 * ky0 * p - hvm * kym * q);
     tH = tH + p;
-    double c = 18 * hd_log(12 * Hm[pos] / P.Ks);
-    double Uf = sqrt(P.g) * fabs(VTH[pos]) / c;
-    double wsm = P.wss * hd_pow((1 - FS[pos]), 4);
-    double Zf = 0, S = 0;
-    if (FS[pos] > 0.0) Zf = wsm / (0.4 * (Uf + 2 * wsm));
-    if (ketdinh) S = source_chs(P, wsm, Zf, FS[pos], Fw[pos], VTH[pos], Hm[pos]);
-    else S = source_nchs(P, wsm, Zf, Uf, Hm[pos], FS[pos]);
-    d.dH[pos] += P.dT / (1 - P.Dorong) * (S + tH);
+    const FsConst K = fs_const(d);
+    FsGuard G;
+    double Zf;
+    double S = fs_source<true>(d, K, ketdinh, 0.0, hm, f0, vth, fw, Zf, G);
+    if (__any(!(K.ok && G.ok() && hd_div::finite(S)))) S = fs_source<false>(d, K, ketdinh, 0.0, hm, f0, vth, fw, Zf, G);
+    d.dH[pos] = dH + P.dT / (1 - P.Dorong) * (S + tH);
 }
 
 } // namespace

@@ -1,0 +1,86 @@
+"""GPU: the concentration sweeps and the bed change against the CPU checker
+bit for bit where their forms change: runs around the 64 rows of a round and
+the 256 of a chunk, and cell values that leave the range of the shared
+reciprocals or reach the special arguments of the powers and logarithms."""
+import numpy as np
+import pytest
+
+import oracle
+from hydist_amd import synth
+from hydist_amd._lib import Solver
+
+pytestmark = pytest.mark.gpu
+
+VALUES = {
+    "FS": [0.0, 1e-290, 5e-324, 1.0, 1.5, -0.0, 2e-5, np.inf, np.nan],
+    "H_moi": [1e-5, 0.0005 / 12, 1e-320, 1e200, 0.0, 1e-40, np.inf, np.nan],
+    "VTH": [0.0, 1e-300, 1e-200, 1e160, 1e90, 2.0, np.nan],
+    "t_u": [0.0, -0.0, 1e-310, -1e-280, 1e300],
+    "t_v": [0.0, -0.0, 1e-310, -1e-280, 1e300],
+    "Htdu": [0.0, -0.0, 1e-305, 1e200],
+    "Htdv": [0.0, -0.0, 1e-305, 1e200],
+    "Fw": [0.0, 1e-300, 10.0],
+}
+
+
+def bits_differ(o, g, names):
+    out = []
+    for n in names:
+        a, b = o.get(n), g.get(n)
+        nan = np.isnan(a) & np.isnan(b)
+        if not np.array_equal(a.view(np.int64)[~nan], b.view(np.int64)[~nan]):
+            out.append(n)
+    return out
+
+
+def channel(N, M, edit=None, seed=0):
+    c = synth.channel_case(N=N, M=M, nsteps=100, Q=500.0 * M / 60.0)
+    o, g = oracle.Oracle(c), Solver(c)
+    o.init()
+    g.init()
+    o.run(0.0, 2, c.opts())
+    g.run(0.0, 2, c.opts())
+    rng = np.random.default_rng(seed)
+    wet = o.get("khouot") == 0
+    fs = np.where(wet, rng.uniform(0.0, 0.4, wet.shape), 0.0)
+    for x in (o, g):
+        x.set("FS", fs)
+    o.kernel("find_vth")
+    o.kernel("heso_k")
+    g.kernel("Find_VTH_hesoK")
+    assert bits_differ(o, g, ("VTH", "Kx", "Ky")) == []
+    if edit:
+        a = o.get(edit)
+        pick = wet & (rng.random(a.shape) < 0.05)
+        a[pick] = rng.choice(VALUES[edit], size=int(pick.sum()))
+        for x in (o, g):
+            x.set(edit, a)
+    return c, o, g
+
+
+def sweep(o, g, which, ketdinh, t, start):
+    o.kernel("sediment_j" if which == 0 else "sediment_i", ketdinh, 0, start, t=t)
+    g.kernel("FSj_solve" if which == 0 else "FSi_solve", t, float(start), ketdinh)
+    assert bits_differ(o, g, ("FS", "tFS")) == []
+
+
+@pytest.mark.parametrize("N,M", [(12, 9), (66, 70), (67, 68), (68, 69), (259, 12), (260, 131), (330, 10)])
+def test_run_lengths(N, M):
+    c, o, g = channel(N, M)
+    for which in (0, 1):
+        for start in (0, 10 ** 9):
+            sweep(o, g, which, 0, 4.0, start)
+
+
+@pytest.mark.parametrize("ketdinh", [0, 1])
+@pytest.mark.parametrize("field", sorted(VALUES))
+def test_values(field, ketdinh):
+    for which in (0, 1):
+        c, o, g = channel(90, 24, field, seed=which)
+        sweep(o, g, which, ketdinh, 4.0, 0)
+    c, o, g = channel(90, 24, field, seed=2)
+    o.kernel("calculate_qb", 1)
+    g.kernel("Calculate_Qb", 1)
+    o.kernel("bed_load", ketdinh, 3, c.N - 1)
+    g.kernel("BedLoad", ketdinh, 3, c.N - 1)
+    assert bits_differ(o, g, ("Qbx", "Qby", "dH")) == []
