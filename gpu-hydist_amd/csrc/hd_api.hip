@@ -365,7 +365,7 @@ int hd_create(int device, const hd_params* p, int N, int M, int series_len, int 
     if ((rc = dalloc(c, (void**)&d.dryflag, F))) { hd_destroy(c); return rc; }
     {
         size_t ncb = (size_t)(M + 3 + 63) / 64;
-        if ((rc = dalloc(c, (void**)&d.tiles, (size_t)(N + 3) * ncb * 4))) { hd_destroy(c); return rc; }
+        if ((rc = dalloc(c, (void**)&d.tiles, (size_t)(N + 3) * ncb * 8))) { hd_destroy(c); return rc; }
         if ((rc = dalloc(c, (void**)&d.ntiles, 4))) { hd_destroy(c); return rc; }
         if ((rc = dalloc(c, (void**)&d.wetb, (size_t)(N + 3) * ncb * 8))) { hd_destroy(c); return rc; }
         if ((rc = dalloc(c, (void**)&d.kh0b, (size_t)(N + 3) * ncb * 8))) { hd_destroy(c); return rc; }
@@ -522,9 +522,12 @@ static int compute_tiles(hd_ctx* c)
                 }
     std::vector<int> list;
     for (size_t t = 0; t < live.size(); ++t)
-        if (live[t]) list.push_back((int)t);
-    int n = (int)list.size();
-    if (n) HIPCHK(c, hipMemcpyAsync(c->d.tiles, list.data(), (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
+        if (live[t]) {
+            list.push_back((int)(t / ncb));
+            list.push_back((int)(t % ncb) * 64);
+        }
+    int n = (int)list.size() / 2;
+    if (n) HIPCHK(c, hipMemcpyAsync(c->d.tiles, list.data(), (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->d.ntiles, &n, 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->ntiles = n;

@@ -1621,20 +1621,16 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
     }
 }
 
-/* Cell (i, j) of a thread of a per-row kernel: with `tiled` the blocks walk
- * the context's list of active 64-column row tiles (tiles that hold, or
+/* Cell (i, j) of a thread of a per-row kernel: with `tiled` the blocks walk,
+ * `tiled` tiles each, the context's list of active 64-column row tiles (tiles that hold, or
  * border, a cell with khouot != 2: elsewhere the per-row kernels are at a
  * fixed point once a full step has run), else the full padded grid
  * (blockIdx.y = row).  Returns false for threads outside the grid. */
 __device__ __forceinline__ bool row_cell(const HdDevG& d, int tiled, int& i, int& j)
 {
     if (tiled) {
-        int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-        if (t >= d.ntiles[0]) return false;
-        int tile = d.tiles[t];
-        int ncb = (d.M + 3 + 63) >> 6;
-        i = tile / ncb;
-        j = (tile % ncb) * 64 + (threadIdx.x & 63);
+        if (!active_tile(d, xcd_block(blockIdx.x, gridDim.x) * tiled + wave_in_block(), i, j)) return false;
+        j += threadIdx.x & 63;
     } else {
         j = blockIdx.x * blockDim.x + threadIdx.x;
         i = blockIdx.y;
@@ -2270,12 +2266,13 @@ __device__ __forceinline__ void dry_store(const HdDevG& d, int i, int j, int hor
 __global__ void __launch_bounds__(256) k_smooth_u_explicit_v(const HdDev* __restrict__ dv, int tiled, int adv)
 {
     const HdDevG& d = dev_view(dv);
+    int i, j;
+    const bool cell = row_cell(d, tiled, i, j);
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
         if (adv) advance_time(d);
         roll_repairs(d, 0);
     }
-    int i, j;
-    if (!row_cell(d, tiled, i, j)) return;
+    if (!cell) return;
     const int N = d.N, M = d.M, W = d.W;
     const int p = i * W + j;
     const double sm = smooth_u_at(d, i, j);
@@ -2324,12 +2321,13 @@ __global__ void __launch_bounds__(256) k_smooth_u_explicit_v(const HdDev* __rest
 __global__ void __launch_bounds__(256) k_smooth_v_explicit_u(const HdDev* __restrict__ dv, int tiled, int adv)
 {
     const HdDevG& d = dev_view(dv);
+    int i, j;
+    const bool cell = row_cell(d, tiled, i, j);
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
         if (adv) advance_time(d);
         roll_repairs(d, 1);
     }
-    int i, j;
-    if (!row_cell(d, tiled, i, j)) return;
+    if (!cell) return;
     const int N = d.N, M = d.M, W = d.W;
     const int p = i * W + j;
     const double sm = smooth_v_at(d, i, j);
@@ -2552,17 +2550,17 @@ __global__ void __launch_bounds__(64) k_smooth_wet(const HdDev* __restrict__ dv,
         wetting_line(d, horizontal, blockIdx.x, mode);
         return;
     }
-    const int t = (int)blockIdx.x - nlb;
+    const int t = xcd_block((int)blockIdx.x - nlb, (int)gridDim.x - nlb);
     const int ncb = (d.M + 3 + 63) >> 6;
-    int tile;
+    int i, j;
     if (tiled) {
-        if (t >= d.ntiles[0]) return;
-        tile = d.tiles[t];
+        if (!active_tile(d, t, i, j)) return;
     } else {
         if (t >= (d.N + 3) * ncb) return;
-        tile = t;
+        i = t / ncb;
+        j = (t % ncb) * 64;
     }
-    const int i = tile / ncb, j = (tile % ncb) * 64 + (int)threadIdx.x;
+    j += (int)threadIdx.x;
     const int N = d.N, M = d.M, W = d.W;
     if (j >= M + 3) return;
     const int p = i * W + j;
@@ -2630,9 +2628,10 @@ __global__ void __launch_bounds__(256) k_uvz(const HdDev* __restrict__ dv, int k
 {
     const HdDevG& d = dev_view(dv);
     /* the run tables are rebuilt by the next kernel on the stream */
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { d.run_cnt[0] = 0; d.run_cnt[1] = 0; }
     int i, j;
-    if (!row_cell(d, tiled, i, j)) return;
+    const bool cell = row_cell(d, tiled, i, j);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { d.run_cnt[0] = 0; d.run_cnt[1] = 0; }
+    if (!cell) return;
     uvz_cell(d, i, j, kd, kn);
 }
 
@@ -3183,17 +3182,17 @@ __global__ void __launch_bounds__(256) k_uvz_segments(const HdDev* __restrict__ 
         find_limits_block(d, bid, nrowb, ncolb, nfsr, count_wet, d.dryflag, kd, kn);
         return;
     }
-    const int t = ((int)blockIdx.x - nseg) * 4 + (threadIdx.x >> 6);
+    const int t = xcd_block((int)blockIdx.x - nseg, (int)gridDim.x - nseg) * 4 + wave_in_block();
     const int ncb = (d.M + 3 + 63) >> 6;
-    int tile;
+    int i, j;
     if (tiled) {
-        if (t >= d.ntiles[0]) return;
-        tile = d.tiles[t];
+        if (!active_tile(d, t, i, j)) return;
     } else {
         if (t >= (d.N + 3) * ncb) return;
-        tile = t;
+        i = t / ncb;
+        j = (t % ncb) * 64;
     }
-    const int i = tile / ncb, j = (tile % ncb) * 64 + (threadIdx.x & 63);
+    j += threadIdx.x & 63;
     if (j >= d.M + 3) return;
     uvz_cell(d, i, j, kd, kn);
 }
@@ -3412,7 +3411,7 @@ static inline dim3 row_grid(const HdBatch& b, int bw, int ntiles)
 void hd_launch_normalize_post(const HdBatch& b, int isU, int post, int horizontal, int bw, int ntiles, hipStream_t s)
 {
     hipLaunchKernelGGL(k_normalize, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, isU, post, horizontal,
-                       ntiles > 0 ? 1 : 0);
+                       ntiles > 0 ? bw >> 6 : 0);
 }
 
 void hd_launch_explicit(const HdBatch& b, int isU, hipStream_t s)
@@ -3439,19 +3438,19 @@ void hd_launch_explicit_margins(const HdBatch& b, int isU, int cells, hipStream_
 
 void hd_launch_smooth_u_explicit_v(const HdBatch& b, int bw, int ntiles, int adv, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_smooth_u_explicit_v, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, ntiles > 0 ? 1 : 0,
+    hipLaunchKernelGGL(k_smooth_u_explicit_v, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, ntiles > 0 ? bw >> 6 : 0,
                        adv);
 }
 
 void hd_launch_smooth_v_explicit_u(const HdBatch& b, int bw, int ntiles, int adv, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_smooth_v_explicit_u, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, ntiles > 0 ? 1 : 0,
+    hipLaunchKernelGGL(k_smooth_v_explicit_u, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, ntiles > 0 ? bw >> 6 : 0,
                        adv);
 }
 
 void hd_launch_explicit_rows_u(const HdBatch& b, int bw, int ntiles, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_explicit_rows_u, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, ntiles > 0 ? 1 : 0);
+    hipLaunchKernelGGL(k_explicit_rows_u, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, ntiles > 0 ? bw >> 6 : 0);
 }
 
 void hd_launch_smooth_wet(const HdBatch& b, int isU, int horizontal, int ntiles, int mode, hipStream_t s)
@@ -3470,7 +3469,7 @@ void hd_launch_wetting(const HdBatch& b, int horizontal, int mode, hipStream_t s
 
 void hd_launch_uvz_dry(const HdBatch& b, int kd, int kn, int bw, int ntiles, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_uvz, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, kd, kn, ntiles > 0 ? 1 : 0);
+    hipLaunchKernelGGL(k_uvz, row_grid(b, bw, ntiles), dim3(bw), 0, s, b.dv, kd, kn, ntiles > 0 ? bw >> 6 : 0);
 }
 
 void hd_launch_flow_refresh(const HdBatch& b, hipStream_t s)

@@ -14,18 +14,14 @@
 
 namespace {
 
-/* Cell (i, j) of a thread over the context's active 64-column row tiles
+/* Cell (i, j) of a thread of a block of 256 over the context's active 64-column row tiles
  * (tiles holding or bordering a cell with khouot != 2): outside them the
  * sediment kernels that run by tiles have reached a fixed point once they
  * have run over the whole grid, which the caller arranges. */
 __device__ __forceinline__ bool tile_cell(const HdDevG& d, int& i, int& j)
 {
-    const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (t >= d.ntiles[0]) return false;
-    const int tile = d.tiles[t];
-    const int ncb = (d.M + 3 + 63) >> 6;
-    i = tile / ncb;
-    j = (tile % ncb) * 64 + (threadIdx.x & 63);
+    if (!active_tile(d, xcd_block(blockIdx.x, gridDim.x) * 4 + wave_in_block(), i, j)) return false;
+    j += threadIdx.x & 63;
     return j < d.M + 3 && i < d.N + 3;
 }
 
