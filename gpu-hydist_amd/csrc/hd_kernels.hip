@@ -2371,20 +2371,25 @@ __global__ void __launch_bounds__(256) k_smooth_v_explicit_u(const HdDev* __rest
  * _vertical (:152-171), one wave per line.  The serial scan can only act at
  * positions next to a khouot == 1 cell; those were recorded by the drying
  * marks (dry_store, or k_normalize with post in the cross-check forms).
- * The wave sorts them (ranks by comparison), every lane loads the window of
- * one recorded position p at once (khouot and htaiz at p-1 .. p+kWetLA+1, z
- * at p .. p+kWetLA, t_z and FS at p), and lane 0 replays the scan over the
- * recorded positions in increasing order from LDS: a visit at q opens q-1
- * and q+1 where khouot == 1 and t_z(q) > z(q), copying q's t_z and FS;
- * opening q+1 makes q+1 the next visit, with q's values (the reference's
- * cascade).  Within a window every value is current except khouot at q-1
- * when an earlier visit opened it from the left, which is tracked; a
- * cascade past the window reads global memory.  With up to kWetFew
- * candidates lane 0 loads as it visits (one round of loads per visit); a
- * line with more candidates than the list holds is scanned in full. */
+ * Count and positions are read in one trip; every lane then loads the window
+ * of one recorded position p at once (khouot and htaiz at p-1 .. p+kWetLA+1,
+ * z at p .. p+kWetLA, t_z and FS at p).  A visit at q opens q-1 and q+1
+ * where khouot == 1 and t_z(q) > z(q), copying q's t_z and FS; opening q+1
+ * makes q+1 the next visit, with q's values (the reference's cascade).
+ * Where no cascade leaves its window and the positions lie kWetApart or more
+ * apart, no visit reads what another wrote, and the lanes do theirs at once
+ * from registers.  Otherwise the windows go to LDS in the order of the
+ * positions (ranks by comparison) and lane 0 replays the scan over the
+ * recorded positions in increasing order: within a window every value is
+ * current except khouot at q-1 when an earlier visit opened it from the
+ * left, which is tracked; a cascade past the window reads global memory.  A
+ * line with more candidates than the list holds is scanned in full.
+ * The lines with candidates end a launch: a trip to memory per visit made
+ * them last up to 7 us, the replay from LDS 5.2 us, this 4.6 us beside 2.7 us
+ * for the tiles of the same launch (980 x 1048 river grid). */
 constexpr int kWetLA = 3;           /* cascade steps a window covers */
-constexpr int kWetFew = 8;          /* up to this many candidates lane 0 loads as it visits */
 constexpr int kWetWin = kWetLA + 3; /* khouot / htaiz entries p-1 .. p+kWetLA+1 */
+constexpr int kWetApart = kWetLA + 2; /* a cascade within its window opens p-1 .. p+kWetLA */
 
 __device__ __forceinline__ void wetting_line(const HdDevG& d, int horizontal, int line, int mode)
 {
@@ -2392,7 +2397,8 @@ __device__ __forceinline__ void wetting_line(const HdDevG& d, int horizontal, in
     const int N = d.N, M = d.M, W = d.W;
     if (line < 1 || line > (horizontal ? N : M)) return;
     int* cand_cnt = d.cand_cnt;
-    const int n = cand_cnt[line];
+    const int cr = d.cand[line * kCand + lane];
+    const int n = __builtin_amdgcn_readfirstlane(cand_cnt[line]);
     if (n == 0) return;
     if (lane == 0) cand_cnt[line] = 0;
     const int pmax = horizontal ? M : N;
@@ -2418,8 +2424,8 @@ __device__ __forceinline__ void wetting_line(const HdDevG& d, int horizontal, in
             atomicOr((unsigned long long*)d.wetb + (size_t)r * ((M + 3 + 63) >> 6) + (cc >> 6), 1ull << (cc & 63));
         }
     };
-    /* mode (a cross-check of the three ways, same bits): 0 as described,
-     * 1 windows for every line, 2 the whole-line scan for every line */
+    /* mode (a cross-check, same bits): 0 and 1 as described, 2 the whole-line
+     * scan for every line */
     if (n > kCand || mode == 2) { /* more candidates than recorded: the whole line, one visit per round of loads */
         if (lane != 0) return;
         bool cascade = false;
@@ -2447,26 +2453,61 @@ __device__ __forceinline__ void wetting_line(const HdDevG& d, int horizontal, in
     __shared__ int s_pos[kCand];
     __shared__ int s_kh[kCand][kWetWin];
     __shared__ double s_ht[kCand][kWetWin], s_z[kCand][kWetLA + 1], s_tz[kCand], s_fs[kCand];
-    /* the recorded positions (distinct), sorted by rank */
-    const int c = lane < n ? d.cand[line * kCand + lane] : 0x7fffffff;
+    /* the window of one position, all loads at once (lanes past the last
+     * candidate repeat it) */
+    const int p = lane < n ? cr : __builtin_amdgcn_readlane(cr, n - 1);
+    int wkh[kWetWin];
+    double wht[kWetWin], wz[kWetLA + 1];
+    const double wtz = tz[at(p)], wfs = FS[at(p)];
+#pragma unroll
+    for (int o = 0; o < kWetWin; ++o) {
+        const int q = p - 1 + o < pmax + 1 ? p - 1 + o : pmax + 1;
+        wkh[o] = kh[at(q)];
+        wht[o] = ht[at(q)];
+    }
+#pragma unroll
+    for (int o = 0; o <= kWetLA; ++o) wz[o] = z[at(p + o < pmax ? p + o : pmax)];
+    /* the rank among the recorded positions (distinct), and whether the next
+     * one is near */
     int rank = 0;
-    for (int k = 0; k < n; ++k) rank += __shfl(c, k, kWave) < c;
-    if (lane < n) s_pos[rank] = c;
-    __syncthreads();
-    const bool win = n > (mode == 1 ? 0 : kWetFew); /* with few candidates lane 0 loads as it visits */
-    if (win && lane < n) { /* the window of one position, all loads at once */
-        const int p = s_pos[lane];
-        s_tz[lane] = tz[at(p)];
-        s_fs[lane] = FS[at(p)];
+    bool near = false;
+    for (int k = 0; k < n; ++k) {
+        const int ck = __builtin_amdgcn_readlane(cr, k);
+        rank += ck < p;
+        near = near || (ck > p && ck - p < kWetApart);
+    }
+    /* the visits o = 0 .. kWetLA of the lane's own cascade: vis[o] that the
+     * visit is made and its level lies above the bed */
+    bool vis[kWetLA + 1], more = lane < n && p >= 2 && p <= pmax;
+#pragma unroll
+    for (int o = 0; o <= kWetLA; ++o) {
+        vis[o] = more && p + o <= pmax && wtz > wz[o];
+        more = vis[o] && p + o + 1 <= pmax + 1 && wkh[o + 2] == 1;
+    }
+    if (!__any(near || more)) {
+        if (lane < n) {
+            /* left of p, p itself (from p + 1), then to the right; cells
+             * further left were opened by the cascade */
+            if (vis[0] && wkh[0] == 1) open(p - 1, wtz, wfs, wht[0]);
+            if (vis[1] && wkh[1] == 1) open(p, wtz, wfs, wht[1]);
+#pragma unroll
+            for (int o = 0; o < kWetLA; ++o)
+                if (vis[o] && p + o + 1 <= pmax + 1 && wkh[o + 2] == 1) open(p + o + 1, wtz, wfs, wht[o + 2]);
+        }
+        return;
+    }
+    if (lane < n) {
+        s_pos[rank] = p;
+        s_tz[rank] = wtz;
+        s_fs[rank] = wfs;
 #pragma unroll
         for (int o = 0; o < kWetWin; ++o) {
-            const int q = p - 1 + o;
-            const bool in = q <= pmax + 1;
-            s_kh[lane][o] = in ? kh[at(q)] : 2;
-            s_ht[lane][o] = in ? ht[at(q)] : 0.0;
+            const bool in = p - 1 + o <= pmax + 1;
+            s_kh[rank][o] = in ? wkh[o] : 2;
+            s_ht[rank][o] = in ? wht[o] : 0.0;
         }
 #pragma unroll
-        for (int o = 0; o <= kWetLA; ++o) s_z[lane][o] = p + o <= pmax ? z[at(p + o)] : 0.0;
+        for (int o = 0; o <= kWetLA; ++o) s_z[rank][o] = p + o <= pmax ? wz[o] : 0.0;
     }
     __syncthreads();
     if (lane != 0) return;
@@ -2488,7 +2529,7 @@ __device__ __forceinline__ void wetting_line(const HdDevG& d, int horizontal, in
         const int o = pos - s_pos[bw];
         double zc, htm, htn, tzv, fsv;
         int km, kn;
-        if (win && o <= kWetLA) {
+        if (o <= kWetLA) {
             zc = s_z[bw][o];
             km = s_kh[bw][o];
             kn = s_kh[bw][o + 2];
@@ -2600,27 +2641,26 @@ __global__ void __launch_bounds__(64) k_smooth_wet(const HdDev* __restrict__ dv,
 __device__ __forceinline__ void uvz_cell(const HdDevG& d, int i, int j, int kd, int kn)
 {
     const unsigned char* dryflag = d.dryflag;
-    int N = d.N, M = d.M, W = d.W;
-    int p = i * W + j;
-    bool me = dryflag[p];
-    bool dn = (i + 1 <= N + 2) ? dryflag[p + W] : false;
-    bool rt = (j + 1 <= M + 2) ? dryflag[p + 1] : false;
+    const int N = d.N, M = d.M, W = d.W;
+    const int p = i * W + j;
+    const int pd = i + 1 <= N + 2 ? p + W : p, pr = j + 1 <= M + 2 ? p + 1 : p;
+    const int pu = i >= 1 ? p - W : p, pl = j >= 1 ? p - 1 : p;
+    /* one round of loads, ahead of the stores */
+    const bool me = dryflag[p], dn = dryflag[pd] && pd != p, rt = dryflag[pr] && pr != p;
     double tu = d.t_u[p], tv = d.t_v[p];
+    const double zc = d.t_z[p], h0 = d.h[p], hl = d.h[pl], hu = d.h[pu];
+    const double zd = (i + 1 <= N ? d.t_z : d.z)[pd], zr = (j + 1 <= M ? d.t_z : d.z)[pr];
     if (me || dn) { tu = 0; d.t_u[p] = 0; }
     if (me || rt) { tv = 0; d.t_v[p] = 0; }
     if (me) { d.khouot[p] = 1; d.FS[p] = 0; }
     if (i <= N && j <= M) {
-        d.z[p] = d.t_z[p];
+        d.z[p] = zc;
         d.u[p] = tu * (1 - kd);
         d.v[p] = tv * (1 - kn);
     }
     if (i >= 1 && i <= N && j >= 1 && j <= M) {
-        const double* h = d.h;
-        double zc = d.t_z[p];
-        double zd = (i + 1 <= N) ? d.t_z[p + W] : d.z[p + W];
-        double zr = (j + 1 <= M) ? d.t_z[p + 1] : d.z[p + 1];
-        d.Htdu[p] = (h[i * W + j - 1] + h[p] + zd + zc) * 0.5;
-        d.Htdv[p] = (h[(i - 1) * W + j] + h[p] + zr + zc) * 0.5;
+        d.Htdu[p] = (hl + h0 + zd + zc) * 0.5;
+        d.Htdv[p] = (hu + h0 + zr + zc) * 0.5;
     }
 }
 
@@ -2898,6 +2938,18 @@ __device__ __forceinline__ RunBits run_bits(unsigned long long m, int base, int 
     return r;
 }
 
+/* inclusive prefix sum over the wave (row shifts and broadcasts) */
+__device__ __forceinline__ int wave_prefix(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 /* The runs of row i (positions 2..M) by one wave from its wet bits: a word
  * per lane (64 words = 4096 cells per batch), neighbours' edge bits by
  * shuffles, ranks by a wave prefix sum.  Entries k < SL go to dau / cuoi
@@ -2918,17 +2970,13 @@ __device__ __forceinline__ int row_word_scan(const HdDevG& d, int i, int lane, i
         unsigned long long m = w < ncb ? row[w] : 0ull;
         m &= bits_upto(L - base) & ~bits_upto(1 - base);
         const unsigned after = wetx(64 * (w0 + kWave));
-        const unsigned long long pw = __shfl_up(m, 1, kWave), nw = __shfl_down(m, 1, kWave);
-        const unsigned prev = lane == 0 ? carry : (unsigned)(pw >> 63);
-        const unsigned next = lane == kWave - 1 ? after : (unsigned)(nw & 1);
-        carry = (unsigned)(__shfl(m, kWave - 1, kWave) >> 63);
+        /* the last bit of the lane before, the first of the lane after */
+        const unsigned prev = (unsigned)__builtin_amdgcn_update_dpp((int)carry, (int)(m >> 63), 0x138, 0xF, 0xF, false);
+        const unsigned next = (unsigned)__builtin_amdgcn_update_dpp((int)after, (int)(m & 1), 0x130, 0xF, 0xF, false);
+        carry = (unsigned)__builtin_amdgcn_readlane((int)(m >> 63), kWave - 1);
         const RunBits rb = run_bits(m, base, L, prev, next, wl2, wl1);
         const int cs = __popcll(rb.st), ce = __popcll(rb.en);
-        int ps = cs, pe = ce; /* inclusive prefix over the lanes */
-        for (int o = 1; o < kWave; o <<= 1) {
-            const int a = __shfl_up(ps, o, kWave), b = __shfl_up(pe, o, kWave);
-            if (lane >= o) { ps += a; pe += b; }
-        }
+        const int ps = wave_prefix(cs), pe = wave_prefix(ce);
         int ks = ns + ps - cs, ke = ne + pe - ce;
         for (unsigned long long b = rb.st; b; b &= b - 1, ++ks) {
             const int x = base + __ffsll(b) - 1;
@@ -2938,27 +2986,55 @@ __device__ __forceinline__ int row_word_scan(const HdDevG& d, int i, int lane, i
             const int x = base + __ffsll(b) - 1;
             if (ke < SL) { cuoi[ke] = x; sl[ke] = x; }
         }
-        ns += __shfl(ps, kWave - 1, kWave);
-        ne += __shfl(pe, kWave - 1, kWave);
+        ns += __builtin_amdgcn_readlane(ps, kWave - 1);
+        ne += __builtin_amdgcn_readlane(pe, kWave - 1);
     }
     return ns;
+}
+
+/* the value of lane ^ S (S a power of two up to 16), without LDS */
+template <int S>
+__device__ __forceinline__ unsigned lane_xor(unsigned v, int lane)
+{
+    if constexpr (S == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return lane & 16 ? r[0] : r[1];
+    } else if constexpr (S == 4) {
+        const int a = __builtin_amdgcn_update_dpp(0, (int)v, 0x104, 0xF, 0x5, false);
+        return (unsigned)__builtin_amdgcn_update_dpp(a, (int)v, 0x114, 0xF, 0xA, false);
+    } else {
+        constexpr int kCtrl = S == 8 ? 0x128 : (S == 2 ? 0x4E : 0xB1); /* row_ror:8, quad_perm */
+        return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xF, 0xF, true);
+    }
+}
+
+template <int S>
+__device__ __forceinline__ void transpose_step(unsigned& lo, unsigned& hi, int lane)
+{
+    constexpr unsigned kKeep = S == 16 ? 0x0000FFFFu : S == 8 ? 0x00FF00FFu : S == 4 ? 0x0F0F0F0Fu
+                                       : S == 2 ? 0x33333333u : 0x55555555u;
+    const unsigned bl = lane_xor<S>(lo, lane), bh = lane_xor<S>(hi, lane);
+    const bool up = lane & S;
+    lo = up ? ((bl >> S) & kKeep) | (lo & ~kKeep) : (lo & kKeep) | ((bl & kKeep) << S);
+    hi = up ? ((bh >> S) & kKeep) | (hi & ~kKeep) : (hi & kKeep) | ((bh & kKeep) << S);
 }
 
 /* Transpose of a 64 x 64 bit block held one row per lane (bit q of lane r
  * = element (r, q)): afterwards lane q holds column q (bit r = element
  * (r, q)).  Six rounds; in round s the lanes r and r ^ s swap the
- * off-diagonal s x s sub-blocks of their 2s x 2s block. */
+ * off-diagonal s x s sub-blocks of their 2s x 2s block (round 32: one swap
+ * of half-waves between the two words), by lane moves that need no trip
+ * through LDS. */
 __device__ __forceinline__ unsigned long long transpose64(unsigned long long a, int lane)
 {
-    constexpr unsigned long long kKeep[6] = {0x00000000FFFFFFFFull, 0x0000FFFF0000FFFFull, 0x00FF00FF00FF00FFull,
-                                             0x0F0F0F0F0F0F0F0Full, 0x3333333333333333ull, 0x5555555555555555ull};
-#pragma unroll
-    for (int k = 0, sh = 32; k < 6; ++k, sh >>= 1) {
-        const unsigned long long b = __shfl_xor(a, sh, kWave);
-        if (lane & sh) a ^= ((b >> sh) ^ a) & kKeep[k];
-        else a ^= (((a >> sh) ^ b) & kKeep[k]) << sh;
-    }
-    return a;
+    const auto w = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)(a >> 32), false, false);
+    unsigned lo = w[0], hi = w[1];
+    transpose_step<16>(lo, hi, lane);
+    transpose_step<8>(lo, hi, lane);
+    transpose_step<4>(lo, hi, lane);
+    transpose_step<2>(lo, hi, lane);
+    transpose_step<1>(lo, hi, lane);
+    return ((unsigned long long)hi << 32) | lo;
 }
 
 /* The column tables of Find_Calculation_limits_Vertical (the run rule of
@@ -3033,15 +3109,11 @@ __device__ __forceinline__ int col_word_scan(const HdDevG& d, int cb, int* s_f, 
             int ns = s_ts[lane];
             for (int w = 0; w < 4; ++w) ns += s_cs[w][lane];
             const int nn = colok ? (ns < SL ? ns : SL) : 0;
-            int p = nn;
-            for (int o = 1; o < kWave; o <<= 1) {
-                const int a = __shfl_up(p, o, kWave);
-                if (lane >= o) p += a;
-            }
-            const int tot = __shfl(p, kWave - 1, kWave);
+            const int p = wave_prefix(nn);
+            const int tot = __builtin_amdgcn_readlane(p, kWave - 1);
             int base = 0;
             if (lane == 0 && tot) base = atomicAdd(d.run_cnt + 0, tot);
-            s_cbase[lane] = __shfl(base, 0, kWave) + p - nn;
+            s_cbase[lane] = __builtin_amdgcn_readfirstlane(base) + p - nn;
         }
         int ks = s_ts[lane], ke = s_te[lane];
         for (int w = 0; w < c; ++w) { ks += s_cs[w][lane]; ke += s_ce[w][lane]; }
