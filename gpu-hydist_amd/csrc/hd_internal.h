@@ -148,10 +148,10 @@ struct RunSlice {
 };
 __device__ __forceinline__ RunSlice run_slice(int cnt, int G = (int)gridDim.x)
 {
-    const int nx = G < 8 ? 1 : 8;
-    const int x = (int)blockIdx.x % nx, slot = (int)blockIdx.x / nx;
-    const int per = (G - x + nx - 1) / nx; /* workgroups on XCD x */
-    const int chunk = (cnt + nx - 1) / nx;
+    const int sh = G < 8 ? 0 : 3, nx = 1 << sh;
+    const int x = (int)blockIdx.x & (nx - 1), slot = (int)blockIdx.x >> sh;
+    const int per = (G - x + nx - 1) >> sh; /* workgroups on XCD x */
+    const int chunk = (cnt + nx - 1) >> sh;
     const int lo = x * chunk;
     return RunSlice{lo + slot, cnt < lo + chunk ? cnt : lo + chunk, per};
 }

@@ -1375,8 +1375,8 @@ __device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreR
 /* Fused UZ / VZ solve of one wet run per wave with the speculative parallel
  * Thomas of hd_thomas.h: the same rows as k_adi_run (_calculate_preindex,
  * _calculate_abcd, _calculate_matrix_coeff, tridiag, _extract_solution,
- * UVZSolver_multithread.cu:203-723) and the same bits.  Chunks of 255 cells
- * (510 rows) are assembled by the lanes, 63 cells a round, into LDS; the
+ * UVZSolver_multithread.cu:203-723) and the same bits.  Chunks of 252 cells
+ * (504 rows) are assembled by the lanes, 63 cells a round, into LDS; the
  * forward sweep (factors replacing C / D) and the back
  * substitution (x replacing A) run over the chunk on all lanes; factors of
  * all but the last chunk go to the run's slice of the Ap/Bp line buffers and
@@ -1401,7 +1401,7 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
 {
     const HdDevG& d = dev_view(dv);
     const int sidx = 2 + shift, eidx = isU ? d.M - shift : d.N;
-    constexpr int CH = 255; /* cells per LDS chunk (the rows of cell t need cells t and t + 1) */
+    constexpr int CH = 252; /* cells per LDS chunk: four rounds */
     constexpr int RW = 2 * CH;
     /* rows at SpecMap positions; the run's first row (0) and last (sn),
      * which the sweeps leave out, at the last two words */
@@ -1513,44 +1513,50 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
                     if (k == last) { sE[3] = o.a2; sE[4] = o.c2; sE[5] = o.d2; }
                     /* rows 2 (k - first) and the one after: continuity of k
                      * and momentum of k, or from an open start momentum of k
-                     * and continuity of k + 1; the end row's condition wins */
+                     * and continuity of k + 1 */
                     int rc = 2 * (k - first), rm = rc + 1;
-                    double md = o.d1, cd = o.d2;
                     if (skind == S_OPEN) {
                         rm = rc++;
-                        o.a2 = o.na2; o.c2 = o.nc2; o.d2 = cd = o.nd2;
-                        if (rm == 0) md = o.d1 - o.a1 * TZ_l;
-                    } else if (skind == S_Q) {
-                        if (rc == 0) cd = o.d2 - o.a2 * ub1;
-                    }
-                    if (ekind == E_OPEN) {
-                        if (rm == sn) md = o.d1 - o.c1 * TZ_r;
-                    } else if (rc == sn) {
-                        cd = ekind == E_Q ? o.d2 - o.c2 * ub2 : o.d2;
+                        o.a2 = o.na2; o.c2 = o.nc2; o.d2 = o.nd2;
                     }
                     if (lane < 63 && k <= c1) {
                         if (rc <= sn) {
                             const int ix = rc == 0 ? kRow0 : (rc == sn ? kRowN : sm.pos(rc - rb));
-                            sA[ix] = o.a2; sB[ix] = 1.0; sC[ix] = o.c2; sD[ix] = cd;
+                            sA[ix] = o.a2; sB[ix] = 1.0; sC[ix] = o.c2; sD[ix] = o.d2;
                         }
                         if (rm <= sn) {
                             const int ix = rm == 0 ? kRow0 : (rm == sn ? kRowN : sm.pos(rm - rb));
-                            sA[ix] = o.a1; sB[ix] = o.b1; sC[ix] = o.c1; sD[ix] = md;
+                            sA[ix] = o.a1; sB[ix] = o.b1; sC[ix] = o.c1; sD[ix] = o.d1;
                         }
                     }
                 }
                 __syncthreads();
+                /* the first and last row's conditions; the end's wins */
+                const bool open1 = skind == S_OPEN, lastmom = ((sn & 1) != 0) != open1;
                 if (c == 0) {
+                    const double A = sA[kRow0], B = sB[kRow0], C = sC[kRow0];
+                    double D = sD[kRow0];
+                    if (sn == 0 && lastmom == (ekind == E_OPEN)) {
+                        if (lastmom) D = D - C * TZ_r;
+                        else if (ekind == E_Q) D = D - C * ub2;
+                    } else if (open1) {
+                        D = D - A * TZ_l;
+                    } else if (skind == S_Q) {
+                        D = D - A * ub1;
+                    }
                     if (sn == 0) {
-                        xs = sD[kRow0] / sB[kRow0];
+                        xs = D / B;
                     } else {
-                        ap0 = ap = -sC[kRow0] / sB[kRow0];
-                        bp0 = bp = sD[kRow0] / sB[kRow0];
+                        ap0 = ap = -C / B;
+                        bp0 = bp = D / B;
                     }
                 }
                 spec_forward<kSpecMaxLg>(sA, sB, sC, sD, sm, n, ap, bp, fails);
                 if (c == nch - 1 && sn > 0) {
-                    const double A = sA[kRowN], B = sB[kRowN], D = sD[kRowN];
+                    const double A = sA[kRowN], B = sB[kRowN], C = sC[kRowN];
+                    double D = sD[kRowN];
+                    if (lastmom && ekind == E_OPEN) D = D - C * TZ_r;
+                    else if (!lastmom && ekind == E_Q) D = D - C * ub2;
                     xs = (D - (A * bp)) / (B + (A * ap));
                 }
                 if (c + 1 < nch) { /* this chunk's factors to the line buffers */
