@@ -63,6 +63,27 @@ __device__ __forceinline__ void st_row(E* base, size_t row, unsigned off, T v)
 {
     *(T*)((char*)(base + row) + off) = v;
 }
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+/* A row of `bytes` bytes as a buffer: loads past either end of it return
+ * zeros and stores there are dropped (an offset below 0 is far past the end),
+ * and none of a row of 0 bytes is touched.  So every step of a walk over
+ * rows has the same memory operations, which is what lets the compiler count
+ * those in flight instead of waiting for all of them. */
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const void* base, size_t at, unsigned bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)base + at), 0, (int)bytes, 0x00020000);
+}
+template <typename T>
+__device__ __forceinline__ T buf_ld16(__amdgpu_buffer_rsrc_t r, unsigned off)
+{
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
+}
+template <typename T>
+__device__ __forceinline__ void buf_st16(__amdgpu_buffer_rsrc_t r, unsigned off, T v)
+{
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, (int)off, 0, 0);
+}
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 /* The work of one convolution launch, in items of a strip of rows: item k
@@ -134,6 +155,7 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
 #pragma unroll
         for (int q = 0; q < 4 * NB; ++q) bv[q] = bias[cb + q];
     }
+    __builtin_amdgcn_s_waitcnt(0x0f70); /* weights and bias are here: no wait for them in the loop */
     const bf16x8 zero8 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
     const int H = it.H, W = it.W;
     constexpr int PER = 64 / (16 * SW); /* items per tile of the list */
@@ -158,45 +180,39 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
         w0 = uniform(w0);
         r0 = uniform(r0);
         r1 = uniform(r1 < H ? r1 : H);
-        /* the thread's pieces of a row: byte offsets; outside the image they
-         * read some other column and are zeroed on their way to LDS */
+        /* the thread's pieces of a row: byte offsets, columns outside the
+         * image past the row's ends */
         struct Piece {
             bf16x8 q[NL];
             unsigned last;
         };
         unsigned vo[NL], vl = 0;
-        bool oq[NL], ol = false;
 #pragma unroll
         for (int q = 0; q < NL; ++q) {
             const int e = threadIdx.x + 256 * q, c = w0 - 1 + e / (CS / 8);
-            oq[q] = c >= 0 && c < W;
-            vo[q] = 2u * ((unsigned)(c < 0 ? 0 : (c < W ? c : W - 1)) * CS + e % (CS / 8) * 8);
+            vo[q] = 2u * (unsigned)(c * CS + e % (CS / 8) * 8);
         }
-        if (!NARROW) {
-            const int c = w0 - 1 + PX - 2 + (l >> 5);
-            ol = c < W;
-            vl = 2u * (unsigned)(c < W ? c : W - 1) * CS + 4u * (l & 31);
-        }
+        if (!NARROW) vl = 2u * (unsigned)((w0 - 1 + PX - 2 + (l >> 5)) * CS) + 4u * (l & 31);
+        /* byte offset of row y of the item's image, E bytes a pixel; rows off
+         * the image have no bytes */
+        auto row_at = [&](int y, int E) -> size_t { return (img + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E; };
         auto load = [&](int i, Piece& r) {
-            if (i < 0 || i >= H) return;
-            const size_t row = (img + (size_t)uniform(i * W)) * CS;
+            const auto b = row_buffer(X, row_at(i, 2 * CS), i >= 0 && i < H && i <= r1 ? 2u * CS * (unsigned)W : 0u);
 #pragma unroll
-            for (int q = 0; q < NL; ++q) r.q[q] = ld_row<bf16x8>(X, row, vo[q]);
-            if (!NARROW) r.last = ld_row<unsigned>(X, row, vl);
+            for (int q = 0; q < NL; ++q) r.q[q] = buf_ld16<bf16x8>(b, vo[q]);
+            if (!NARROW) r.last = __builtin_amdgcn_raw_buffer_load_b32(b, (int)vl, 0, 0);
         };
         auto store = [&](int i, const Piece& r) {
-            const bool in = i >= 0 && i < H;
             bf16* to = ring[i & 3];
 #pragma unroll
             for (int q = 0; q < NL; ++q) {
                 const int e = threadIdx.x + 256 * q;
-                if (!NARROW || e < PX) *(bf16x8*)(to + e / (CS / 8) * PS + e % (CS / 8) * 8) = in && oq[q] ? r.q[q] : zero8;
+                if (!NARROW || e < PX) *(bf16x8*)(to + e / (CS / 8) * PS + e % (CS / 8) * 8) = r.q[q];
             }
-            if (!NARROW && wv == 0) *(unsigned*)(to + (PX - 2 + (l >> 5)) * PS + 2 * (l & 31)) = in && ol ? r.last : 0u;
+            if (!NARROW && wv == 0) *(unsigned*)(to + (PX - 2 + (l >> 5)) * PS + 2 * (l & 31)) = r.last;
         };
         const int col = w0 + 16 * strip + n;
-        const bool live = w0 + 16 * strip < W, out = col < W;
-        const unsigned oe = (unsigned)(out ? col : W - 1) * kWidth + cb; /* the lane's results in a row of 64 channels */
+        const unsigned oe = (unsigned)col * kWidth + cb; /* the lane's results in a row of 64 channels */
         /* old dA and the gate of an output row, loaded a row ahead */
         struct Old {
             f32x4 a, b;
@@ -204,19 +220,34 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
         };
         auto load_old = [&](int y, Old& o) {
             if (EPI != EPI_BWD_SET && EPI != EPI_BWD_ADD) return;
-            if (y < r0 || y >= r1) return;
-            const size_t p = img + (size_t)uniform(y * W);
+            const unsigned w = y >= r0 && y < r1 ? (unsigned)W : 0u;
             if (EPI == EPI_BWD_ADD) {
-                o.a = ld_row<f32x4>(Yf, p * kWidth, 4 * oe);
-                o.b = ld_row<f32x4>(Yf, p * kWidth, 4 * oe + 16);
+                const auto b = row_buffer(Yf, row_at(y, 4 * kWidth), 4 * kWidth * w);
+                o.a = buf_ld16<f32x4>(b, 4 * oe);
+                o.b = buf_ld16<f32x4>(b, 4 * oe + 16);
             }
-            o.gate = ld_row<unsigned char>(gate, p * 8, oe >> 3);
+            o.gate = __builtin_amdgcn_raw_buffer_load_b8(row_buffer(gate, row_at(y, 8), 8 * w), (int)(oe >> 3), 0, 0);
+        };
+        /* the results of output row y, or with w = 0 the same stores to nowhere */
+        auto put = [&](int y, unsigned w, bf16x8 yv, unsigned bits, const f32x4& d0, const f32x4& d1) {
+            if (EPI == EPI_LINEAR) {
+                buf_st16(row_buffer(Yf, row_at(y, 4 * kOut4), 4 * kOut4 * w), g == 0 ? 16u * col : ~0u, d0);
+                return;
+            }
+            if (EPI == EPI_BWD_SET || EPI == EPI_BWD_ADD) {
+                const auto b = row_buffer(Yf, row_at(y, 4 * kWidth), store_f ? 4 * kWidth * w : 0u);
+                buf_st16(b, 4 * oe, d0);
+                buf_st16(b, 4 * oe + 16, d1);
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b8((unsigned char)bits, row_buffer(gate, row_at(y, 8), gate ? 8 * w : 0u),
+                                                     (int)(oe >> 3), 0, 0);
+            }
+            buf_st16(row_buffer(Y, row_at(y, 2 * kWidth), 2 * kWidth * w), 2 * oe, yv);
         };
         /* input row i: its products for the output rows i - 1 (below it in
          * the order of the taps: their last three), i and i + 1, then the
          * epilogue of row i - 1 */
         auto step = [&](int i, f32x4(&above)[NB], f32x4(&at)[NB], f32x4(&below)[NB], const Old& o) {
-            if (!live) return;
             const int y = i - 1;
             const bool done = y >= r0;
             bf16x8 f[3][KC];
@@ -242,15 +273,12 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
                 for (int nb = 0; nb < NB; ++nb) below[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
                 taps(0, below);
             }
-            if (!done || !out) return;
-            const size_t p = img + (size_t)uniform(y * W); /* the row's first pixel */
+            const unsigned w = done ? (unsigned)W : 0u;
             if (EPI == EPI_LINEAR) {
-                if (g == 0) {
-                    f32x4 v;
+                f32x4 v;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = above[0][r] + bv[r];
-                    st_row(Yf, p * kOut4, 16u * col, v);
-                }
+                for (int r = 0; r < 4; ++r) v[r] = above[0][r] + bv[r];
+                put(y, w, zero8, 0, v, v);
                 return;
             }
             bf16x8 yv;
@@ -265,37 +293,49 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
                     /* the rounded value is positive (the smallest bf16 is 2^-133) */
                     bits |= v > 0x1p-134f ? 1u << q : 0u;
                 }
-                st_row(Y, p * kWidth, 2 * oe, yv);
-                if (gate) st_row(gate, p * 8, oe >> 3, (unsigned char)bits);
+                put(y, w, yv, bits, above[0], above[NB - 1]);
             } else {
                 f32x4 d0 = above[0], d1 = above[NB - 1];
                 if (EPI == EPI_BWD_ADD) { d0 = o.a + d0; d1 = o.b + d1; }
-                if (store_f) {
-                    st_row(Yf, p * kWidth, 4 * oe, d0);
-                    st_row(Yf, p * kWidth, 4 * oe + 16, d1);
-                }
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
                     yv[q] = (o.gate >> q) & 1 ? (bf16)(q < 4 ? d0[q & 3] : d1[q & 3]) : (bf16)0.f;
-                st_row(Y, p * kWidth, 2 * oe, yv);
+                put(y, w, yv, 0, d0, d1);
             }
         };
         f32x4 a0[NB], a1[NB], a2[NB];
         Piece p0, p1, p2;
         Old o0, o1, o2;
         int i = r0 - 1;
+        /* the loads of the first rows with a step's other operations between
+         * them (on no bytes), so that the loop is entered with the same
+         * operations in flight that it leaves */
+        auto idle = [&](Old& o) {
+            load_old(-1, o);
+            put(0, 0u, zero8, 0, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f});
+        };
         load(i, p0);
+        __builtin_amdgcn_sched_barrier(0);
         load(i + 1, p1);
+        __builtin_amdgcn_sched_barrier(0);
+        idle(o1);
+        __builtin_amdgcn_sched_barrier(0);
         load(i + 2, p2);
+        __builtin_amdgcn_sched_barrier(0);
+        idle(o2);
         __syncthreads(); /* the item before has read its last rows */
         store(i, p0);
+        __builtin_amdgcn_sched_barrier(0);
         load(i + 3, p0);
+        __builtin_amdgcn_sched_barrier(0);
+        idle(o0);
         __syncthreads();
         /* three steps a round: accumulators, pieces and old values change
          * roles without moving.  Step i: row i + 1 to LDS, row i + 4 on its way */
         auto round = [&](f32x4(&above)[NB], f32x4(&at)[NB], f32x4(&below)[NB], Piece& pc, const Old& o, Old& on) {
-            if (i < r1) store(i + 1, pc);
-            if (i + 4 <= r1) load(i + 4, pc);
+            store(i + 1, pc);
+            load(i + 4, pc);
+            if (EPI != EPI_BWD_ADD) __builtin_amdgcn_sched_barrier(0);
             load_old(i, on);
             step(i, above, at, below, o);
             __syncthreads();
@@ -372,52 +412,61 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
         const int w0 = (k % it.cols) * 64, t = k / it.cols;
         const int r0 = (t % it.rows) * it.R, r1 = r0 + it.R < H ? r0 + it.R : H;
         const size_t img = (size_t)(t / it.rows) * H * W;
-        bf16x8 zr[NZ], xr[NX];
-        auto ld_z = [&](int h) {
-#pragma unroll
-            for (int q = 0; q < NZ; ++q) {
-                const int e = threadIdx.x + 256 * q, c = w0 + e / (CZ / 8);
-                zr[q] = zero8;
-                if (e < QZ && c < W) zr[q] = *(const bf16x8*)(dZ + (img + (size_t)h * W + c) * CZ + e % (CZ / 8) * 8);
-            }
+        /* row h of dZ and row h + 1 of X, as each thread carries them */
+        struct Rows {
+            bf16x8 z[NZ], x[NX];
         };
-        auto st_z = [&](int h) {
-#pragma unroll
-            for (int q = 0; q < NZ; ++q) {
-                const int e = threadIdx.x + 256 * q;
-                if (e < QZ) *(bf16x8*)(sZ[h & 1] + e / (CZ / 8) * SZ + e % (CZ / 8) * 8) = zr[q];
-            }
-        };
-        auto ld_x = [&](int h) {
-#pragma unroll
-            for (int q = 0; q < NX; ++q) {
-                const int e = threadIdx.x + 256 * q, c = w0 - 1 + e / (CX / 8);
-                xr[q] = zero8;
-                if (e < QX && c >= 0 && c < W && h >= 0 && h < H)
-                    xr[q] = *(const bf16x8*)(X + (img + (size_t)h * W + c) * CX + e % (CX / 8) * 8);
-            }
-        };
-        auto st_x = [&](int h) {
+        auto row_at = [&](int y, int E) -> size_t { return (img + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E; };
+        auto ld_x = [&](int h, bool on, bf16x8(&x)[NX]) {
+            const auto b = row_buffer(X, row_at(h, 2 * CX), on && h >= 0 && h < H ? 2u * CX * (unsigned)W : 0u);
 #pragma unroll
             for (int q = 0; q < NX; ++q) {
                 const int e = threadIdx.x + 256 * q;
-                if (e < QX) *(bf16x8*)(sX[h & 3] + e / (CX / 8) * SX + e % (CX / 8) * 8) = xr[q];
+                x[q] = buf_ld16<bf16x8>(b, e < QX ? 2u * (unsigned)((w0 - 1 + e / (CX / 8)) * CX + e % (CX / 8) * 8) : ~0u);
             }
         };
-        __syncthreads(); /* the item before has read its last rows */
-        for (int h = r0 - 1; h <= r0 + 1; ++h) {
-            ld_x(h);
-            st_x(h);
+        auto ld = [&](int h, Rows& r) {
+            const auto b = row_buffer(dZ, row_at(h, 2 * CZ), h < r1 ? 2u * CZ * (unsigned)W : 0u);
+#pragma unroll
+            for (int q = 0; q < NZ; ++q) {
+                const int e = threadIdx.x + 256 * q;
+                r.z[q] = buf_ld16<bf16x8>(b, e < QZ ? 2u * (unsigned)((w0 + e / (CZ / 8)) * CZ + e % (CZ / 8) * 8) : ~0u);
+            }
+            ld_x(h + 1, h < r1, r.x);
+        };
+        auto st_x = [&](int h, const bf16x8(&x)[NX]) {
+#pragma unroll
+            for (int q = 0; q < NX; ++q) {
+                const int e = threadIdx.x + 256 * q;
+                if (e < QX) *(bf16x8*)(sX[h & 3] + e / (CX / 8) * SX + e % (CX / 8) * 8) = x[q];
+            }
+        };
+        auto st = [&](int h, const Rows& r) {
+#pragma unroll
+            for (int q = 0; q < NZ; ++q) {
+                const int e = threadIdx.x + 256 * q;
+                if (e < QZ) *(bf16x8*)(sZ[h & 1] + e / (CZ / 8) * SZ + e % (CZ / 8) * 8) = r.z[q];
+            }
+            st_x(h + 1, r.x);
+        };
+        Rows ra, rb;
+        {
+            bf16x8 x0[NX], x1[NX];
+            ld_x(r0 - 1, true, x0);
+            ld_x(r0, true, x1);
+            ld(r0, ra);
+            ld(r0 + 1, rb);
+            __syncthreads(); /* the item before has read its last rows */
+            st_x(r0 - 1, x0);
+            st_x(r0, x1);
+            st(r0, ra);
         }
-        ld_z(r0);
-        st_z(r0);
         __syncthreads();
-        for (int h = r0; h < r1; ++h) {
-            const bool more = h + 1 < r1;
-            if (more) {
-                ld_x(h + 2);
-                ld_z(h + 1);
-            }
+        /* row h's products; row h + 1 to LDS, loaded two rows of products
+         * ago, row h + 2 on its way */
+        auto row = [&](int h, Rows& next, Rows& after) {
+            ld(h + 2, after);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int kc = 0; kc < 2; ++kc) {
                 bf16x8 af[MW];
@@ -439,11 +488,13 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
                     accb = mfma(af[0], ones, accb);
                 }
             }
-            if (more) {
-                st_x(h + 2);
-                st_z(h + 1);
-            }
+            st(h + 1, next);
             __syncthreads();
+        };
+#pragma unroll 1
+        for (int h = r0; h < r1; h += 2) {
+            row(h, rb, ra);
+            if (h + 1 < r1) row(h + 1, ra, rb);
         }
     }
     const int ci = nb0 * 16 + (l & 15), c4 = 4 * (l >> 4);
