@@ -373,16 +373,21 @@ __device__ __forceinline__ bf16x8 ld_tr(const bf16* p)
  * db[co] += sum of dZ[p][co].  MB, NBI: 16-channel blocks of dZ and of X (1
  * where 8 channels are stored).
  *
- * Bound: the matrix cores, then LDS.  A workgroup walks down 64 columns: each
- * row of dZ and of X comes to LDS once (the X rows in a ring of four, the next
- * row's loads behind this row's products, one barrier a row) and is read from
- * there transposed.  A wave takes 16 input channels, all output channels and
+ * Bound: the matrix cores, then LDS.  Each half of a workgroup walks down 64
+ * columns: each row of dZ and of X comes to LDS once (the X rows in a ring of
+ * four, loaded two rows ahead, one barrier a row) and is read from there
+ * transposed.  A wave takes 16 input channels, all output channels and
  * all taps: 13 operands for 36 MFMAs, 0.7 of the LDS rate.  Pixels are 160
  * bytes apart, so that the four rows of a transposing read lie in different
  * banks.  The bias gradient is one more product, with ones.  Sums stay in
- * registers until the workgroup has no rows left. */
+ * registers until the workgroup has no rows left; then the halves' meet in
+ * LDS, since the additions to the shared gradient are 0.09 us for every
+ * workgroup, whatever its work.  64 -> 64 layer, two images of 983 x 1051:
+ * 232 us with a workgroup per four waves and rows one ahead, 192 now; half
+ * the LDS reads (32 columns, rows of dZ kept in registers) made no
+ * difference. */
 template <int MB, int NBI>
-__global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ,
+__global__ void __launch_bounds__(512, 2) k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ,
                                                   ConvItems it, float* __restrict__ dw, float* __restrict__ db)
 {
     constexpr int SZ = MB == 4 ? 80 : 16, SX = NBI == 4 ? 80 : 16;
@@ -391,16 +396,26 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
     constexpr int QZ = 64 * CZ / 8, QX = 66 * CX / 8;                        /* 16-byte pieces of a row */
     constexpr int NZ = (QZ + 255) / 256, NX = (QX + 255) / 256;
     constexpr int MW = NBI == 4 ? MB : 1;                                    /* dZ blocks of a wave */
-    __shared__ __attribute__((aligned(16))) bf16 sZ[2][64 * SZ];
-    __shared__ __attribute__((aligned(16))) bf16 sX[4][66 * SX];
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    constexpr int NA = 9 * MW + 1;                                           /* sums of a lane, by four */
+    struct Half {
+        bf16 z[2][64 * SZ], x[4][66 * SX];
+    };
+    union Lds {
+        Half half[2];
+        f32x4 sum[NA][256];
+    };
+    __shared__ __attribute__((aligned(16))) Lds lds;
+    const int half = uniform(threadIdx.x >> 8), tid = threadIdx.x & 255;
+    const int wv = uniform(tid >> 6), l = threadIdx.x & 63;
+    auto& sZ = lds.half[half].z;
+    auto& sX = lds.half[half].x;
     const int H = it.H, W = it.W;
     const bf16x8 zero8 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
     const bf16x8 ones = bf16x8{1, 1, 1, 1, 1, 1, 1, 1};
     if (MB == 1)
-        for (int q = threadIdx.x; q < 128; q += 256) *(bf16x8*)(sZ[q >> 6] + (q & 63) * SZ + 8) = zero8;
+        for (int q = tid; q < 128; q += 256) *(bf16x8*)(sZ[q >> 6] + (q & 63) * SZ + 8) = zero8;
     if (NBI == 1)
-        for (int q = threadIdx.x; q < 4 * 66; q += 256) *(bf16x8*)(sX[q / 66] + (q % 66) * SX + 8) = zero8;
+        for (int q = tid; q < 4 * 66; q += 256) *(bf16x8*)(sX[q / 66] + (q % 66) * SX + 8) = zero8;
     f32x4 acc[9][MW], accb = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 9; ++t)
@@ -408,10 +423,14 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
         for (int m = 0; m < MW; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int mb0 = NBI == 4 ? 0 : wv, nb0 = NBI == 4 ? wv : 0; /* the wave's first blocks */
     const int px = 8 * (l >> 4) + ((l & 15) >> 2), ch = 4 * (l & 3);
-    for (int k = blockIdx.x; k < it.total; k += gridDim.x) {
-        const int w0 = (k % it.cols) * 64, t = k / it.cols;
-        const int r0 = (t % it.rows) * it.R, r1 = r0 + it.R < H ? r0 + it.R : H;
-        const size_t img = (size_t)(t / it.rows) * H * W;
+    for (int k2 = 2 * blockIdx.x; k2 < it.total; k2 += 2 * gridDim.x) {
+        /* an item for each half; they share the barriers, so both walk R
+         * rows (those past an item's end, or of no item, are zeros) */
+        const int k = k2 + half < it.total ? k2 + half : it.total - 1;
+        const int w0 = uniform((k % it.cols) * 64), t = k / it.cols;
+        const int r0 = uniform((t % it.rows) * it.R);
+        const int r1 = uniform(k != k2 + half ? r0 : (r0 + it.R < H ? r0 + it.R : H));
+        const size_t img = (size_t)uniform(t / it.rows) * H * W;
         /* row h of dZ and row h + 1 of X, as each thread carries them */
         struct Rows {
             bf16x8 z[NZ], x[NX];
@@ -421,7 +440,7 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
             const auto b = row_buffer(X, row_at(h, 2 * CX), on && h >= 0 && h < H ? 2u * CX * (unsigned)W : 0u);
 #pragma unroll
             for (int q = 0; q < NX; ++q) {
-                const int e = threadIdx.x + 256 * q;
+                const int e = tid + 256 * q;
                 x[q] = buf_ld16<bf16x8>(b, e < QX ? 2u * (unsigned)((w0 - 1 + e / (CX / 8)) * CX + e % (CX / 8) * 8) : ~0u);
             }
         };
@@ -429,7 +448,7 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
             const auto b = row_buffer(dZ, row_at(h, 2 * CZ), h < r1 ? 2u * CZ * (unsigned)W : 0u);
 #pragma unroll
             for (int q = 0; q < NZ; ++q) {
-                const int e = threadIdx.x + 256 * q;
+                const int e = tid + 256 * q;
                 r.z[q] = buf_ld16<bf16x8>(b, e < QZ ? 2u * (unsigned)((w0 + e / (CZ / 8)) * CZ + e % (CZ / 8) * 8) : ~0u);
             }
             ld_x(h + 1, h < r1, r.x);
@@ -437,14 +456,14 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
         auto st_x = [&](int h, const bf16x8(&x)[NX]) {
 #pragma unroll
             for (int q = 0; q < NX; ++q) {
-                const int e = threadIdx.x + 256 * q;
+                const int e = tid + 256 * q;
                 if (e < QX) *(bf16x8*)(sX[h & 3] + e / (CX / 8) * SX + e % (CX / 8) * 8) = x[q];
             }
         };
         auto st = [&](int h, const Rows& r) {
 #pragma unroll
             for (int q = 0; q < NZ; ++q) {
-                const int e = threadIdx.x + 256 * q;
+                const int e = tid + 256 * q;
                 if (e < QZ) *(bf16x8*)(sZ[h & 1] + e / (CZ / 8) * SZ + e % (CZ / 8) * 8) = r.z[q];
             }
             st_x(h + 1, r.x);
@@ -452,8 +471,8 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
         Rows ra, rb;
         {
             bf16x8 x0[NX], x1[NX];
-            ld_x(r0 - 1, true, x0);
-            ld_x(r0, true, x1);
+            ld_x(r0 - 1, r0 < r1, x0);
+            ld_x(r0, r0 < r1, x1);
             ld(r0, ra);
             ld(r0 + 1, rb);
             __syncthreads(); /* the item before has read its last rows */
@@ -492,11 +511,26 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(const bf16* __restrict__ X, co
             __syncthreads();
         };
 #pragma unroll 1
-        for (int h = r0; h < r1; h += 2) {
+        for (int h = r0; h < r0 + it.R; h += 2) {
             row(h, rb, ra);
-            if (h + 1 < r1) row(h + 1, ra, rb);
+            if (h + 1 < r0 + it.R) row(h + 1, ra, rb);
         }
     }
+    /* the halves' sums meet in LDS */
+    if (half == 1) {
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+            for (int m = 0; m < MW; ++m) lds.sum[tap * MW + m][tid] = acc[tap][m];
+        lds.sum[NA - 1][tid] = accb;
+    }
+    __syncthreads();
+    if (half == 1) return;
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+        for (int m = 0; m < MW; ++m) acc[tap][m] += lds.sum[tap * MW + m][tid];
+    accb += lds.sum[NA - 1][tid];
     const int ci = nb0 * 16 + (l & 15), c4 = 4 * (l >> 4);
 #pragma unroll
     for (int tap = 0; tap < 9; ++tap)
@@ -827,8 +861,9 @@ static int refresh_layer(hd_cnn* n, int l)
 }
 
 /* Rows per item such that the items fill the 512 resident workgroups (two on
- * each CU) in whole rounds, weighing the rows an item reads beyond its own. */
-static ConvItems conv_items(const hd_cnn* n, int nimg, int width)
+ * each CU) in whole rounds, weighing the rows an item reads beyond its own
+ * and, in rows' time, what each workgroup adds at its end (k_wgrad). */
+static ConvItems conv_items(const hd_cnn* n, int nimg, int width, double add = 0)
 {
     ConvItems c{};
     c.H = n->H;
@@ -838,7 +873,7 @@ static ConvItems conv_items(const hd_cnn* n, int nimg, int width)
     for (int R = 4; R <= 64; ++R) {
         const int rows = (n->H + R - 1) / R;
         const long items = (long)nimg * rows * c.cols;
-        const double cost = (double)((items + 511) / 512) * (R + 1.5);
+        const double cost = (double)((items + 511) / 512) * (R + 1.5) + add * (items < 512 ? items : 512);
         if (c.R == 0 || cost < best) {
             best = cost;
             c.R = R;
@@ -867,9 +902,9 @@ static void conv(hd_cnn* n, const bf16* X, const Layer& y, bool transposed, int 
 template <int MB, int NBI>
 static void wgrad(hd_cnn* n, const bf16* X, const bf16* dZ, const Layer& y, int nimg)
 {
-    const ConvItems it = conv_items(n, nimg, 64);
-    hipLaunchKernelGGL((k_wgrad<MB, NBI>), dim3(it.total < 512 ? it.total : 512), dim3(256), 0, n->stream, X, dZ, it,
-                       y.dw, y.db);
+    const ConvItems it = conv_items(n, nimg, 64, 0.017);
+    hipLaunchKernelGGL((k_wgrad<MB, NBI>), dim3(it.total < 512 ? (it.total + 1) / 2 : 256), dim3(512), 0, n->stream, X,
+                       dZ, it, y.dw, y.db);
 }
 
 /* gates: whether a backward pass may follow */
