@@ -1123,6 +1123,10 @@ int hd_cnn_get_grad(hd_cnn* n, int l, float* host_dw, float* host_db)
     if (!n || l < 0 || l >= n->L) return HD_EINVAL;
     const Layer& y = n->layer[l];
     CHK(n, hipStreamSynchronize(n->stream));
+    if (host_dw && host_db == host_dw + y.nw() && y.db == y.dw + y.nw()) { /* adjacent on both sides: one copy */
+        CHK(n, hipMemcpy(host_dw, y.dw, (y.nw() + y.cout) * 4, hipMemcpyDeviceToHost));
+        return HD_OK;
+    }
     if (host_dw) CHK(n, hipMemcpy(host_dw, y.dw, y.nw() * 4, hipMemcpyDeviceToHost));
     if (host_db) CHK(n, hipMemcpy(host_db, y.db, (size_t)y.cout * 4, hipMemcpyDeviceToHost));
     return HD_OK;

@@ -133,8 +133,11 @@ class Network:
 
     def get_grad(self, l):
         ci, co = self.dims(l)
-        w = np.zeros((9, co, ci), np.float32)
-        b = np.zeros(co, np.float32)
+        # one buffer, so that one copy fills both; not zeroed first: a fresh
+        # zeroed one is unmapped pages that the copy then waits for (226 us
+        # per 64 -> 64 layer, against 20)
+        g = np.empty(9 * co * ci + co, np.float32)
+        w, b = g[:9 * co * ci].reshape(9, co, ci), g[9 * co * ci:]
         self._chk(lib().hd_cnn_get_grad(self.h, l, _f32(w)[1], _f32(b)[1]))
         return w, b
 
@@ -151,7 +154,7 @@ class Network:
 
     def forward(self):
         """Prediction of the loaded batch, [b,H,W,3] (normalised u, v, z)."""
-        out = np.zeros((self._n, self.H, self.W, 3), np.float32)
+        out = np.empty((self._n, self.H, self.W, 3), np.float32)
         self._chk(lib().hd_cnn_forward(self.h, out.ctypes.data_as(ctypes.POINTER(ctypes.c_float))))
         return out
 
