@@ -2144,11 +2144,13 @@ struct EdgeVals {
  * their own.  The old values of positions 2 and 3 are used only where no
  * other thread writes those positions. */
 template <bool ROWS>
-__device__ __forceinline__ EdgeVals edge_vals(const HdDevG& d, int line, int x)
+__device__ __forceinline__ EdgeVals edge_vals(const HdDevG& d, int line, int x, bool wx, bool wn, bool wl2, bool wl1)
 {
     EdgeVals e{0.0, 0.0, 0.0, 0.0};
     const int W = d.W, L = ROWS ? d.M : d.N;
     if (line < 2 || line > (ROWS ? d.N : d.M)) return e;
+    /* only where a run starts at 2 or ends at L, else margin_at does not look */
+    if (!(x == 1 ? wn && !wx && 2 <= L - 2 : wx && !wn && wl1 && wl2)) return e;
     auto at = [&](int k) { return ROWS ? line * W + k : k * W + line; };
     auto ex_at = [&](int k) -> double { return ROWS ? explicit_v_at(d, line, k) : explicit_u_at(d, k, line); };
     if (x == 1) {
@@ -2304,7 +2306,7 @@ __global__ void __launch_bounds__(256) k_smooth_u_explicit_v(const HdDev* __rest
         r.t3 = smooth_u_at(d, i, j + 1);
         vn = v_solver_ev(d.P, r);
     }
-    const EdgeVals ev = in ? EdgeVals{0.0, 0.0, 0.0, 0.0} : edge_vals<true>(d, i, j);
+    const EdgeVals ev = in ? EdgeVals{0.0, 0.0, 0.0, 0.0} : edge_vals<true>(d, i, j, wx, wn, wl2, wl1);
     d.tmp_u[p] = sm;
     if (in) d.t_v[p] = vn;
     dry_store(d, i, j, 1, dm);
@@ -2359,7 +2361,7 @@ __global__ void __launch_bounds__(256) k_smooth_v_explicit_u(const HdDev* __rest
         r.t3 = smooth_v_at(d, i + 1, j);
         un = u_solver_ev(d.P, r);
     }
-    const EdgeVals ev = in ? EdgeVals{0.0, 0.0, 0.0, 0.0} : edge_vals<false>(d, j, i);
+    const EdgeVals ev = in ? EdgeVals{0.0, 0.0, 0.0, 0.0} : edge_vals<false>(d, j, i, wx, wn, wl2, wl1);
     d.tmp_v[p] = sm;
     if (in) d.t_u[p] = un;
     dry_store(d, i, j, 0, dm);
