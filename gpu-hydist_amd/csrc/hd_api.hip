@@ -602,9 +602,9 @@ static int check_series(hd_ctx* c, double t, const hd_step_opts& o)
  * VZ), enqueued on the stream for every context of the batch.  The boundary
  * values of the half-step (Update_Boundary_Value) and the device time step:
  * in the default form with the boundary series (not the analytic channel
- * tide, not the narrow-channel index shifts), the sweep's runs that own the
- * edge cells write the values and the explicit pass after it advances the
- * time; otherwise a k_boundary launch does both.  Returns in *slo / *eoff
+ * tide), the sweep's runs that own the edge cells write the values and the
+ * explicit pass after it advances the time; otherwise a k_boundary launch
+ * (4 us and a gap) does both.  Returns in *slo / *eoff
  * the row range of a following bed change (rows slo .. N - eoff - 1). */
 static void enqueue_half(Exec& x, int which, const hd_step_opts& o, bool sediment, int count_wet, int ntiles,
                          int sed_ntiles, int* slo_out, int* eoff_out)
@@ -612,7 +612,7 @@ static void enqueue_half(Exec& x, int which, const hd_step_opts& o, bool sedimen
     hipStream_t s = x.stream;
     bool channel = o.kenhhepd || o.kenhhepng;
     int an = analytic_mode(o) ? 1 : 0;
-    const int own = (x.solver == 0 && !an && !channel) ? 1 : 0;
+    const int own = (x.solver == 0 && !an) ? 1 : 0;
     if (!own) launch(x, "boundary", [&] { hd_launch_boundary_t(x.b(), an, s); });
     int slo = 2, eoff = 0;
     if (which == 0) {

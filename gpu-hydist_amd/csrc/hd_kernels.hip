@@ -1441,7 +1441,10 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
         const int4 rn = runs[ri];
         const int line = __builtin_amdgcn_readfirstlane(rn.x), first = __builtin_amdgcn_readfirstlane(rn.y),
                   last = __builtin_amdgcn_readfirstlane(rn.z);
-        if (line < sidx || line > eidx) continue;
+        /* a line that the narrow-channel shift leaves out has its boundary
+         * cells written all the same */
+        const bool left_out = line < sidx || line > eidx;
+        if (left_out && !bnd) continue;
         auto at = [&](int k) -> size_t { return isU ? (size_t)k * W + line : (size_t)line * W + k; };
         /* one round of loads: wall-flag depths (locate_segment_u / _v,
          * constant.cuh:135-178), boundary depths, edge values, first cells */
@@ -1456,6 +1459,7 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
         /* this run's boundary cells, before its end values are read (one
          * wave: its own stores are seen by its later loads) */
         if (bnd) run_boundary<isU>(d, line, first, last, lane);
+        if (left_out) continue;
         const double TZ_l = tz[at(first)];
         const double TZ_r = tz[at(last)];
         const double ub1 = isU ? d.ubt[line] : d.vbd[line];
