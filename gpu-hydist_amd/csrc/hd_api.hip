@@ -607,7 +607,7 @@ static int check_series(hd_ctx* c, double t, const hd_step_opts& o)
  * (4 us and a gap) does both.  Returns in *slo / *eoff
  * the row range of a following bed change (rows slo .. N - eoff - 1). */
 static void enqueue_half(Exec& x, int which, const hd_step_opts& o, bool sediment, int count_wet, int ntiles,
-                         int sed_ntiles, int* slo_out, int* eoff_out)
+                         int sed_ntiles, bool fs_later, int* slo_out, int* eoff_out)
 {
     hipStream_t s = x.stream;
     bool channel = o.kenhhepd || o.kenhhepng;
@@ -710,25 +710,30 @@ static void enqueue_half(Exec& x, int which, const hd_step_opts& o, bool sedimen
                                  which == 0 ? x.run_blocks_u : x.run_blocks_v, x.solver == 0, s);
             });
         }
-        launch(x, "update_fs", [&] { hd_launch_update_fs(x.b(), sed_ntiles, s); });
+        if (!fs_later) launch(x, "update_fs", [&] { hd_launch_update_fs(x.b(), sed_ntiles, s); });
         if (which == 1) { slo = 3; eoff = 1; }
     }
     if (slo_out) *slo_out = slo;
     if (eoff_out) *eoff_out = eoff;
 }
 
-static void enqueue_bed(Exec& x, const hd_step_opts& o, int slo, int eoff, int bed_ntiles)
+/* update: with the FS update that the half-step before left to it */
+static void enqueue_bed(Exec& x, const hd_step_opts& o, int slo, int eoff, int bed_ntiles, bool update)
 {
-    launch(x, "calc_qb", [&] { hd_launch_calc_qb(x.b(), o.qb_mode, bed_ntiles, x.stream); });
+    launch(x, "calc_qb", [&] { hd_launch_calc_qb(x.b(), o.qb_mode, bed_ntiles, update, x.stream); });
     launch(x, "bedload", [&] { hd_launch_bedload(x.b(), o.ketdinh, slo, eoff, bed_ntiles, x.stream); });
 }
+
+/* The second half-step's FS update goes with the bed-load flux when both run
+ * over the active tiles. */
+static bool update_in_bed(const GraphKey& k) { return k.sed1 && k.bed && k.sed_ntiles > 0 && k.bed_ntiles > 0; }
 
 static void enqueue_step(Exec& x, const hd_step_opts& o, const GraphKey& k)
 {
     int slo = 2, eoff = 0;
-    enqueue_half(x, 0, o, k.sed0, 0, k.ntiles, k.sed_ntiles, nullptr, nullptr);
-    enqueue_half(x, 1, o, k.sed1, k.count, k.ntiles, k.sed_ntiles, &slo, &eoff);
-    if (k.bed) enqueue_bed(x, o, slo, eoff, k.bed_ntiles);
+    enqueue_half(x, 0, o, k.sed0, 0, k.ntiles, k.sed_ntiles, false, nullptr, nullptr);
+    enqueue_half(x, 1, o, k.sed1, k.count, k.ntiles, k.sed_ntiles, update_in_bed(k), &slo, &eoff);
+    if (k.bed) enqueue_bed(x, o, slo, eoff, k.bed_ntiles, update_in_bed(k));
 }
 
 static GraphKey make_key(hd_ctx* c, double t, const hd_step_opts& o, int count)
@@ -786,7 +791,7 @@ int hd_halfstep(hd_ctx* c, int which, double t, const hd_step_opts* o)
     if (rc) return rc;
     Exec x = exec_of(c);
     set_time(x, t - c->P.dT * 0.5);
-    enqueue_half(x, which, *o, t >= o->sediment_start, 0, 0, 0, nullptr, nullptr);
+    enqueue_half(x, which, *o, t >= o->sediment_start, 0, 0, 0, false, nullptr, nullptr);
     HIPCHK(c, hipGetLastError());
     return HD_OK;
 }
@@ -798,7 +803,7 @@ int hd_bed_change(hd_ctx* c, double t, const hd_step_opts* o)
     if ((o->kenhhepd || o->kenhhepng) && o->kenhhepng == 1) slo = 3;
     if (t >= o->sediment_start) { slo = 3; eoff = 1; }
     Exec x = exec_of(c);
-    enqueue_bed(x, *o, slo, eoff, 0);
+    enqueue_bed(x, *o, slo, eoff, 0, false);
     HIPCHK(c, hipGetLastError());
     return HD_OK;
 }
@@ -865,11 +870,12 @@ static void enqueue_sed_step(Exec& x, const hd_step_opts& o, const GraphKey& k)
                 hd_launch_fs_run(x.b(), which, o.bed_change_start, o.ketdinh,
                                  which == 0 ? x.run_blocks_u : x.run_blocks_v, x.solver == 0, x.stream);
             });
-            launch(x, "update_fs", [&] { hd_launch_update_fs(x.b(), k.sed_ntiles, x.stream); });
+            if (which == 0 || !update_in_bed(k))
+                launch(x, "update_fs", [&] { hd_launch_update_fs(x.b(), k.sed_ntiles, x.stream); });
             if (which == 1) { slo = 3; eoff = 1; }
         }
     }
-    if (k.bed) enqueue_bed(x, o, slo, eoff, k.bed_ntiles);
+    if (k.bed) enqueue_bed(x, o, slo, eoff, k.bed_ntiles, update_in_bed(k));
 }
 
 static int run_impl(hd_ctx* c, double t, int nsteps, const hd_step_opts* o, double* t_out, int count)
@@ -1658,7 +1664,7 @@ int hd_k_Scan_FSi(hd_ctx* c, double t, double s_start, int ketdinh, double* AA, 
 int hd_k_Calculate_Qb(hd_ctx* c, int qb_mode)
 {
     Exec x; int rc = unit_begin(c, x); if (rc) return rc;
-    hd_launch_calc_qb(x.b(), qb_mode, 0, x.stream);
+    hd_launch_calc_qb(x.b(), qb_mode, 0, 0, x.stream);
     return unit_end(c, false);
 }
 

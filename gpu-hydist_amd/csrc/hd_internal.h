@@ -198,7 +198,8 @@ void hd_launch_fs_line(const HdBatch& b, int which, double s_start, int ketdinh,
 void hd_launch_fs_run(const HdBatch& b, int which, double s_start, int ketdinh, int nblocks, int spec,
                       hipStream_t s);
 void hd_launch_update_fs(const HdBatch& b, int ntiles, hipStream_t s);
-void hd_launch_calc_qb(const HdBatch& b, int qb_mode, int ntiles, hipStream_t s);
+/* update (tiles only): Update_FS of the half-step before in the same launch */
+void hd_launch_calc_qb(const HdBatch& b, int qb_mode, int ntiles, int update, hipStream_t s);
 void hd_launch_bedload(const HdBatch& b, int ketdinh, int slo, int eoff, int ntiles, hipStream_t s);
 void hd_launch_wet_count(const HdBatch& b, hipStream_t s);
 void hd_launch_flow_refresh(const HdBatch& b, hipStream_t s);
