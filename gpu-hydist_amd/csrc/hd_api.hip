@@ -120,8 +120,8 @@ struct hd_ctx {
     double* z_snap = nullptr;   /* z snapshot for hd_z_change (allocated on first use), + 5 result slots */
     int ntiles = 0;             /* active row tiles (computed at init / prepare) */
     bool settled = false;       /* a full step has run since init / upload: land tiles are at a fixed point */
-    bool sed_settled = false;   /* ... and a sediment sweep over the whole grid (VTH, hesoK, FS = tFS) */
-    bool bed_settled = false;   /* ... and a bed-load flux over the whole grid */
+    bool sed_settled = false;   /* a sediment sweep over the whole grid (VTH, hesoK, FS = tFS) on the flow as it is there */
+    bool bed_settled = false;   /* and a bed-load flux */
     int rb_mult = 2;            /* solver blocks per line (autotuned) */
     int bw = 256;               /* block width of the per-row full-grid kernels (autotuned) */
     Prof prof;
@@ -736,9 +736,14 @@ static void enqueue_step(Exec& x, const hd_step_opts& o, const GraphKey& k)
     if (k.bed) enqueue_bed(x, o, slo, eoff, k.bed_ntiles, update_in_bed(k));
 }
 
-static GraphKey make_key(hd_ctx* c, double t, const hd_step_opts& o, int count)
+/* flow: the step advances the flow.  On a frozen flow (hd_sediment_run) the
+ * sediment kernels' own pass over the whole grid is enough for later ones to
+ * run over the active tiles; a flow step over the whole grid can change the
+ * cells outside them once more. */
+static GraphKey make_key(hd_ctx* c, double t, const hd_step_opts& o, int count, bool flow = true)
 {
     GraphKey k;
+    if (flow && !c->settled) c->sed_settled = c->bed_settled = false;
     double t1 = t + c->P.dT * 0.5;
     double t2 = t1 + c->P.dT * 0.5;
     k.sed0 = t1 >= o.sediment_start;
@@ -752,8 +757,8 @@ static GraphKey make_key(hd_ctx* c, double t, const hd_step_opts& o, int count)
     k.ntiles = c->settled ? c->ntiles : 0;
     /* the first step that runs the sediment sweep (the bed-load flux) does
      * it over the whole grid; later ones over the active tiles */
-    k.sed_ntiles = (c->settled && c->sed_settled) ? c->ntiles : 0;
-    k.bed_ntiles = (c->settled && c->bed_settled) ? c->ntiles : 0;
+    k.sed_ntiles = c->sed_settled ? c->ntiles : 0;
+    k.bed_ntiles = c->bed_settled ? c->ntiles : 0;
     if (k.sed0 || k.sed1) c->sed_settled = true;
     if (k.bed) c->bed_settled = true;
     return k;
@@ -791,6 +796,7 @@ int hd_halfstep(hd_ctx* c, int which, double t, const hd_step_opts* o)
     if (rc) return rc;
     Exec x = exec_of(c);
     set_time(x, t - c->P.dT * 0.5);
+    if (!c->settled) c->sed_settled = c->bed_settled = false;
     enqueue_half(x, which, *o, t >= o->sediment_start, 0, 0, 0, false, nullptr, nullptr);
     HIPCHK(c, hipGetLastError());
     return HD_OK;
@@ -931,7 +937,7 @@ int hd_sediment_run(hd_ctx* c, double t, int nsteps, const hd_step_opts* o, doub
     set_time(x, t);
     std::string why;
     hipError_t e = run_steps(x, c->sed_graphs, t, nsteps, *o, c->P.dT, 0,
-                             [&](double tt) { return make_key(c, tt, *o, 0); }, why, enqueue_sed_step);
+                             [&](double tt) { return make_key(c, tt, *o, 0, false); }, why, enqueue_sed_step);
     if (e != hipSuccess) return fail(c, HD_EHIP, why + ": " + hipGetErrorString(e));
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1365,11 +1371,15 @@ int hd_ensemble_run(hd_ensemble* e, double t, int nsteps, const hd_step_opts* o,
         bed_settled = bed_settled && c->bed_settled;
         maxtiles = std::max(maxtiles, c->ntiles);
     }
+    if (!settled) { /* the first step runs over the whole grid (make_key) */
+        sed_settled = bed_settled = false;
+        for (hd_ctx* c : e->m) c->sed_settled = c->bed_settled = false;
+    }
     auto key = [&](double tt) {
         GraphKey k = make_key(c0, tt, *o, count);
         k.ntiles = settled ? maxtiles : 0;
-        k.sed_ntiles = (settled && sed_settled) ? maxtiles : 0;
-        k.bed_ntiles = (settled && bed_settled) ? maxtiles : 0;
+        k.sed_ntiles = sed_settled ? maxtiles : 0;
+        k.bed_ntiles = bed_settled ? maxtiles : 0;
         if (k.sed0 || k.sed1) {
             sed_settled = true;
             for (hd_ctx* c : e->m) c->sed_settled = true;
@@ -1478,6 +1488,7 @@ static int unit_begin(hd_ctx* c, Exec& x)
     if (c->state() != 0) return fail(c, HD_ESTATE, "per-kernel entry point inside a half-step");
     HIPCHK(c, hipSetDevice(c->device));
     x = exec_of(c);
+    if (!c->settled) c->sed_settled = c->bed_settled = false; /* the kernel may change the flow outside the tiles */
     return HD_OK;
 }
 

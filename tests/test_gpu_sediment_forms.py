@@ -8,6 +8,9 @@ import pytest
 import oracle
 from hydist_amd import synth
 from hydist_amd._lib import Solver
+from hydist_amd.case import BED_EVERY_STEP
+
+from _parity import diff_fields
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +87,43 @@ def test_values(field, ketdinh):
     o.kernel("bed_load", ketdinh, 3, c.N - 1)
     g.kernel("BedLoad", ketdinh, 3, c.N - 1)
     assert bits_differ(o, g, ("Qbx", "Qby", "dH")) == []
+
+
+def test_frozen_flow_runs_over_the_active_tiles():
+    """hd_sediment_run over the active tiles after its first step, against one
+    whole-grid step at a time (an upload of the same mask starts over): on a
+    flow written from outside, and after flow steps without sediment."""
+    c = synth.config(3, scale=0.1)
+    c.sediment_start, c.bed_change_start, c.bed_mode = 0.0, 0.0, BED_EVERY_STEP
+    op, off = c.opts(), c.opts(sediment_start=1e9, bed_change_start=1e9)
+    a = Solver(c)
+    a.init()
+    t = a.run(0.0, 10, op)
+    rng = np.random.default_rng(3)
+    for n in ("u", "v"):
+        a.set(n, a.get(n) + 0.05 * rng.standard_normal(a.get(n).shape))  # land too
+    a.flow_refresh()
+    b = a.clone()
+
+    def single(n):
+        for k in range(n):
+            b.set("khouot", b.get("khouot"))
+            b.sediment_run(t + k * c.dT, 1, op)
+
+    a.sediment_run(t, 5, op)
+    single(5)
+    assert diff_fields(a.get, b.get) == []
+    # a flow step over the whole grid, without sediment, then sediment again
+    for n in ("u", "v"):
+        f = a.get(n) + 0.05 * rng.standard_normal(a.get(n).shape)
+        a.set(n, f)
+        b.set(n, f)
+    a.flow_refresh()
+    b.flow_refresh()
+    a.sediment_run(t, 2, op)
+    single(2)
+    a.run(t, 2, off)
+    b.run(t, 2, off)
+    a.sediment_run(t, 3, op)
+    single(3)
+    assert diff_fields(a.get, b.get) == []
