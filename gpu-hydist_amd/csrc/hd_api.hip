@@ -1026,6 +1026,34 @@ int hd_flow_refresh(hd_ctx* c)
     return HD_OK;
 }
 
+/* dst's state allocations from src's, of the same sizes, on dst's stream: in
+ * one launch for every 64 of them, or a copy command each where the contexts
+ * are on two devices. */
+static hipError_t copy_allocs(hd_ctx* dst, const hd_ctx* src)
+{
+    HdCopies c;
+    c.n = 0;
+    const size_t n = dst->state_allocs.size();
+    for (size_t k = 0; k < n; ++k) {
+        void *to = dst->state_allocs[k].first, *from = src->state_allocs[k].first;
+        const size_t bytes = src->state_allocs[k].second;
+        if (dst->device != src->device || (((uintptr_t)to | (uintptr_t)from) & 15)) {
+            const hipError_t e = hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, dst->stream);
+            if (e != hipSuccess) return e;
+            continue;
+        }
+        c.dst[c.n] = (char*)to;
+        c.src[c.n] = (char*)from;
+        c.bytes[c.n++] = bytes;
+        if (c.n == HdCopies::kMax) {
+            hd_launch_copies(c, dst->stream);
+            c.n = 0;
+        }
+    }
+    hd_launch_copies(c, dst->stream);
+    return hipGetLastError();
+}
+
 int hd_copy_state(hd_ctx* dst, hd_ctx* src)
 {
     if (!dst || !src) return HD_EINVAL;
@@ -1035,12 +1063,10 @@ int hd_copy_state(hd_ctx* dst, hd_ctx* src)
     if (src->state() != 0 || dst->state() != 0) return fail(dst, HD_ESTATE, "hd_copy_state between half-steps");
     HIPCHK(dst, hipSetDevice(dst->device));
     HIPCHK(dst, hipStreamSynchronize(src->stream));
-    for (size_t k = 0; k < dst->state_allocs.size(); ++k) {
+    for (size_t k = 0; k < dst->state_allocs.size(); ++k)
         if (dst->state_allocs[k].second != src->state_allocs[k].second)
             return fail(dst, HD_ESHAPE, "hd_copy_state: layout");
-        HIPCHK(dst, hipMemcpyAsync(dst->state_allocs[k].first, src->state_allocs[k].first, src->state_allocs[k].second,
-                                   hipMemcpyDeviceToDevice, dst->stream));
-    }
+    HIPCHK(dst, copy_allocs(dst, src));
     HIPCHK(dst, hipStreamSynchronize(dst->stream));
     dst->ntiles = src->ntiles;
     dst->settled = src->settled;
@@ -1061,11 +1087,9 @@ int hd_clone(hd_ctx* src, hd_ctx** out)
     hd_ctx* c = *out;
     HIPCHK(src, hipStreamSynchronize(src->stream));
     if (c->state_allocs.size() != src->state_allocs.size()) { hd_destroy(c); return fail(src, HD_EHIP, "layout"); }
-    for (size_t k = 0; k < c->state_allocs.size(); ++k) {
+    for (size_t k = 0; k < c->state_allocs.size(); ++k)
         if (c->state_allocs[k].second != src->state_allocs[k].second) { hd_destroy(c); return fail(src, HD_EHIP, "layout"); }
-        HIPCHK(src, hipMemcpyAsync(c->state_allocs[k].first, src->state_allocs[k].first, src->state_allocs[k].second,
-                                   hipMemcpyDeviceToDevice, c->stream));
-    }
+    HIPCHK(src, copy_allocs(c, src));
     HIPCHK(src, hipStreamSynchronize(c->stream));
     set_knobs(c, src->rb_mult, src->bw);
     c->ntiles = src->ntiles;

@@ -13,8 +13,9 @@
  *    at L * tw + r, tw = 2*len+2, with the elimination factors Ap/Bp beside
  *    them; per-segment continuity coefficients at the two line ends live in
  *    a small side table (SEG_*).
- * Kernels receive HdDev by value (kernel arguments), so a captured HIP graph
- * replays with exactly the pointers of the step it recorded.
+ * Kernels take a pointer to HdDev copies in device memory, one copy per swap
+ * state of the buffers above, so a captured HIP graph replays with exactly the
+ * pointers of the step it recorded.
  */
 #ifndef HD_INTERNAL_H
 #define HD_INTERNAL_H
@@ -203,6 +204,14 @@ void hd_launch_calc_qb(const HdBatch& b, int qb_mode, int ntiles, int update, hi
 void hd_launch_bedload(const HdBatch& b, int ketdinh, int slo, int eoff, int ntiles, hipStream_t s);
 void hd_launch_wet_count(const HdBatch& b, hipStream_t s);
 void hd_launch_flow_refresh(const HdBatch& b, hipStream_t s);
+/* byte copies between device allocations of one device, from their starts */
+struct HdCopies {
+    static constexpr int kMax = 64;
+    int n;
+    char *dst[kMax], *src[kMax]; /* 16-byte aligned */
+    unsigned long long bytes[kMax];
+};
+void hd_launch_copies(const HdCopies& c, hipStream_t s);
 void hd_launch_bed_extrapolate(const HdBatch& b, const double* snap, double f, hipStream_t s);
 void hd_launch_z_change(const HdBatch& b, const double* zref, double bound, double* out, hipStream_t s);
 /* batched Thomas on device arrays; systems outside rows [0, nrows) are skipped */

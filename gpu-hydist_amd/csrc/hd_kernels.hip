@@ -2711,6 +2711,34 @@ __global__ void __launch_bounds__(256) k_flow_refresh(const HdDev* __restrict__ 
     }
 }
 
+/* The copies of a context's state in one launch: blockIdx.y is the allocation,
+ * blockIdx.x 32 KB of it, eight 16-byte loads a thread in flight before the
+ * first store.  Bound: HBM.  hd_copy_state between two 980 x 1048 rivers (350
+ * MB) takes 142 us, 4.9 TB/s; a copy command per allocation, about fifty of
+ * them from 4 bytes to 18 MB one after another, took 284 us. */
+constexpr unsigned kCopyBlock = 32768;
+__global__ void __launch_bounds__(256) k_copies(HdCopies c)
+{
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const int k = blockIdx.y;
+    const size_t at = (size_t)blockIdx.x * kCopyBlock, n = c.bytes[k];
+    if (at >= n) return;
+    HD_GLOBAL_AS char* to = (HD_GLOBAL_AS char*)c.dst[k] + at;
+    HD_GLOBAL_AS const char* from = (HD_GLOBAL_AS const char*)c.src[k] + at;
+    const unsigned t = threadIdx.x * 16;
+    if (n - at >= kCopyBlock) {
+        u4 v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = *(HD_GLOBAL_AS const u4*)(from + t + 4096 * q);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) *(HD_GLOBAL_AS u4*)(to + t + 4096 * q) = v[q];
+        return;
+    }
+    const unsigned rest = (unsigned)(n - at), whole = rest & ~15u;
+    for (unsigned x = t; x < whole; x += 4096) *(HD_GLOBAL_AS u4*)(to + x) = *(HD_GLOBAL_AS const u4*)(from + x);
+    if (threadIdx.x < rest - whole) to[whole + threadIdx.x] = from[whole + threadIdx.x];
+}
+
 /* dH += f * (dH - snap) over the padded grid (bed-change extrapolation) */
 __global__ void __launch_bounds__(256) k_bed_extrapolate(const HdDev* __restrict__ dv, const double* snap, double f)
 {
@@ -3597,6 +3625,14 @@ int hd_thomas_spec_device(int nsys, const int* off, const int* sn, const double*
     if (nsys > 0)
         hipLaunchKernelGGL(k_thomas_spec, dim3(nsys), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap, Bp, nrows);
     return 0;
+}
+
+void hd_launch_copies(const HdCopies& c, hipStream_t s)
+{
+    unsigned long long most = 0;
+    for (int k = 0; k < c.n; ++k) most = c.bytes[k] > most ? c.bytes[k] : most;
+    if (most == 0) return;
+    hipLaunchKernelGGL(k_copies, dim3((unsigned)((most + kCopyBlock - 1) / kCopyBlock), c.n), dim3(256), 0, s, c);
 }
 
 void hd_launch_bed_extrapolate(const HdBatch& b, const double* snap, double f, hipStream_t s)
