@@ -696,7 +696,7 @@ static void enqueue_half(Exec& x, int which, const hd_step_opts& o, bool sedimen
         launch(x, "segments_fs_edges", [&] { hd_launch_segments(x.b(), count_wet, s); });
     }
     if (sediment) {
-        launch(x, "vth_hesok", [&] { hd_launch_vth_hesok(x.b(), sed_ntiles, s); });
+        launch(x, "vth_hesok", [&] { hd_launch_vth_hesok(x.b(), sed_ntiles, 0, s); });
         if (x.solver_v1) {
             launch(x, which == 0 ? "fs_coef_j" : "fs_coef_i",
                    [&] { hd_launch_fs_coef(x.b(), which, o.bed_change_start, o.ketdinh, s); });
@@ -862,16 +862,19 @@ static hipError_t run_steps(Exec& x, std::map<GraphKey, hipGraphExec_t>& graphs,
 
 /* The sediment half of one step on a frozen flow: per half-step the
  * boundary values (device time advanced) and, when the sediment module is on,
- * VTH / hesoK, the FS sweep of that direction and the FS update; then the
+ * VTH / hesoK (over the active tiles with the series' boundary values in the
+ * same launch), the FS sweep of that direction and the FS update; then the
  * bed change when triggered. */
 static void enqueue_sed_step(Exec& x, const hd_step_opts& o, const GraphKey& k)
 {
     int an = analytic_mode(o) ? 1 : 0;
     int slo = 2, eoff = 0;
     for (int which = 0; which < 2; ++which) {
-        launch(x, "boundary", [&] { hd_launch_boundary_t(x.b(), an, x.stream); });
-        if (which == 0 ? k.sed0 : k.sed1) {
-            launch(x, "vth_hesok", [&] { hd_launch_vth_hesok(x.b(), k.sed_ntiles, x.stream); });
+        const bool sed = which == 0 ? k.sed0 : k.sed1;
+        const int bnd = x.solver == 0 && !an && sed && k.sed_ntiles > 0; /* by a workgroup of vth_hesok */
+        if (!bnd) launch(x, "boundary", [&] { hd_launch_boundary_t(x.b(), an, x.stream); });
+        if (sed) {
+            launch(x, "vth_hesok", [&] { hd_launch_vth_hesok(x.b(), k.sed_ntiles, bnd, x.stream); });
             launch(x, which == 0 ? (x.solver == 0 ? "fs_spec_j" : "fs_run_j") : (x.solver == 0 ? "fs_spec_i" : "fs_run_i"), [&] {
                 hd_launch_fs_run(x.b(), which, o.bed_change_start, o.ketdinh,
                                  which == 0 ? x.run_blocks_u : x.run_blocks_v, x.solver == 0, x.stream);
@@ -1655,7 +1658,7 @@ int hd_k_Reset_states(hd_ctx* c, int horizontal, int kenhhepd, int kenhhepng)
 int hd_k_Find_VTH_hesoK(hd_ctx* c)
 {
     Exec x; int rc = unit_begin(c, x); if (rc) return rc;
-    hd_launch_vth_hesok(x.b(), 0, x.stream);
+    hd_launch_vth_hesok(x.b(), 0, 0, x.stream);
     return unit_end(c, false);
 }
 

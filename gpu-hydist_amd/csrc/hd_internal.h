@@ -192,7 +192,8 @@ void hd_launch_smooth_u_explicit_v(const HdBatch& b, int bw, int ntiles, int adv
 void hd_launch_wetting(const HdBatch& b, int horizontal, int mode, hipStream_t s);
 void hd_launch_smooth_wet(const HdBatch& b, int isU, int horizontal, int ntiles, int mode, hipStream_t s);
 void hd_launch_uvz_dry(const HdBatch& b, int kd, int kn, int bw, int ntiles, hipStream_t s);
-void hd_launch_vth_hesok(const HdBatch& b, int ntiles, hipStream_t s);
+/* bnd (1, tiles only): the half-step's series boundary values in the same launch */
+void hd_launch_vth_hesok(const HdBatch& b, int ntiles, int bnd, hipStream_t s);
 void hd_launch_fs_coef(const HdBatch& b, int which, double s_start, int ketdinh, hipStream_t s);
 void hd_launch_fs_solve(const HdBatch& b, int which, hipStream_t s);
 void hd_launch_fs_line(const HdBatch& b, int which, double s_start, int ketdinh, hipStream_t s);
