@@ -107,9 +107,8 @@ struct ConvItems {
  * LDS reads; pixels are 144 bytes apart there, free of bank conflicts.
  * Staging each tap's weights in LDS instead, for 4 x 64 tiles, needed an LDS
  * read of half its time for every MFMA: 224 us per 64 -> 64 layer at 983 x
- * 1051, against 107 now
- * (dZ and dA of the data gradient: 242 + 158 for the ReLU pass, against 190,
- * 4.2 TB/s).
+ * 1051, against 80 now (dZ and dA of the data gradient: 242 + 158 for the
+ * ReLU pass, against 151, 5.3 TB/s).
  *
  * Workgroups stay for as many items as there are; a wave's three
  * accumulators are the output rows above, at and below the input row at

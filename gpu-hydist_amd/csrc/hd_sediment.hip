@@ -141,8 +141,7 @@ __device__ __forceinline__ double fs_source(const HdDevG& d, const FsConst& K, i
  * bnd (with tiles): the launch has one workgroup more, the first, which
  * writes the half-step's boundary values, a wave an edge, as k_boundary does;
  * nothing here reads those.  A step on a frozen flow, bed change included, same
- * grid: 69.8 us
- * with two k_boundary launches, 64.1 without. */
+ * grid: 69.8 us with two k_boundary launches, 64.1 without. */
 __global__ void __launch_bounds__(256) k_vth_hesok(const HdDev* __restrict__ dv, int tiled, int bnd)
 {
     const HdDevG& d = dev_view(dv);

@@ -12,11 +12,12 @@
  * the plain FP64 step checks it periodically (hydist_amd.surrogate).
  *
  * Layout: images are NHWC on the case's padded grid, H = N+3 rows, W = M+3
- * columns.  Activations BF16, channels padded to 32 (input) / 64 (hidden) /
- * 32 (output).  Weights BF16 [tap][cout][cin] (tap = 3*(dy+1)+(dx+1)) with
- * FP32 master copies, biases FP32.  Layer 0: conv cin->64, ReLU; layers
- * 1..L-2: a += ReLU(conv(a)); layer L-1: conv 64->cout, linear.  The
- * network's output is added to the normalised input u, v, z (residual).
+ * columns.  Activations BF16, 8 channels (input) / 64 (hidden); the output is
+ * FP32.  Weights BF16 [tap][cout][cin] (tap = 3*(dy+1)+(dx+1)), channels
+ * padded to 32 (input) / 64 (hidden) / 32 (output), with FP32 master copies,
+ * biases FP32.  Layer 0: conv cin->64, ReLU; layers 1..L-2:
+ * a += ReLU(conv(a)); layer L-1: conv 64->cout, linear.  The network's output
+ * is added to the normalised input u, v, z (residual).
  *
  * All pointers are device pointers unless named host_*.  Errors as in
  * hydist.h (0 or a negative HD_E* code; hd_cnn_last_error).
