@@ -113,7 +113,7 @@ struct ConvItems {
  * Workgroups stay for as many items as there are; a wave's three
  * accumulators are the output rows above, at and below the input row at
  * hand.  gate: a bit per channel and pixel, whether the layer's ReLU passed
- * (written forward when given; read backward for the layer below: dZ is
+ * (written forward; read backward for the layer below: dZ is
  * bf16(dA) where it did).  The layer adds its input to its output (RESRELU)
  * from the ring. */
 template <int EPI>
@@ -238,7 +238,7 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
                 buf_st16(b, 4 * oe, d0);
                 buf_st16(b, 4 * oe + 16, d1);
             } else {
-                __builtin_amdgcn_raw_buffer_store_b8((unsigned char)bits, row_buffer(gate, row_at(y, 8), gate ? 8 * w : 0u),
+                __builtin_amdgcn_raw_buffer_store_b8((unsigned char)bits, row_buffer(gate, row_at(y, 8), 8 * w),
                                                      (int)(oe >> 3), 0, 0);
             }
             buf_st16(row_buffer(Y, row_at(y, 2 * kWidth), 2 * kWidth * w), 2 * oe, yv);
@@ -934,13 +934,14 @@ static void wgrad(hd_cnn* n, const bf16* X, const bf16* dZ, const Layer& y, int 
                        dZ, it, y.dw, y.db);
 }
 
-/* gates: whether a backward pass may follow */
-static int forward(hd_cnn* n, int nimg, bool gates)
+/* The gates are written in every pass: a backward pass takes the activations
+ * of the last one, a prediction's too, and the gates have to be that one's. */
+static int forward(hd_cnn* n, int nimg)
 {
     const int L = n->L;
-    conv<EPI_RELU>(n, n->x0, n->layer[0], false, nimg, n->act[1], gates ? n->gate[0] : nullptr, nullptr);
+    conv<EPI_RELU>(n, n->x0, n->layer[0], false, nimg, n->act[1], n->gate[0], nullptr);
     for (int l = 1; l <= L - 2; ++l)
-        conv<EPI_RESRELU>(n, n->act[l], n->layer[l], false, nimg, n->act[l + 1], gates ? n->gate[l] : nullptr, nullptr);
+        conv<EPI_RESRELU>(n, n->act[l], n->layer[l], false, nimg, n->act[l + 1], n->gate[l], nullptr);
     conv<EPI_LINEAR>(n, n->act[L - 1], n->layer[L - 1], false, nimg, nullptr, nullptr, n->out);
     CHK(n, hipGetLastError());
     return HD_OK;
@@ -1187,7 +1188,7 @@ int hd_cnn_load_batch(hd_cnn* n, int b, const float* host_x, const float* host_y
 int hd_cnn_forward(hd_cnn* n, float* host_out)
 {
     if (!n || n->nb < 1) return cfail(n, HD_ESTATE, "hd_cnn_forward: no batch loaded");
-    int rc = forward(n, n->nb, true);
+    int rc = forward(n, n->nb);
     if (rc) return rc;
     if ((rc = loss_and_grad(n, n->nb, false))) return rc;
     if (host_out) {
@@ -1218,7 +1219,7 @@ int hd_cnn_adam(hd_cnn* n, float lr)
 int hd_cnn_train_step(hd_cnn* n, float lr, double* loss)
 {
     if (!n || n->nb < 1) return cfail(n, HD_ESTATE, "hd_cnn_forward: no batch loaded");
-    int rc = forward(n, n->nb, true);
+    int rc = forward(n, n->nb);
     if (!rc) rc = loss_and_grad(n, n->nb, true);
     if (!rc) rc = backward(n, n->nb);
     if (!rc) rc = adam(n, lr);
@@ -1289,7 +1290,7 @@ int hd_cnn_eval_samples(hd_cnn* n, const int* host_idx, int b, double* loss)
 {
     if (!n) return HD_EINVAL;
     int rc = gather(n, host_idx, b);
-    if (!rc) rc = forward(n, b, true);
+    if (!rc) rc = forward(n, b);
     if (!rc) rc = loss_and_grad(n, b, false);
     if (!rc) rc = finish(n, loss);
     return rc;
@@ -1318,7 +1319,7 @@ int hd_cnn_predict_into_ctx(hd_cnn* n, hd_ctx* c, float q, float zb)
         hipLaunchKernelGGL(k_active_tiles, dim3((tiles + 15) / 16), dim3(1024), 0, n->stream, dv, n->L - 1, n->tlist, n->tcount);
         n->tl = n->tlist;
     }
-    int rc = forward(n, 1, false);
+    int rc = forward(n, 1);
     n->tl = nullptr;
     if (rc) return rc;
     hipLaunchKernelGGL(k_unpack, dim3(nblk(n->P)), dim3(256), 0, n->stream, dv, n->sc, n->out);
