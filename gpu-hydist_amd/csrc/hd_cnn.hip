@@ -65,9 +65,11 @@ __device__ __forceinline__ void st_row(E* base, size_t row, unsigned off, T v)
 }
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-/* A row of `bytes` bytes as a buffer: loads past either end of it return
- * zeros and stores there are dropped (an offset below 0 is far past the end),
- * and none of a row of 0 bytes is touched.  So every step of a walk over
+/* A stretch of `bytes` bytes of a row as a buffer: loads past either end of
+ * it return zeros and stores there are dropped (an offset below 0 is far past
+ * the end), and none of a stretch of 0 bytes is touched.  A stretch is what a
+ * workgroup's columns need of the row and no more, so that offsets are small
+ * however wide the image is.  So every step of a walk over
  * rows has the same memory operations, which is what lets the compiler count
  * those in flight instead of waiting for all of them. */
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const void* base, size_t at, unsigned bytes)
@@ -179,8 +181,13 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
         w0 = uniform(w0);
         r0 = uniform(r0);
         r1 = uniform(r1 < H ? r1 : H);
-        /* the thread's pieces of a row: byte offsets, columns outside the
-         * image past the row's ends */
+        /* the columns that the item reads, those of the image from c0 on, and
+         * that it writes */
+        const int c0 = w0 > 0 ? w0 - 1 : 0;
+        const unsigned wr = (unsigned)uniform(W - c0 < PX ? W - c0 : PX);
+        const unsigned ww = (unsigned)uniform(W - w0 < 16 * SW ? W - w0 : 16 * SW);
+        /* the thread's pieces of a row: byte offsets from column c0, columns
+         * outside the image past the row's ends */
         struct Piece {
             bf16x8 q[NL];
             unsigned last;
@@ -188,15 +195,17 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
         unsigned vo[NL], vl = 0;
 #pragma unroll
         for (int q = 0; q < NL; ++q) {
-            const int e = threadIdx.x + 256 * q, c = w0 - 1 + e / (CS / 8);
+            const int e = threadIdx.x + 256 * q, c = w0 - 1 - c0 + e / (CS / 8);
             vo[q] = 2u * (unsigned)(c * CS + e % (CS / 8) * 8);
         }
-        if (!NARROW) vl = 2u * (unsigned)((w0 - 1 + PX - 2 + (l >> 5)) * CS) + 4u * (l & 31);
-        /* byte offset of row y of the item's image, E bytes a pixel; rows off
-         * the image have no bytes */
-        auto row_at = [&](int y, int E) -> size_t { return (img + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E; };
+        if (!NARROW) vl = 2u * (unsigned)((w0 - 1 - c0 + PX - 2 + (l >> 5)) * CS) + 4u * (l & 31);
+        /* byte offset of column c of row y of the item's image, E bytes a
+         * pixel; rows off the image have no bytes */
+        auto row_at = [&](int y, int c, int E) -> size_t {
+            return (img + c + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E;
+        };
         auto load = [&](int i, Piece& r) {
-            const auto b = row_buffer(X, row_at(i, 2 * CS), i >= 0 && i < H && i <= r1 ? 2u * CS * (unsigned)W : 0u);
+            const auto b = row_buffer(X, row_at(i, c0, 2 * CS), i >= 0 && i < H && i <= r1 ? 2u * CS * wr : 0u);
 #pragma unroll
             for (int q = 0; q < NL; ++q) r.q[q] = buf_ld16<bf16x8>(b, vo[q]);
             if (!NARROW) r.last = __builtin_amdgcn_raw_buffer_load_b32(b, (int)vl, 0, 0);
@@ -210,8 +219,8 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
             }
             if (!NARROW && wv == 0) *(unsigned*)(to + (PX - 2 + (l >> 5)) * PS + 2 * (l & 31)) = r.last;
         };
-        const int col = w0 + 16 * strip + n;
-        const unsigned oe = (unsigned)col * kWidth + cb; /* the lane's results in a row of 64 channels */
+        const int col = 16 * strip + n;                  /* of the item */
+        const unsigned oe = (unsigned)col * kWidth + cb; /* the lane's results in its row of 64 channels */
         /* old dA and the gate of an output row, loaded a row ahead */
         struct Old {
             f32x4 a, b;
@@ -219,29 +228,29 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
         };
         auto load_old = [&](int y, Old& o) {
             if (EPI != EPI_BWD_SET && EPI != EPI_BWD_ADD) return;
-            const unsigned w = y >= r0 && y < r1 ? (unsigned)W : 0u;
+            const unsigned w = y >= r0 && y < r1 ? ww : 0u;
             if (EPI == EPI_BWD_ADD) {
-                const auto b = row_buffer(Yf, row_at(y, 4 * kWidth), 4 * kWidth * w);
+                const auto b = row_buffer(Yf, row_at(y, w0, 4 * kWidth), 4 * kWidth * w);
                 o.a = buf_ld16<f32x4>(b, 4 * oe);
                 o.b = buf_ld16<f32x4>(b, 4 * oe + 16);
             }
-            o.gate = __builtin_amdgcn_raw_buffer_load_b8(row_buffer(gate, row_at(y, 8), 8 * w), (int)(oe >> 3), 0, 0);
+            o.gate = __builtin_amdgcn_raw_buffer_load_b8(row_buffer(gate, row_at(y, w0, 8), 8 * w), (int)(oe >> 3), 0, 0);
         };
         /* the results of output row y, or with w = 0 the same stores to nowhere */
         auto put = [&](int y, unsigned w, bf16x8 yv, unsigned bits, const f32x4& d0, const f32x4& d1) {
             if (EPI == EPI_LINEAR) {
-                buf_st16(row_buffer(Yf, row_at(y, 4 * kOut4), 4 * kOut4 * w), g == 0 ? 16u * col : ~0u, d0);
+                buf_st16(row_buffer(Yf, row_at(y, w0, 4 * kOut4), 4 * kOut4 * w), g == 0 ? 16u * col : ~0u, d0);
                 return;
             }
             if (EPI == EPI_BWD_SET || EPI == EPI_BWD_ADD) {
-                const auto b = row_buffer(Yf, row_at(y, 4 * kWidth), store_f ? 4 * kWidth * w : 0u);
+                const auto b = row_buffer(Yf, row_at(y, w0, 4 * kWidth), store_f ? 4 * kWidth * w : 0u);
                 buf_st16(b, 4 * oe, d0);
                 buf_st16(b, 4 * oe + 16, d1);
             } else {
-                __builtin_amdgcn_raw_buffer_store_b8((unsigned char)bits, row_buffer(gate, row_at(y, 8), 8 * w),
+                __builtin_amdgcn_raw_buffer_store_b8((unsigned char)bits, row_buffer(gate, row_at(y, w0, 8), 8 * w),
                                                      (int)(oe >> 3), 0, 0);
             }
-            buf_st16(row_buffer(Y, row_at(y, 2 * kWidth), 2 * kWidth * w), 2 * oe, yv);
+            buf_st16(row_buffer(Y, row_at(y, w0, 2 * kWidth), 2 * kWidth * w), 2 * oe, yv);
         };
         /* input row i: its products for the output rows i - 1 (below it in
          * the order of the taps: their last three), i and i + 1, then the
@@ -272,7 +281,7 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
                 for (int nb = 0; nb < NB; ++nb) below[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
                 taps(0, below);
             }
-            const unsigned w = done ? (unsigned)W : 0u;
+            const unsigned w = done ? ww : 0u;
             if (EPI == EPI_LINEAR) {
                 f32x4 v;
 #pragma unroll
@@ -430,25 +439,31 @@ __global__ void __launch_bounds__(512, 2) k_wgrad(const bf16* __restrict__ X, co
         const int r0 = uniform((t % it.rows) * it.R);
         const int r1 = uniform(k != k2 + half ? r0 : (r0 + it.R < H ? r0 + it.R : H));
         const size_t img = (size_t)uniform(t / it.rows) * H * W;
+        /* the columns of X, from c0 on, and of dZ that the item reads */
+        const int c0 = w0 > 0 ? w0 - 1 : 0;
+        const unsigned wx = (unsigned)uniform(W - c0 < 66 ? W - c0 : 66);
+        const unsigned wz = (unsigned)uniform(W - w0 < 64 ? W - w0 : 64);
         /* row h of dZ and row h + 1 of X, as each thread carries them */
         struct Rows {
             bf16x8 z[NZ], x[NX];
         };
-        auto row_at = [&](int y, int E) -> size_t { return (img + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E; };
+        auto row_at = [&](int y, int c, int E) -> size_t {
+            return (img + c + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E;
+        };
         auto ld_x = [&](int h, bool on, bf16x8(&x)[NX]) {
-            const auto b = row_buffer(X, row_at(h, 2 * CX), on && h >= 0 && h < H ? 2u * CX * (unsigned)W : 0u);
+            const auto b = row_buffer(X, row_at(h, c0, 2 * CX), on && h >= 0 && h < H ? 2u * CX * wx : 0u);
 #pragma unroll
             for (int q = 0; q < NX; ++q) {
                 const int e = tid + 256 * q;
-                x[q] = buf_ld16<bf16x8>(b, e < QX ? 2u * (unsigned)((w0 - 1 + e / (CX / 8)) * CX + e % (CX / 8) * 8) : ~0u);
+                x[q] = buf_ld16<bf16x8>(b, e < QX ? 2u * (unsigned)((w0 - 1 - c0 + e / (CX / 8)) * CX + e % (CX / 8) * 8) : ~0u);
             }
         };
         auto ld = [&](int h, Rows& r) {
-            const auto b = row_buffer(dZ, row_at(h, 2 * CZ), h < r1 ? 2u * CZ * (unsigned)W : 0u);
+            const auto b = row_buffer(dZ, row_at(h, w0, 2 * CZ), h < r1 ? 2u * CZ * wz : 0u);
 #pragma unroll
             for (int q = 0; q < NZ; ++q) {
                 const int e = tid + 256 * q;
-                r.z[q] = buf_ld16<bf16x8>(b, e < QZ ? 2u * (unsigned)((w0 + e / (CZ / 8)) * CZ + e % (CZ / 8) * 8) : ~0u);
+                r.z[q] = buf_ld16<bf16x8>(b, e < QZ ? 2u * (unsigned)(e / (CZ / 8) * CZ + e % (CZ / 8) * 8) : ~0u);
             }
             ld_x(h + 1, h < r1, r.x);
         };
