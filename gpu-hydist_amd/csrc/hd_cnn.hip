@@ -71,7 +71,11 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
  * workgroup's columns need of the row and no more, so that offsets are small
  * however wide the image is.  So every step of a walk over
  * rows has the same memory operations, which is what lets the compiler count
- * those in flight instead of waiting for all of them. */
+ * those in flight instead of waiting for all of them.  An access that is to
+ * touch nothing at all takes kNowhere: past every stretch (66 columns of 256
+ * bytes at most), aligned to 16 bytes, and far enough from 2^32 that none of
+ * its words wraps round to the row's start. */
+constexpr unsigned kNowhere = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const void* base, size_t at, unsigned bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)base + at), 0, (int)bytes, 0x00020000);
@@ -239,7 +243,7 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
         /* the results of output row y, or with w = 0 the same stores to nowhere */
         auto put = [&](int y, unsigned w, bf16x8 yv, unsigned bits, const f32x4& d0, const f32x4& d1) {
             if (EPI == EPI_LINEAR) {
-                buf_st16(row_buffer(Yf, row_at(y, w0, 4 * kOut4), 4 * kOut4 * w), g == 0 ? 16u * col : ~0u, d0);
+                buf_st16(row_buffer(Yf, row_at(y, w0, 4 * kOut4), 4 * kOut4 * w), g == 0 ? 16u * col : kNowhere, d0);
                 return;
             }
             if (EPI == EPI_BWD_SET || EPI == EPI_BWD_ADD) {
@@ -455,7 +459,8 @@ __global__ void __launch_bounds__(512, 2) k_wgrad(const bf16* __restrict__ X, co
 #pragma unroll
             for (int q = 0; q < NX; ++q) {
                 const int e = tid + 256 * q;
-                x[q] = buf_ld16<bf16x8>(b, e < QX ? 2u * (unsigned)((w0 - 1 - c0 + e / (CX / 8)) * CX + e % (CX / 8) * 8) : ~0u);
+                const int c = w0 - 1 - c0 + e / (CX / 8);
+                x[q] = buf_ld16<bf16x8>(b, e < QX ? 2u * (unsigned)(c * CX + e % (CX / 8) * 8) : kNowhere);
             }
         };
         auto ld = [&](int h, Rows& r) {
@@ -463,7 +468,8 @@ __global__ void __launch_bounds__(512, 2) k_wgrad(const bf16* __restrict__ X, co
 #pragma unroll
             for (int q = 0; q < NZ; ++q) {
                 const int e = tid + 256 * q;
-                r.z[q] = buf_ld16<bf16x8>(b, e < QZ ? 2u * (unsigned)(e / (CZ / 8) * CZ + e % (CZ / 8) * 8) : ~0u);
+                const unsigned at = 2u * (unsigned)(e / (CZ / 8) * CZ + e % (CZ / 8) * 8);
+                r.z[q] = buf_ld16<bf16x8>(b, e < QZ ? at : kNowhere);
             }
             ld_x(h + 1, h < r1, r.x);
         };
