@@ -1217,7 +1217,9 @@ struct SweepConst {
     double k, kx;      /* dTchia2dX, dTchia2dY (UZ; exchanged for VZ) */
     double dT, H, cor, wind;
     double e1, e2, e3; /* dXbp, dY2, dYbp (UZ); dYbp, dX2, dXbp (VZ) */
-    double y1, y2, y3; /* their refined reciprocals */
+    double y1, y2, y3; /* their refined reciprocals; y1 is NaN, and every fast
+                        * row with it, unless k, e1, e2 and e3 are within
+                        * 2^-50 .. 2^50 */
 };
 template <bool isU>
 __device__ __forceinline__ SweepConst sweep_const(const hd_params& P)
@@ -1235,6 +1237,11 @@ __device__ __forceinline__ SweepConst sweep_const(const hd_params& P)
     K.y1 = hd_div::rcp_refined(K.e1);
     K.y2 = hd_div::rcp_refined(K.e2);
     K.y3 = hd_div::rcp_refined(K.e3);
+    const double c[] = {K.k, K.e1, K.e2, K.e3};
+    bool ok = true;
+#pragma unroll
+    for (double v : c) ok = ok && v > 0x1p-50 && v < 0x1p50;
+    if (!ok) K.y1 = __builtin_nan("");
     return K;
 }
 
@@ -1302,8 +1309,9 @@ __device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreR
     o.c1 = useC ? -f4 - t4 : -f4;
     o.b1 = useC ? o.b1 - t5 : o.b1;
     o.d1 = useC ? o.d1 - t6 : o.d1;
-    /* zero or at least 2^-400 here and divisors in 2^[-100, 100] keep the
-     * products divided above in the range of hd_fastdiv.h */
+    /* zero or at least 2^-400 here, divisors in 2^[-100, 100] and case
+     * constants in 2^[-50, 50] keep the products divided above in the range
+     * of hd_fastdiv.h */
     rg.num(nv); rg.num(nk); rg.num(np); rg.num(nq); rg.num(nw);
     rg.num(f1); rg.num(f3); rg.num(o.d2);
     rg.den(htu);
