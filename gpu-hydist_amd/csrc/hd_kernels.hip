@@ -14,6 +14,7 @@
  * so the bits match the CPU checker.  Wave size is 64.
  */
 #include "hd_edges.h"
+#include "hd_forms.h"
 #include "hd_internal.h"
 #include "hd_thomas.h"
 
@@ -1260,9 +1261,9 @@ struct CellRow {
 };
 __device__ __forceinline__ double lane_after(double v) { return dpp_any<0x130>(v); }
 
-__device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreRaw& r, double f4, bool mom, bool useA,
-                                                 bool useC)
+__device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreRaw& r, double f4, const HdCellUse& use)
 {
+    const bool useA = use.behind, useC = use.ahead;
     CellRow o;
     hd_div::Range rg;
     const double uc = r.c;
@@ -1291,8 +1292,8 @@ __device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreR
     const double s3 = dm ? -3.0 : 3.0, s4 = dm ? 4.0 : -4.0, s1 = dm ? -1.0 : 1.0;
     const double pn = one ? s3 * uc + s4 * w1 + s1 * w2 : r.n1 - r.m1;
     const double qn = one ? uc - 2 * w1 + w2 : r.n1 - 2 * uc + r.m1;
-    const bool use = !one || (dm ? vtb < 0 : (r.hm_m2 > K.H && vtb > 0));
-    const double np = use ? vtb * pn : 0.0, nq = use ? qn : 0.0;
+    const bool with = !one || (dm ? vtb < 0 : (r.hm_m2 > K.H && vtb > 0));
+    const double np = with ? vtb * pn : 0.0, nq = with ? qn : 0.0;
     const double p = hd_div::quot_pos(np, K.e2, K.y2);
     const double q = hd_div::quot_pos(nq, K.e3, K.y3);
     const double nw = K.dT * (K.wind - r.ts);
@@ -1316,7 +1317,7 @@ __device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreR
     rg.num(f1); rg.num(f3); rg.num(o.d2);
     rg.den(htu);
     rg.den(useA ? r.ht_m : 1.0); rg.den(useC ? o.nc2 : 1.0);
-    o.bad = mom && !(rg.lo >= -400 && rg.den_ok() && htu > 0 && (!useA || r.ht_m > 0) && (!useC || o.nc2 > 0) &&
+    o.bad = use.row && !(rg.lo >= -400 && rg.den_ok() && htu > 0 && (!useA || r.ht_m > 0) && (!useC || o.nc2 > 0) &&
                      hd_div::finite((o.a1 + o.b1) + (o.c1 + o.d1)));
     return o;
 }
@@ -1453,9 +1454,7 @@ __global__ void __launch_bounds__(64, 2) k_adi_spec(const HdDev* __restrict__ dv
                     const PreRaw cur = raw;
                     if (k0 + 63 <= c1) raw = pre_ld_off<isU>(d, base(k0 + 63), cell_off(k0 + 63));
                     const int k = k0 + lane;
-                    const bool mom = k < last, inner = last - 1 > first;
-                    const bool useA = inner && !(br1 && k == first), useC = inner && !(br2 && k == last - 1);
-                    CellRow o = cell_rows_rcp(K, cur, f4, mom, useA, useC);
+                    CellRow o = cell_rows_rcp(K, cur, f4, hd_cell_use(lane, k, first, last, br1, br2));
                     if (__any(o.bad)) {
                         const Pre pa = isU ? pre_uz_ev(d.P, cur) : pre_vz_ev(d.P, cur);
                         const Pre pb = shfl_pre(pa, nbr);
