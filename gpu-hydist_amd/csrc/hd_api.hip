@@ -112,8 +112,9 @@ struct hd_ctx {
      * kernel + one lane per line ("rows").  All four give identical bits. */
     int solver = 0;
     bool solver_v1 = false;     /* two-kernel sediment form as well (HYDIST_SOLVER=rows) */
-    /* wetting form (HYDIST_WETTING): 0 default, 1 candidate windows for every
-     * line ("window"), 2 whole-line scans ("scan"); identical bits */
+    /* wetting form (HYDIST_WETTING): 0 default, 1 the replay from candidate
+     * windows for every line ("window"), 2 whole-line scans ("scan");
+     * identical bits */
     int wet_mode = 0;
     int run_blocks_u = 0, run_blocks_v = 0;
     double* bed_snap = nullptr; /* dH snapshot for hd_bed_extrapolate (allocated on first use) */

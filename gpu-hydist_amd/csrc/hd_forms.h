@@ -31,4 +31,15 @@ HD_FORM HdCellUse hd_cell_use(int lane, int k, int first, int last, bool br1, bo
     return u;
 }
 
+/* The wetting pass of a line with n recorded candidates, of which the list
+ * holds `most`; dependent: candidates near each other, or a cascade that
+ * leaves its window.  mode (HYDIST_WETTING): 1 the replay for every line, 2
+ * the scan. */
+enum { HD_WET_AT_ONCE, HD_WET_REPLAY, HD_WET_SCAN };
+HD_FORM int hd_wet_form(int mode, int n, int most, bool dependent)
+{
+    if (n > most || mode == 2) return HD_WET_SCAN;
+    return mode == 1 || dependent ? HD_WET_REPLAY : HD_WET_AT_ONCE;
+}
+
 #endif

@@ -2384,9 +2384,9 @@ __device__ __forceinline__ void wetting_line(const HdDevG& d, int horizontal, in
             atomicOr((unsigned long long*)d.wetb + (size_t)r * ((M + 3 + 63) >> 6) + (cc >> 6), 1ull << (cc & 63));
         }
     };
-    /* mode (a cross-check, same bits): 0 and 1 as described, 2 the whole-line
-     * scan for every line */
-    if (n > kCand || mode == 2) { /* more candidates than recorded: the whole line, one visit per round of loads */
+    /* mode (a cross-check, same bits): 0 as described, 1 the replay for every
+     * line that the list holds, 2 the whole-line scan for every line */
+    if (hd_wet_form(mode, n, kCand, false) == HD_WET_SCAN) { /* more candidates than recorded: the whole line, one visit per round of loads */
         if (lane != 0) return;
         bool cascade = false;
         double tzc = 0, fsc = 0;
@@ -2444,7 +2444,7 @@ __device__ __forceinline__ void wetting_line(const HdDevG& d, int horizontal, in
         vis[o] = more && p + o <= pmax && wtz > wz[o];
         more = vis[o] && p + o + 1 <= pmax + 1 && wkh[o + 2] == 1;
     }
-    if (!__any(near || more)) {
+    if (hd_wet_form(mode, n, kCand, __any(near || more)) == HD_WET_AT_ONCE) {
         if (lane < n) {
             /* left of p, p itself (from p + 1), then to the right; cells
              * further left were opened by the cascade */

@@ -43,3 +43,21 @@ int use(int lane, int k, int first, int last, int br1, int br2)
                 assert bool(u & 2) == (n > 2 and not (br1 and k == first))
                 assert bool(u & 4) == (n > 2 and not (br2 and k == last - 1))
         assert (rows[:-1] == 1).all() and rows[-1] == 0
+
+
+def test_wetting_forms(tmp_path):
+    """HYDIST_WETTING=window replays every line that the candidate list holds
+    and =scan scans every line; by default the lanes visit their candidates at
+    once unless one depends on another."""
+    L = compiled(tmp_path, "wet", """
+int form(int mode, int n, int dependent) { return hd_wet_form(mode, n, 64, dependent); }
+int at_once() { return HD_WET_AT_ONCE; }
+int replay() { return HD_WET_REPLAY; }
+int scan() { return HD_WET_SCAN; }""")
+    at_once, replay, scan = L.at_once(), L.replay(), L.scan()
+    for n in (1, 8, 9, 64):
+        for dependent in (0, 1):
+            assert L.form(0, n, dependent) == (replay if dependent else at_once)
+            assert L.form(1, n, dependent) == replay
+            assert L.form(2, n, dependent) == scan
+    assert {L.form(m, 65, 0) for m in (0, 1, 2)} == {scan}
