@@ -42,4 +42,14 @@ HD_FORM int hd_wet_form(int mode, int n, int most, bool dependent)
     return mode == 1 || dependent ? HD_WET_REPLAY : HD_WET_AT_ONCE;
 }
 
+/* Whether a batch of nsys tridiagonal systems, `some` of which have `rows`
+ * rows together, goes by a lane per system rather than a wave.  A lane takes about 0.75 us per row of
+ * the longest system, waves about 4.2 us for every 2048 systems (eight
+ * workgroups of 18 KB of LDS on each of 256 CUs): the lane form where the
+ * first is less.  Measured, lane against wave form, us: 4 rows x 64 systems
+ * 3.4 / 4.2, 8 x 64 4.8 / 4.1, 8 x 2000 5.1 / 6.1, 12 x 2000 6.9 / 6.2, 16 x
+ * 2000 11 / 6.1, 24 x 20000 24 / 48, 32 x 20000 32 / 46, 64 x 20000 61 / 53,
+ * 64 x 2000 41 / 7.5. */
+HD_FORM bool hd_thomas_lanes(int nsys, int some, long long rows) { return (nsys + 2048LL) * some > 384 * rows; }
+
 #endif

@@ -3272,14 +3272,13 @@ __global__ void k_wet_count(const HdDev* __restrict__ dv)
 
 /* ================================================================ batched Thomas */
 
-/* One system per lane.  A system outside rows [0, nrows) is skipped (its x
- * is left as it is): the host checks the tables where it holds them, and this
- * check covers tables that only the device holds. */
-__global__ void k_thomas_batch(int nsys, const int* off, const int* sn, const double* A, const double* B,
-                               const double* C, const double* D, double* x, double* Ap, double* Bp, int nrows)
+/* System s by one lane, serially.  A system outside rows [0, nrows) is
+ * skipped (its x is left as it is): the host checks the tables where it holds
+ * them, and this check covers tables that only the device holds. */
+__device__ __forceinline__ void thomas_lane(int s, const int* off, const int* sn, const double* A, const double* B,
+                                            const double* C, const double* D, double* x, double* Ap, double* Bp,
+                                            int nrows)
 {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsys) return;
     int o = off[s], n = sn[s];
     if (n < 0 || o < 0 || n >= nrows - o) return;
     if (n == 0) { x[o] = D[o] / B[o]; return; }
@@ -3297,22 +3296,49 @@ __global__ void k_thomas_batch(int nsys, const int* off, const int* sn, const do
     for (int r = n - 1; r >= 0; --r) { xv = Bp[o + r] + (Ap[o + r] * xv); x[o + r] = xv; }
 }
 
+/* One system per lane. */
+__global__ void k_thomas_batch(int nsys, const int* off, const int* sn, const double* A, const double* B,
+                               const double* C, const double* D, double* x, double* Ap, double* Bp, int nrows)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < nsys) thomas_lane(s, off, sn, A, B, C, D, x, Ap, Bp, nrows);
+}
+
 /* One wave per system: the speculative parallel Thomas of the run solvers
  * (hd_thomas.h) on a caller's system, rows in LDS chunks of 510, the
  * factors of earlier chunks through Ap / Bp (as k_adi_spec spills them).
  * The same bits as the serial solve of tridiag
  * (UVZSolver_multithread.cu:203-228); a system outside rows [0, nrows) is
  * skipped (its x is left as it is): the host checks the tables where it
- * holds them, and this check covers tables that only the device holds. */
+ * holds them, and this check covers tables that only the device holds.
+ * by_lanes: systems 64 g .. 64 g + 63 go by a lane each in workgroup g if all
+ * of them are short enough, and their own workgroups leave: the host knows
+ * the length of the arrays and not that of the systems.  Their sn arrive in
+ * one load, the workgroup's own among them, so that long systems pay nothing
+ * (2000 of 24-503 rows: 12 us either way).  8 rows x 15000 systems in arrays
+ * of 10^6 rows: 6.5 us, with a wave each 29, lanes alone 6.1; in the first
+ * system's workgroup, 64 g, all the work is on one XCD (4000 systems: 15.9 us
+ * against 5.3). */
 __global__ void __launch_bounds__(64) k_thomas_spec(int nsys, const int* off, const int* sn, const double* A,
                                                     const double* B, const double* C, const double* D, double* x,
-                                                    double* Ap, double* Bp, int nrows)
+                                                    double* Ap, double* Bp, int nrows, int by_lanes)
 {
     constexpr int RW = 510;
     __shared__ double sA[spec_words(RW)], sB[spec_words(RW)], sC[spec_words(RW)], sD[spec_words(RW)];
     const int s = blockIdx.x, lane = threadIdx.x;
     if (s >= nsys) return;
-    const int o = off[s], n = sn[s];
+    const int q = (s & ~63) + lane;
+    const int nq = sn[q < nsys ? q : nsys - 1];
+    const int o = off[s], n = __builtin_amdgcn_readlane(nq, s & 63);
+    if (by_lanes) {
+        auto long_ones = [&](int len) -> bool { return __any(!hd_thomas_lanes(nsys, 1, len + 1LL)); };
+        if (s <= (nsys - 1) >> 6) {
+            const int g = 64 * s + lane;
+            if (!long_ones(sn[g < nsys ? g : nsys - 1]) && g < nsys)
+                thomas_lane(g, off, sn, A, B, C, D, x, Ap, Bp, nrows);
+        }
+        if (!long_ones(nq)) return;
+    }
     if (n < 0 || o < 0 || n >= nrows - o) return;
     if (n == 0) {
         if (lane == 0) x[o] = D[o] / B[o];
@@ -3542,27 +3568,20 @@ void hd_launch_wet_count(const HdBatch& b, hipStream_t s)
     hipLaunchKernelGGL(k_wet_count, dim3(b.N + 3, 1, b.n), dim3(64), 0, s, b.dv);
 }
 
-/* One lane per system takes about 0.75 us per row of the mean system, one
- * wave per system about 4.2 us for every 2048 systems (eight workgroups of
- * 18 KB of LDS on each of 256 CUs): the lane form where the first is less.
- * Measured, lane against wave form, us: 4 rows x 64 systems 3.4 / 4.2, 8 x 64
- * 4.8 / 4.1, 8 x 2000 5.1 / 6.1, 12 x 2000 6.9 / 6.2, 16 x 2000 11 / 6.1, 24 x
- * 20000 24 / 48, 32 x 20000 32 / 46, 64 x 20000 61 / 53, 64 x 2000 41 / 7.5. */
-static bool batch_lane_form(int nsys, int nrows)
-{
-    return ((long long)nsys + 2048) * nsys > 384LL * nrows;
-}
-
+/* The lane form where the arrays are short enough that the systems' mean
+ * length takes it, else a wave or, as the device finds the lengths, a lane per
+ * system (k_thomas_spec). */
 int hd_thomas_batch_device(int nsys, const int* off, const int* sn, const double* A, const double* B,
                            const double* C, const double* D, double* x, double* Ap, double* Bp, int nrows,
                            hipStream_t s)
 {
     if (nsys <= 0) return 0;
-    if (batch_lane_form(nsys, nrows))
+    if (hd_thomas_lanes(nsys, nsys, nrows))
         hipLaunchKernelGGL(k_thomas_batch, dim3((nsys + 63) / 64), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap,
                            Bp, nrows);
     else
-        hipLaunchKernelGGL(k_thomas_spec, dim3(nsys), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap, Bp, nrows);
+        hipLaunchKernelGGL(k_thomas_spec, dim3(nsys), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap, Bp, nrows,
+                           1);
     return 0;
 }
 
@@ -3571,7 +3590,8 @@ int hd_thomas_spec_device(int nsys, const int* off, const int* sn, const double*
                           hipStream_t s)
 {
     if (nsys > 0)
-        hipLaunchKernelGGL(k_thomas_spec, dim3(nsys), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap, Bp, nrows);
+        hipLaunchKernelGGL(k_thomas_spec, dim3(nsys), dim3(64), 0, s, nsys, off, sn, A, B, C, D, x, Ap, Bp, nrows,
+                           0);
     return 0;
 }
 

@@ -61,3 +61,15 @@ int scan() { return HD_WET_SCAN; }""")
             assert L.form(1, n, dependent) == replay
             assert L.form(2, n, dependent) == scan
     assert {L.form(m, 65, 0) for m in (0, 1, 2)} == {scan}
+
+
+def test_batched_thomas_form(tmp_path):
+    """Short systems of a large batch go by lanes whatever the arrays' length
+    is: the device takes the longest of 64 systems."""
+    L = compiled(tmp_path, "thomas", "int lanes(int nsys, int some, long long rows) "
+                                     "{ return hd_thomas_lanes(nsys, some, rows); }")
+    lanes = lambda nsys, some, rows: L.lanes(nsys, some, ctypes.c_longlong(rows))
+    for nsys, rows, want in ((64, 4, 1), (64, 8, 0), (2000, 8, 1), (2000, 12, 0), (20000, 24, 1), (20000, 64, 0),
+                             (1, 2, 1), (1, 503, 0), (2000, 503, 0), (2**31 - 1, 2**20, 1), (5, 2**31, 0), (9, 0, 1)):
+        assert lanes(nsys, 1, rows) == want
+        assert lanes(nsys, nsys, rows * nsys) == want
