@@ -188,8 +188,8 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
         /* the columns that the item reads, those of the image from c0 on, and
          * that it writes */
         const int c0 = w0 > 0 ? w0 - 1 : 0;
-        const unsigned wr = (unsigned)uniform(W - c0 < PX ? W - c0 : PX);
-        const unsigned ww = (unsigned)uniform(W - w0 < 16 * SW ? W - w0 : 16 * SW);
+        const unsigned wr = W - c0 < PX ? W - c0 : PX, ww = W - w0 < 16 * SW ? W - w0 : 16 * SW;
+        const size_t imgx = img + c0, imgy = img + w0;
         /* the thread's pieces of a row: byte offsets from column c0, columns
          * outside the image past the row's ends */
         struct Piece {
@@ -203,13 +203,13 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
             vo[q] = 2u * (unsigned)(c * CS + e % (CS / 8) * 8);
         }
         if (!NARROW) vl = 2u * (unsigned)((w0 - 1 - c0 + PX - 2 + (l >> 5)) * CS) + 4u * (l & 31);
-        /* byte offset of column c of row y of the item's image, E bytes a
-         * pixel; rows off the image have no bytes */
-        auto row_at = [&](int y, int c, int E) -> size_t {
-            return (img + c + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E;
+        /* byte offset of row y of the item's image from its column at, E
+         * bytes a pixel; rows off the image have no bytes */
+        auto row_at = [&](size_t at, int y, int E) -> size_t {
+            return (at + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E;
         };
         auto load = [&](int i, Piece& r) {
-            const auto b = row_buffer(X, row_at(i, c0, 2 * CS), i >= 0 && i < H && i <= r1 ? 2u * CS * wr : 0u);
+            const auto b = row_buffer(X, row_at(imgx, i, 2 * CS), i >= 0 && i < H && i <= r1 ? 2u * CS * wr : 0u);
 #pragma unroll
             for (int q = 0; q < NL; ++q) r.q[q] = buf_ld16<bf16x8>(b, vo[q]);
             if (!NARROW) r.last = __builtin_amdgcn_raw_buffer_load_b32(b, (int)vl, 0, 0);
@@ -234,27 +234,27 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wt, const float* __r
             if (EPI != EPI_BWD_SET && EPI != EPI_BWD_ADD) return;
             const unsigned w = y >= r0 && y < r1 ? ww : 0u;
             if (EPI == EPI_BWD_ADD) {
-                const auto b = row_buffer(Yf, row_at(y, w0, 4 * kWidth), 4 * kWidth * w);
+                const auto b = row_buffer(Yf, row_at(imgy, y, 4 * kWidth), 4 * kWidth * w);
                 o.a = buf_ld16<f32x4>(b, 4 * oe);
                 o.b = buf_ld16<f32x4>(b, 4 * oe + 16);
             }
-            o.gate = __builtin_amdgcn_raw_buffer_load_b8(row_buffer(gate, row_at(y, w0, 8), 8 * w), (int)(oe >> 3), 0, 0);
+            o.gate = __builtin_amdgcn_raw_buffer_load_b8(row_buffer(gate, row_at(imgy, y, 8), 8 * w), (int)(oe >> 3), 0, 0);
         };
         /* the results of output row y, or with w = 0 the same stores to nowhere */
         auto put = [&](int y, unsigned w, bf16x8 yv, unsigned bits, const f32x4& d0, const f32x4& d1) {
             if (EPI == EPI_LINEAR) {
-                buf_st16(row_buffer(Yf, row_at(y, w0, 4 * kOut4), 4 * kOut4 * w), g == 0 ? 16u * col : kNowhere, d0);
+                buf_st16(row_buffer(Yf, row_at(imgy, y, 4 * kOut4), 4 * kOut4 * w), g == 0 ? 16u * col : kNowhere, d0);
                 return;
             }
             if (EPI == EPI_BWD_SET || EPI == EPI_BWD_ADD) {
-                const auto b = row_buffer(Yf, row_at(y, w0, 4 * kWidth), store_f ? 4 * kWidth * w : 0u);
+                const auto b = row_buffer(Yf, row_at(imgy, y, 4 * kWidth), store_f ? 4 * kWidth * w : 0u);
                 buf_st16(b, 4 * oe, d0);
                 buf_st16(b, 4 * oe + 16, d1);
             } else {
-                __builtin_amdgcn_raw_buffer_store_b8((unsigned char)bits, row_buffer(gate, row_at(y, w0, 8), 8 * w),
+                __builtin_amdgcn_raw_buffer_store_b8((unsigned char)bits, row_buffer(gate, row_at(imgy, y, 8), 8 * w),
                                                      (int)(oe >> 3), 0, 0);
             }
-            buf_st16(row_buffer(Y, row_at(y, w0, 2 * kWidth), 2 * kWidth * w), 2 * oe, yv);
+            buf_st16(row_buffer(Y, row_at(imgy, y, 2 * kWidth), 2 * kWidth * w), 2 * oe, yv);
         };
         /* input row i: its products for the output rows i - 1 (below it in
          * the order of the taps: their last three), i and i + 1, then the
@@ -445,17 +445,17 @@ __global__ void __launch_bounds__(512, 2) k_wgrad(const bf16* __restrict__ X, co
         const size_t img = (size_t)uniform(t / it.rows) * H * W;
         /* the columns of X, from c0 on, and of dZ that the item reads */
         const int c0 = w0 > 0 ? w0 - 1 : 0;
-        const unsigned wx = (unsigned)uniform(W - c0 < 66 ? W - c0 : 66);
-        const unsigned wz = (unsigned)uniform(W - w0 < 64 ? W - w0 : 64);
+        const unsigned wx = W - c0 < 66 ? W - c0 : 66, wz = W - w0 < 64 ? W - w0 : 64;
+        const size_t imgx = img + c0, imgz = img + w0;
         /* row h of dZ and row h + 1 of X, as each thread carries them */
         struct Rows {
             bf16x8 z[NZ], x[NX];
         };
-        auto row_at = [&](int y, int c, int E) -> size_t {
-            return (img + c + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E;
+        auto row_at = [&](size_t at, int y, int E) -> size_t {
+            return (at + (size_t)uniform((y < 0 ? 0 : (y < H ? y : H - 1)) * W)) * E;
         };
         auto ld_x = [&](int h, bool on, bf16x8(&x)[NX]) {
-            const auto b = row_buffer(X, row_at(h, c0, 2 * CX), on && h >= 0 && h < H ? 2u * CX * wx : 0u);
+            const auto b = row_buffer(X, row_at(imgx, h, 2 * CX), on && h >= 0 && h < H ? 2u * CX * wx : 0u);
 #pragma unroll
             for (int q = 0; q < NX; ++q) {
                 const int e = tid + 256 * q;
@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(512, 2) k_wgrad(const bf16* __restrict__ X, co
             }
         };
         auto ld = [&](int h, Rows& r) {
-            const auto b = row_buffer(dZ, row_at(h, w0, 2 * CZ), h < r1 ? 2u * CZ * wz : 0u);
+            const auto b = row_buffer(dZ, row_at(imgz, h, 2 * CZ), h < r1 ? 2u * CZ * wz : 0u);
 #pragma unroll
             for (int q = 0; q < NZ; ++q) {
                 const int e = tid + 256 * q;
