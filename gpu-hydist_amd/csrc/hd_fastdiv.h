@@ -5,13 +5,15 @@
  * The correctly rounded division n / e is computed on this part as
  *   y0 = rcp(e), two Newton steps y -> y + y (1 - e y), q0 = n y,
  *   r = n - e q0 (one FMA, exact), q = q0 + r y (one FMA),
- * around which it scales operands that are near the ends of the exponent
- * range and repairs zeros, infinities and NaNs.  Every operation in the
- * middle is invariant under scaling by powers of two, so wherever nothing
- * overflows or underflows, leaving the scaling out changes no bit; and y
- * depends on e alone, so quotients by the same e share it (75 cycles for a
- * division, about 45 for y and 20 for each quotient, the part's measured
- * latencies).  The two cases that differ are kept out by the caller:
+ * (the last two steps are Markstein's correction of a quotient, P. Markstein,
+ * IBM J. Res. Dev. 34, 1990, with y accurate to about a rounding of 1 / e and
+ * r exact), around which it scales operands that are near the ends of the
+ * exponent range and repairs zeros, infinities and NaNs.
+ * Every operation in the middle is invariant under scaling by powers of two,
+ * so wherever nothing overflows or underflows, leaving the scaling out changes
+ * no bit; and y depends on e alone, so quotients by the same e share it (75
+ * cycles for a division, about 45 for y and 20 for each quotient, the part's
+ * measured latencies).  The two cases that differ are kept out by the caller:
  *  - a numerator of -0 over e > 0 would give +0 (quot; quot_pos gives the
  *    right zeros for every numerator while e > 0);
  *  - operands out of range: Range collects the exponents of divisors and

@@ -1340,8 +1340,8 @@ __device__ __forceinline__ CellRow cell_rows_rcp(const SweepConst& K, const PreR
  * divisor and selects instead of branches (cell_rows_rcp), loads from scalar
  * bases with 16-byte pairs, one copy of the boundary code, the next round's
  * loads behind this round's arithmetic.  Longest run of a launch, on the
- * device, river 980 x 1048: 24.0 -> 19.0 us once the flow is steady, 35 -> 27
- * while it starts up; 300-cell channel lines 38 -> 26.6 us. */
+ * device, river 980 x 1048: 24.0 -> 17.8 us once the flow is steady, 35 -> 27
+ * while it starts up; 300-cell channel lines 38 -> 25.8 us. */
 /* repaired chunks of a sweep above which the next sweep of the same
  * direction takes 8 rows per lane */
 constexpr int kAdaptRuns = 32;

@@ -238,15 +238,17 @@ int hd_ensemble_kernel_times(hd_ensemble* e, int n, const char** names, double* 
 /* Batched Thomas solve (UVZSolver_multithread.cu:203-228 applied per system):
  * nsys systems, system s occupies rows off[s] .. off[s]+sn[s] of the device
  * arrays A,B,C,D (lower, diagonal, upper, rhs); x receives the solution.
- * All pointers are host pointers; the call copies in and out. */
+ * A lane or a wave per system, by their number and lengths (64 successive
+ * systems at a time; nrows is the length of the arrays and need not be that
+ * of the systems); the same bits either way.  All pointers are host pointers;
+ * the call copies in and out. */
 int hd_thomas_batch(int device, int nsys, const int* off, const int* sn,
                     const double* A, const double* B, const double* C,
                     const double* D, double* x, int nrows);
-/* The same systems through the run solvers' speculative parallel Thomas
- * (one wave per system, rows in LDS chunks of 510; the tridiag of
- * UVZSolver_multithread.cu:203-228 that k_adi_spec runs): the same bits as
- * hd_thomas_batch, for unit tests of the speculation and its repairs on
- * chosen systems. */
+/* The same with a wave for every system, whatever its length: the run
+ * solvers' speculative parallel Thomas (rows in LDS chunks of 510; the tridiag
+ * of UVZSolver_multithread.cu:203-228 that k_adi_spec runs), for unit tests of
+ * the speculation and its repairs on chosen systems. */
 int hd_thomas_batch_spec(int device, int nsys, const int* off, const int* sn,
                          const double* A, const double* B, const double* C,
                          const double* D, double* x, int nrows);

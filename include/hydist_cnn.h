@@ -75,8 +75,8 @@ int hd_cnn_load_batch(hd_cnn* n, int b, const float* host_x, const float* host_y
 /* Forward over the loaded batch; host_out (optional) [b][H][W][3] receives
  * the prediction (normalised, input u, v, z + network output). */
 int hd_cnn_forward(hd_cnn* n, float* host_out);
-/* Masked mean-squared error of the last forward against the loaded targets
- * and its gradients (into the grad buffers); *loss receives the loss. */
+/* Masked mean-squared error of the last forward pass (a prediction by
+ * hd_cnn_predict_into_ctx is one) against the loaded targets and its gradients (into the grad buffers); *loss receives the loss. */
 int hd_cnn_backward(hd_cnn* n, double* loss);
 /* One Adam step (lr, beta1 0.9, beta2 0.999, eps 1e-8) on every layer from
  * the gradient buffers; refreshes the BF16 weights. */
